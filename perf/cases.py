@@ -4,7 +4,8 @@ Every case is one problem (its equation, grid, network and precision) and one
 call on it, through the entry points a program uses:
 
 * ``train``: a short ``Model.train`` with Adam, as a script calls it (initial
-  loss, captured step, replays): small problems, where launches count.
+  loss, captured step, replays), each pass from the problem's first weights:
+  small problems, where launches count.
 * ``step``: one fused training step of the compiled problem
   (``engine.train_step``, ``train_step_to`` on a grid, ``SweepSolver.step``
   for a sweep): loss, new weights and both Adam moments.
@@ -41,11 +42,11 @@ def listed():
         # the smallest solve: an ordinary differential equation on 100 points,
         # trained by Model.train; launches and latency
         dict(name='legendre_train', call='train', eq='legendre', n0=100, n1=1, width=100,
-             hidden=2, dtype='float32', epochs=401),
+             hidden=2, dtype='float32', epochs=151),
         # a small grid tensor under Model.train, one step a few microseconds
         # of work
         dict(name='wave_train', call='train', eq='wave', n0=128, n1=128, dtype='float32',
-             epochs=501),
+             epochs=301),
         # a large grid tensor: the streaming case
         dict(name='wave_large_step', call='step', eq='wave', n0=8192, n1=8192, dtype='float32'),
         # a ragged grid in double precision under a torch optimizer
@@ -86,7 +87,7 @@ def draw(rng):
         if rng.random() < 0.5:
             return dict(call='train', eq='legendre', n0=size(40, 400), n1=1,
                         width=rng.choice([16, 32, 50, 64, 100]), hidden=rng.randint(2, 4),
-                        dtype='float32', epochs=201)
+                        dtype='float32', epochs=151)
         return dict(call='train', eq='wave', n0=size(32, 300), n1=size(32, 300),
                     dtype='float32', epochs=201)
     if kind == 'wave':
@@ -238,6 +239,8 @@ def prepare(case, seed):
     state = dict(case=case, model=model, sol=model.solution_cls, eng=model.solution_cls.engine)
     if case['call'] == 'train':
         state['optimizer'] = Optimizer('Adam', {'lr': LR})
+        leaves = [model.net] if case['eq'] == 'wave' else list(model.net.parameters())
+        state['first'] = [(p, p.detach().clone()) for p in leaves]
     elif case['call'] == 'step':
         flat = model.net if case['eq'] == 'wave' else \
             torch.cat([p.detach().reshape(-1) for p in model.net.parameters()])
@@ -258,6 +261,8 @@ def run(state):
     case = state['case']
     if case['call'] == 'train':
         model = state['model']
+        for p, first in state['first']:
+            p.data.copy_(first)
         model.train(state['optimizer'], case['epochs'])
         if case['eq'] == 'wave':
             return [model.cur_loss, model.net]
@@ -338,11 +343,12 @@ def tolerance(case):
     """About four times the largest error against 64 bits seen over the ranges
     of ``draw``.  The network problems take differences of 32-bit network
     values over h (1e-3; KdV: over h^3, 1e-6), which is what remains of them
-    in gradients.  Of runs of many steps the same is said from one sum order
-    to another."""
+    in gradients.  Of Legendre runs of 150 steps the same is said from one
+    order of the gradient's sums to another (work items of one tile and of
+    eight: weights up to 3.1e-3 apart, single ones 1.5e-2)."""
     eq, wide = case['eq'], case['dtype'] == 'float64'
     if case['call'] == 'train':
-        return {'rel': 0.02, 'max': 0.5} if eq == 'legendre' else {'rel': 2e-3}
+        return {'rel': 0.012, 'max': 0.06} if eq == 'legendre' else {'rel': 2e-3}
     if eq == 'wave':
         return {'rel': 4e-15} if wide else {'rel': 1.2e-6, 'max': 2e-3}
     if eq in ('poisson', 'lotka'):
