@@ -1855,6 +1855,38 @@ int nn_dispatch(const tdx_nn_plan *p, int op, const void *params, void *params_m
 #undef TDX_NB_CASE
 }
 
+// Tiles per work item for a launch whose workgroups walk items of up to
+// `cap` tiles of one group.  tiles: tiles of each group; slots: workgroups
+// resident on the device at once (256 CUs); overhead: an item's fixed cost
+// (staging, the final sums, its gradient partial) in tiles.  The launch
+// takes about ceil(items / slots) rounds of `chunk` tiles each, so the chunk
+// with the smallest rounds * (chunk + overhead) is taken, the larger one of
+// equals: a small problem gets single-tile items that spread over the
+// device, a middling one items that fill whole rounds.  Beyond 16 rounds
+// the last one no longer counts and the cap stands.  Measured against fixed
+// chunks (256 tiles wavefront-private, 8 block-owning): evaluate and backward
+// of 201 x 77 Burgers on 2-32x3-1 1090 -> 264 us (7 items before), Legendre's
+// 100 points on 1-100x2-1 192 -> 38 us a step (2 items before), Burgers
+// 256 x 100 on 2-100x4-1 755 -> 526 us (346 items of 8 tiles took two rounds
+// of 256; now 252 of 11 take one), KdV 512 x 128 489 -> 429 us.
+constexpr int kCUs = 256;
+int pick_chunk(const std::vector<int64_t> &tiles, int64_t slots, int cap, double overhead) {
+  int best = cap;
+  double best_cost = 0;
+  for (int c = cap; c >= 1; --c) {
+    int64_t items = 0;
+    for (int64_t t : tiles) items += (t + c - 1) / c;
+    const int64_t rounds = (items + slots - 1) / slots;
+    const double cost = (double)rounds * (c + overhead);
+    if (c == cap && rounds > 16) return cap;
+    if (c == cap || cost < best_cost) {
+      best = c;
+      best_cost = cost;
+    }
+  }
+  return best;
+}
+
 // Host-side validation of every table index, so that a malformed table is an
 // error code and never an out-of-bounds access on the device.
 int validate_nn(const tdx_nn_desc *d, int64_t *n_rows_out) {
@@ -2116,8 +2148,16 @@ extern "C" int tdx_nn_plan_create(const tdx_nn_desc *d, tdx_nn_plan **out) {
   p->persist = (d->persistent > 0 && p->k1_stage && d->causal_tol == 0.0 &&
                 d->weak_levels == 0) ? 1 : 0;
   const int TR = 16 * p->k2_waves;
-  const int chunk_tiles = d->chunk_tiles > 0 ? d->chunk_tiles
-                        : (p->k2_wave_private ? 256 : (p->k2_block ? 8 : (p->acc_lds ? 16 : 4)));
+  std::vector<int64_t> k2_tiles;
+  for (int g = 0; g < d->n_groups; ++g) {
+    const int32_t *G = d->groups + (int64_t)g * TDX_GROUP_INTS;
+    k2_tiles.push_back(((int64_t)G[1] * G[2] + TR - 1) / TR);
+  }
+  const int chunk_tiles =
+      d->chunk_tiles > 0  ? d->chunk_tiles
+      : p->k2_wave_private ? pick_chunk(k2_tiles, 3 * kCUs, 256, 1.0)
+      : p->k2_block        ? pick_chunk(k2_tiles, kCUs, 16, 0.25)
+                           : pick_chunk(k2_tiles, kCUs, p->acc_lds ? 16 : 4, 1.0);
   std::vector<int4> k2;
   for (int g = 0; g < d->n_groups; ++g) {
     const int32_t *G = d->groups + (int64_t)g * TDX_GROUP_INTS;
@@ -2159,7 +2199,10 @@ extern "C" int tdx_nn_plan_create(const tdx_nn_desc *d, tdx_nn_plan **out) {
     }
   }
   if (fuse) {
-    const int C = d->chunk_tiles > 0 ? d->chunk_tiles : 4;
+    std::vector<int64_t> blocks;
+    for (int g = 0; g < d->n_groups; ++g)
+      blocks.push_back((d->groups[(int64_t)g * TDX_GROUP_INTS + 1] + 63) / 64);
+    const int C = d->chunk_tiles > 0 ? d->chunk_tiles : pick_chunk(blocks, 4 * kCUs, 4, 0.25);
     for (int g = 0; g < d->n_groups; ++g) {
       const int32_t *G = d->groups + (int64_t)g * TDX_GROUP_INTS;
       const int nblk = (G[1] + 63) / 64;
@@ -2218,7 +2261,12 @@ extern "C" int tdx_nn_plan_create(const tdx_nn_desc *d, tdx_nn_plan **out) {
       prog_reals.insert(prog_reals.end(), fp.reals.begin(), fp.reals.end());
     }
     std::vector<std::vector<int>> inst_k4(d->n_inst);
-    const int C = d->chunk_tiles > 0 ? d->chunk_tiles : 8;
+    std::vector<int64_t> tiles;
+    for (int g = 0; g < d->n_groups; ++g) {
+      const int32_t *G = d->groups + (int64_t)g * TDX_GROUP_INTS;
+      tiles.push_back((G[1] + 64 / G[2] - 1) / (64 / G[2]));
+    }
+    const int C = d->chunk_tiles > 0 ? d->chunk_tiles : pick_chunk(tiles, kCUs, 16, 0.25);
     for (int g = 0; g < d->n_groups; ++g) {
       const int32_t *G = d->groups + (int64_t)g * TDX_GROUP_INTS;
       const int E = 64 / G[2];
