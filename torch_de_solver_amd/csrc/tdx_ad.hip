@@ -966,7 +966,7 @@ template <int NB>
 __global__ void k_ad_pack(NNArgs<float> a, int64_t *step) {
   constexpr int HP = 16 * NB;
   if (blockIdx.x == 0 && threadIdx.x == 0) *step += 1;
-  const int IMG = image_words(HP, a.NH, a.d_in, a.n_out);
+  const int IMG = image_words(HP, a.NH, a.d_in, a.n_out, 4);
   for (int t = blockIdx.x * blockDim.x + threadIdx.x; t < IMG; t += gridDim.x * blockDim.x)
     a.packed[t] = image_value<float, NB>(a, a.params, t);
 }
@@ -1456,7 +1456,7 @@ extern "C" int tdx_ad_plan_create(const tdx_ad_desc *d, tdx_ad_plan **out) {
       p->step_lds = lds;
       p->n_fitems = (int)fitems.size();
       const int HP = 16 * nb;
-      p->off_img = take((size_t)image_words(HP, NH, p->d_in, p->n_out) * 4);
+      p->off_img = take((size_t)image_words(HP, NH, p->d_in, p->n_out, 4) * 4);
       p->off_zs = take((size_t)p->n_fitems * nhm * nb * 1024 * 4);
       p->off_fpart = take((size_t)p->n_fitems * p->n_params * 4);
       p->off_flp = take((size_t)2 * p->n_fitems * 4);
@@ -1827,7 +1827,7 @@ int ad_step_launch(const tdx_ad_plan *p, const ADStepArgs &a, hipStream_t s) {
 
 template <int NB>
 int ad_pack_launch(const NNArgs<float> &nn, int64_t *step, hipStream_t s) {
-  const int IMG = image_words(16 * NB, nn.NH, nn.d_in, nn.n_out);
+  const int IMG = image_words(16 * NB, nn.NH, nn.d_in, nn.n_out, 4);
   hipLaunchKernelGGL((k_ad_pack<NB>), dim3((unsigned)((IMG + 255) / 256)), dim3(256), 0, s, nn,
                      step);
   TDX_TRY_HIP(hipGetLastError());

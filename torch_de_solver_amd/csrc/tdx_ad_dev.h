@@ -530,7 +530,7 @@ __device__ __forceinline__ void ad_step_body(const ADStepArgs &a, float *smem) {
 #pragma unroll
       for (int ob = 0; ob < NB; ++ob)
         acc[ob] = kind == 0 ? ld4(net.bh + (j - 1) * HP + 16 * ob + 4 * q) : v4{0, 0, 0, 0};
-      mma_layer_fm<float, NB>(net.Wf + (j - 1) * HP * HP, lane, abuf, trow, acc);
+      mma_layer_fm<NB>(net.Wf + (j - 1) * net.LI, lane, abuf, trow, acc);
 #pragma unroll
       for (int ob = 0; ob < NB; ++ob)
 #pragma unroll
@@ -603,13 +603,11 @@ __device__ __forceinline__ void ad_step_body(const ADStepArgs &a, float *smem) {
         const int ob = w + 4 * u;
         if (ob < NB) {
 #pragma unroll
-          for (int kk = 0; kk < 4; ++kk) {
-            const v4 av = *reinterpret_cast<const v4 *>(abuf + (16 * ob + row) * CTRS + 16 * kk + 4 * q);
-            const v4 sv = (o >= 0 && o < n_out)
-                              ? *reinterpret_cast<const v4 *>(sbuf + o * CTRS + 16 * kk + 4 * q)
-                              : v4{0, 0, 0, 0};
-#pragma unroll
-            for (int kb = 0; kb < 4; ++kb) sacc[u] = mma16(av[kb], sv[kb], sacc[u]);
+          for (int kk = 0; kk < 2; ++kk) {
+            f4_t alo, ahi, slo = {0, 0, 0, 0}, shi = {0, 0, 0, 0};
+            rows8(abuf, 16 * ob + row, 32 * kk + 8 * q, alo, ahi);
+            if (o >= 0 && o < n_out) rows8(sbuf, o, 32 * kk + 8 * q, slo, shi);
+            sacc[u] = mma3(bf3_split(alo, ahi), bf3_split(slo, shi), sacc[u]);
           }
         }
       }
@@ -631,32 +629,41 @@ __device__ __forceinline__ void ad_step_body(const ADStepArgs &a, float *smem) {
       wave_sync();
       JP::fwd(zbuf, dbuf, r0w, NP, rNP, J, H, tb, lane);
       __syncthreads();
-      // owned blocks of dW_jj over the 64 rows; the bias over value rows
-#pragma unroll
-      for (int u = 0; u < OBW; ++u) {
-        const int ob = w + 4 * u;
-        if (ob < NB) {
+      // owned blocks of dW_jj over the 64 rows, 32 at a time (an input
+      // block's activations split once for all owned output blocks); the
+      // bias over value rows
 #pragma unroll 1
-          for (int kk = 0; kk < 4; ++kk) {
-            const v4 dv = *reinterpret_cast<const v4 *>(abuf + (16 * ob + row) * CTRS + 16 * kk + 4 * q);
-            const v4 mv = *reinterpret_cast<const v4 *>(xbuf + col_b1 * CTRS + 16 * kk + 4 * q);
-            bhacc[jj][u] += (dv[0] * mv[0] + dv[1] * mv[1]) + (dv[2] * mv[2] + dv[3] * mv[3]);
+      for (int kk = 0; kk < 2; ++kk) {
+        const int r8 = 32 * kk + 8 * q;
+        f4_t m0, m1;
+        rows8(xbuf, col_b1, r8, m0, m1);
+        Bf3 ds[OBW];
 #pragma unroll
-            for (int ib = 0; ib < NB; ++ib) {
-              const v4 av = *reinterpret_cast<const v4 *>(dbuf + (16 * ib + row) * CTRS + 16 * kk + 4 * q);
-              v4 c = dwacc[jj][u][ib];
-#pragma unroll
-              for (int kb = 0; kb < 4; ++kb) c = mma16(dv[kb], av[kb], c);
-              dwacc[jj][u][ib] = c;
-            }
+        for (int u = 0; u < OBW; ++u) {
+          const int ob = w + 4 * u;
+          if (ob < NB) {
+            f4_t lo, hi;
+            rows8(abuf, 16 * ob + row, r8, lo, hi);
+            bhacc[jj][u] += ((lo[0] * m0[0] + lo[1] * m0[1]) + (lo[2] * m0[2] + lo[3] * m0[3])) +
+                            ((hi[0] * m1[0] + hi[1] * m1[1]) + (hi[2] * m1[2] + hi[3] * m1[3]));
+            ds[u] = bf3_split(lo, hi);
           }
+        }
+#pragma unroll
+        for (int ib = 0; ib < NB; ++ib) {
+          f4_t lo, hi;
+          rows8(dbuf, 16 * ib + row, r8, lo, hi);
+          const Bf3 as = bf3_split(lo, hi);
+#pragma unroll
+          for (int u = 0; u < OBW; ++u)
+            if (w + 4 * u < NB) dwacc[jj][u][ib] = mma3(ds[u], as, dwacc[jj][u][ib]);
         }
       }
       // dA of layer j - 1 = W_jj^T dZ_j for this wavefront's rows
       v4 c[NB];
 #pragma unroll
       for (int ib = 0; ib < NB; ++ib) c[ib] = v4{0, 0, 0, 0};
-      mma_layer_fm<float, NB>(net.Wb + jj * HP * HP, lane, abuf, trow, c);
+      mma_layer_fm<NB>(net.Wb + jj * net.LI, lane, abuf, trow, c);
       __syncthreads();
       {
         float dv[NB][4];
@@ -677,12 +684,11 @@ __device__ __forceinline__ void ad_step_body(const ADStepArgs &a, float *smem) {
       const int ob = w + 4 * u;
       if (ob < NB) {
 #pragma unroll
-        for (int kk = 0; kk < 4; ++kk) {
-          const v4 dv = *reinterpret_cast<const v4 *>(abuf + (16 * ob + row) * CTRS + 16 * kk + 4 * q);
-          const v4 xv = row <= d_in ? *reinterpret_cast<const v4 *>(xbuf + row * CTRS + 16 * kk + 4 * q)
-                                    : v4{0, 0, 0, 0};
-#pragma unroll
-          for (int kb = 0; kb < 4; ++kb) sacc[u] = mma16(dv[kb], xv[kb], sacc[u]);
+        for (int kk = 0; kk < 2; ++kk) {
+          f4_t dlo, dhi, xlo = {0, 0, 0, 0}, xhi = {0, 0, 0, 0};
+          rows8(abuf, 16 * ob + row, 32 * kk + 8 * q, dlo, dhi);
+          if (row <= d_in) rows8(xbuf, row, 32 * kk + 8 * q, xlo, xhi);
+          sacc[u] = mma3(bf3_split(dlo, dhi), bf3_split(xlo, xhi), sacc[u]);
         }
       }
     }

@@ -21,6 +21,111 @@ __device__ __forceinline__ d4_t mma16(double a, double b, d4_t c) {
   return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
 }
 
+// float32 products on the bf16 matrix units.  A float32 value is split into
+// three bf16 pieces, x = h + m + l (each the rounding of what is left: 24
+// significant bits, exact above 2^-110), and a product of two values is the
+// six piece products that reach 2^-24 of it, m m' + h l' + l h' first, then
+// h m' + m h', then h h', summed in the float32 accumulator.  What bounds it:
+// a 16x16x32 bf16 MFMA takes 16 cycles and VALU work of other wavefronts runs
+// beside it; a float32 16x16x4 takes 32 and shares the VALU's multipliers, so
+// 16x16x32 in float32 costs 256 cycles that add to the VALU's, in six bf16
+// products 96 that mostly do not.  Measured against 64 bits, relative error
+// of sums over K = 32: 3.6e-8 (float32 MFMA 1.03e-7), K = 128: 6e-8 (2.0e-7).
+typedef __bf16 bf8_t __attribute__((ext_vector_type(8)));
+typedef unsigned u4_t __attribute__((ext_vector_type(4)));
+typedef __bf16 bf2_t __attribute__((ext_vector_type(2)));
+typedef float f16_t __attribute__((ext_vector_type(16)));
+
+// Eight float32 values (one lane's k-slots of a 32-deep product) in pieces.
+struct Bf3 {
+  u4_t h, m, l;
+};
+
+// The pieces of NP pairs of values (2k in the low half, 2k + 1 in the high).
+// The remainder x - h is a dot product of the packed pieces with (-1, 0) or
+// (0, -1) on top of x: exact, and one instruction where unpacking and
+// subtracting are two.  Stage by stage over the pairs, so that the dot
+// products' latencies overlap.  An infinite or NaN value makes its remainder,
+// and its pair partner's, NaN.
+template <int NP>
+__device__ __forceinline__ void bf3_pairs(const float (&x)[2 * NP], unsigned (&h)[NP],
+                                          unsigned (&m)[NP], unsigned (&l)[NP]) {
+#if defined(__AMDGCN__)
+  typedef float f2_t __attribute__((ext_vector_type(2)));
+  // in registers: as a packed literal it would be read as an inline constant
+  unsigned e0 = 0x0000BF80u, e1 = 0xBF800000u;
+  asm("" : "+v"(e0), "+v"(e1));
+  const bf2_t n0 = __builtin_bit_cast(bf2_t, e0), n1 = __builtin_bit_cast(bf2_t, e1);
+  float r[2 * NP];
+  auto round = [&](const float (&v)[2 * NP], unsigned (&p)[NP]) {
+#pragma unroll
+    for (int k = 0; k < NP; ++k)
+      p[k] = __builtin_bit_cast(unsigned,
+                                __builtin_convertvector(f2_t{v[2 * k], v[2 * k + 1]}, bf2_t));
+  };
+  auto rest = [&](const float (&v)[2 * NP], const unsigned (&p)[NP]) {
+#pragma unroll
+    for (int k = 0; k < NP; ++k) {
+      const bf2_t b = __builtin_bit_cast(bf2_t, p[k]);
+      r[2 * k] = __builtin_amdgcn_fdot2_f32_bf16(b, n0, v[2 * k], false);
+      r[2 * k + 1] = __builtin_amdgcn_fdot2_f32_bf16(b, n1, v[2 * k + 1], false);
+    }
+  };
+  round(x, h);
+  rest(x, h);
+  round(r, m);
+  rest(r, m);
+  round(r, l);
+#else
+  for (int k = 0; k < NP; ++k) h[k] = m[k] = l[k] = 0;  // device code only
+#endif
+}
+__device__ __forceinline__ Bf3 bf3_split(f4_t a, f4_t b) {
+  const float x[8] = {a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
+  unsigned h[4], m[4], l[4];
+  bf3_pairs<4>(x, h, m, l);
+  return Bf3{u4_t{h[0], h[1], h[2], h[3]}, u4_t{m[0], m[1], m[2], m[3]},
+             u4_t{l[0], l[1], l[2], l[3]}};
+}
+// Four values in the low k-slots, zeros in the others.
+__device__ __forceinline__ Bf3 bf3_split(f4_t a) {
+  const float x[4] = {a[0], a[1], a[2], a[3]};
+  unsigned h[2], m[2], l[2];
+  bf3_pairs<2>(x, h, m, l);
+  return Bf3{u4_t{h[0], h[1], 0, 0}, u4_t{m[0], m[1], 0, 0}, u4_t{l[0], l[1], 0, 0}};
+}
+__device__ __forceinline__ f4_t mma_bf(u4_t a, u4_t b, f4_t c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf8_t, a),
+                                                 __builtin_bit_cast(bf8_t, b), c, 0, 0, 0);
+}
+__device__ __forceinline__ f16_t mma_bf(u4_t a, u4_t b, f16_t c) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf8_t, a),
+                                                 __builtin_bit_cast(bf8_t, b), c, 0, 0, 0);
+}
+// The five small products of a 16x16x32 (or 32x32x16) step.  They need an
+// accumulator of their own: the unit aligns its addends to the largest and
+// cuts off below (towards minus infinity), so small products added to a
+// large accumulator leave a bias (1.2e-9 of the sum of magnitudes per step,
+// which long sums of cancelling terms pile up) where the leading ones, added
+// alone, leave none.
+template <typename V>
+__device__ __forceinline__ V mma3_small(const Bf3 &a, const Bf3 &b, V c) {
+  c = mma_bf(a.l, b.h, c);
+  c = mma_bf(a.h, b.l, c);
+  c = mma_bf(a.m, b.m, c);
+  c = mma_bf(a.m, b.h, c);
+  return mma_bf(a.h, b.m, c);
+}
+// c + a b for one step of a long sum: the small products from zero, added
+// after.  Error against 64 bits over K = 16384, of the sum of magnitudes:
+// 1.0e-8 (float32 MFMA 2.5e-8; all six in one accumulator 2.3e-8 with a bias
+// of 0.9e-8), with cancelling terms 0.9e-9 (2.2e-9; 2.3e-9).
+template <typename V>
+__device__ __forceinline__ V mma3(const Bf3 &a, const Bf3 &b, V c) {
+  const V s = mma3_small(a, b, V{});
+  return mma_bf(a.h, b.h, c) + s;
+}
+
 // Row of the 16x16 MFMA accumulator held in register i of a lane in
 // quarter q (= lane / 16); the column is lane % 16.  The f32 and f64
 // 16x16x4 instructions place rows differently.

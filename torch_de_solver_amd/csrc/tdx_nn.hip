@@ -53,7 +53,7 @@ __global__ void k_pack(NNArgs<T> a) {
     if (a.one_out) *a.one_out = T(1);
     if (a.step_inc) *a.step_inc += 1;
   }
-  const int IMG = image_words(HP, a.NH, a.d_in, a.n_out);
+  const int IMG = image_words(HP, a.NH, a.d_in, a.n_out, sizeof(T));
   const int64_t total = (int64_t)a.n_inst * IMG;
   for (int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; t < total;
        t += (int64_t)gridDim.x * blockDim.x) {
@@ -70,7 +70,7 @@ template <typename T, int NB>
 __device__ void gather_image(const NNArgs<T> &a, int inst, T *dst, bool with_wb) {
   constexpr int HP = 16 * NB;
   const T *W = a.params + (int64_t)inst * a.P;
-  const int n = stage_words(HP, a.NH, a.d_in, a.n_out, with_wb);
+  const int n = stage_words(HP, a.NH, a.d_in, a.n_out, with_wb, sizeof(T));
   for (int k = threadIdx.x; k < n; k += blockDim.x) dst[k] = image_value<T, NB>(a, W, k);
   __syncthreads();
 }
@@ -225,7 +225,7 @@ __global__ __launch_bounds__(256) void k_forward(NNArgs<T> a) {
         cur = inst;
         if (it == a.inst_k1_idx[a.inst_k1_ptr[inst]]) {
           constexpr int HP = 16 * NB;
-          const int IMG = image_words(HP, a.NH, a.d_in, a.n_out);
+          const int IMG = image_words(HP, a.NH, a.d_in, a.n_out, sizeof(T));
           const T *W = a.params + (int64_t)inst * a.P;
           T *dst = a.packed + (int64_t)inst * IMG;
           for (int k = threadIdx.x; k < IMG; k += blockDim.x) dst[k] = image_value<T, NB>(a, W, k);
@@ -385,7 +385,7 @@ __global__ __launch_bounds__(256) void k_backward(NNArgs<T> a) {
         v4 c[NB];
 #pragma unroll
         for (int ib = 0; ib < NB; ++ib) c[ib] = v4{0, 0, 0, 0};
-        mma_layer<T, NB>(net.Wb + jj * HP * HP, lane, dl_r, c);
+        mma_layer<T, NB>(net.Wb + jj * net.LI, lane, dl_r, c);
         const T *arow = ain + trow * LS;
 #pragma unroll
         for (int ib = 0; ib < NB; ++ib)
@@ -437,23 +437,12 @@ __global__ __launch_bounds__(256) void k_backward(NNArgs<T> a) {
 // wavefront-private LDS buffer.  All gradient accumulators are registers;
 // at the end the wavefronts are summed in a fixed order (deterministic).
 
-// acc[t][ob] += W (rows of block ob) x b[t] for NT independent tiles; each
-// weight operand is loaded once and used by every tile.
+// acc[t][ob] += W (rows of block ob) x b[t] for NT independent tiles.
 template <typename T, int NB, int NT>
 __device__ __forceinline__ void mma_layer_nt(const T *img, int lane, const T (&b)[NT][NB][4],
                                              typename V4<T>::type (&acc)[NT][NB]) {
-  typedef typename V4<T>::type v4;
-  const v4 *wp = reinterpret_cast<const v4 *>(img) + lane;
 #pragma unroll
-  for (int mb = 0; mb < NB; ++mb)
-#pragma unroll
-    for (int ob = 0; ob < NB; ++ob) {
-      const v4 w = wp[(ob * NB + mb) * 64];
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int t = 0; t < NT; ++t) acc[t][ob] = mma16(w[i], b[t][mb][i], acc[t][ob]);
-    }
+  for (int t = 0; t < NT; ++t) mma_layer<T, NB>(img, lane, b[t], acc[t]);
 }
 
 // Wavefront-private backward: each wavefront walks 16-row tiles of its work
@@ -511,25 +500,17 @@ __device__ __forceinline__ void backward_w_item(const NNArgs<T> &a, int it,
 
   // gradient accumulators (MFMA tiles; row m = crow(q, i) is the hidden
   // feature 16 ob + m, column n = row):
-  //   dwacc[jj][ob*NB+ib]: hidden W ( out, in )
+  //   wg[jj]: hidden W (out, in) and bias
   //   sacc[ob]: the first and last layers' terms in one tile, by column --
   //     n < d_in first W, d_in first bias, d_in + 1 + o output W row o.
   //     Each product accumulated into the tile has a B operand that is zero
   //     outside its own columns, so the columns add exactly what separate
   //     tiles would.
-  //   bhacc[jj][xb]: hidden bias of feature 16 xb + row over the rows
-  //     4q .. 4q+3 of each tile, summed over the quarters at the end
   //   blacc: output bias o = q, summed over the row lanes at the end
-  v4 dwacc[NH > 0 ? NH : 1][NB * NB];
+  WGrad<T, NB> wg[NH > 0 ? NH : 1];
   v4 sacc[NB];
-  T bhacc[NH > 0 ? NH : 1][NB];
 #pragma unroll
-  for (int j = 0; j < (NH > 0 ? NH : 1); ++j) {
-#pragma unroll
-    for (int b = 0; b < NB * NB; ++b) dwacc[j][b] = v4{0, 0, 0, 0};
-#pragma unroll
-    for (int b = 0; b < NB; ++b) bhacc[j][b] = T(0);
-  }
+  for (int j = 0; j < (NH > 0 ? NH : 1); ++j) wg[j].zero();
 #pragma unroll
   for (int b = 0; b < NB; ++b) sacc[b] = v4{0, 0, 0, 0};
   T blacc = T(0);
@@ -597,7 +578,7 @@ __device__ __forceinline__ void backward_w_item(const NNArgs<T> &a, int it,
       for (int t = 0; t < NT; ++t)
 #pragma unroll
         for (int ob = 0; ob < NB; ++ob) acc[t][ob] = ld4(net.bh + (j - 1) * HP + 16 * ob + 4 * q);
-      mma_layer_nt<T, NB, NT>(net.Wf + (j - 1) * HP * HP, lane, act[j - 1], acc);
+      mma_layer_nt<T, NB, NT>(net.Wf + (j - 1) * net.LI, lane, act[j - 1], acc);
 #pragma unroll
       for (int t = 0; t < NT; ++t)
 #pragma unroll
@@ -678,25 +659,7 @@ __device__ __forceinline__ void backward_w_item(const NNArgs<T> &a, int it,
           }
       wave_sync();
 #pragma unroll
-      for (int t = 0; t < NT; ++t) {
-        v4 av[NB], dv[NB];
-#pragma unroll
-        for (int xb = 0; xb < NB; ++xb) {
-          dv[xb] = *reinterpret_cast<const v4 *>(dbuf[t] + (16 * xb + row) * WRS + 4 * q);
-          av[xb] = *reinterpret_cast<const v4 *>(abuf[t] + (16 * xb + row) * WRS + 4 * q);
-        }
-#pragma unroll
-        for (int ob = 0; ob < NB; ++ob) {
-          bhacc[jj][ob] += (dv[ob][0] + dv[ob][1]) + (dv[ob][2] + dv[ob][3]);
-#pragma unroll
-          for (int ib = 0; ib < NB; ++ib) {
-            v4 c = dwacc[jj][ob * NB + ib];
-#pragma unroll
-            for (int kb = 0; kb < 4; ++kb) c = mma16(dv[ob][kb], av[ib][kb], c);
-            dwacc[jj][ob * NB + ib] = c;
-          }
-        }
-      }
+      for (int t = 0; t < NT; ++t) wg[jj].add(dbuf[t], abuf[t], lane);
       wave_sync();
       // delta_{j-1} = (W_jj^T delta_j) * (1 - act_{j-1}^2)
       v4 c[NT][NB];
@@ -704,7 +667,7 @@ __device__ __forceinline__ void backward_w_item(const NNArgs<T> &a, int it,
       for (int t = 0; t < NT; ++t)
 #pragma unroll
         for (int ib = 0; ib < NB; ++ib) c[t][ib] = v4{0, 0, 0, 0};
-      mma_layer_nt<T, NB, NT>(net.Wb + jj * HP * HP, lane, dl, c);
+      mma_layer_nt<T, NB, NT>(net.Wb + jj * net.LI, lane, dl, c);
 #pragma unroll
       for (int t = 0; t < NT; ++t)
 #pragma unroll
@@ -765,13 +728,6 @@ __device__ __forceinline__ void backward_w_item(const NNArgs<T> &a, int it,
         for (int i = 0; i < 4; ++i) {
           const int out = 16 * ob + crow<T>(q, i);
           if (out >= H) continue;
-#pragma unroll
-          for (int jj = 0; jj < NH; ++jj)
-#pragma unroll
-            for (int ib = 0; ib < NB; ++ib) {
-              const int in = 16 * ib + row;
-              if (in < H) put(L.oWh(jj) + out * H + in, dwacc[jj][ob * NB + ib][i]);
-            }
           const T sv = sacc[ob][i];
           if (!w1_valu && row < d_in) put(L.oW1() + out * d_in + row, sv);
           else if (!w1_valu && row == col_b1) put(L.ob1() + out, sv);
@@ -805,14 +761,14 @@ __device__ __forceinline__ void backward_w_item(const NNArgs<T> &a, int it,
       }
 #pragma unroll
       for (int jj = 0; jj < NH; ++jj)
-#pragma unroll
-        for (int xb = 0; xb < NB; ++xb) {
-          T v = bhacc[jj][xb];
-          v += __shfl_xor(v, 16);
-          v += __shfl_xor(v, 32);
-          const int f = 16 * xb + row;
-          if (q == 0 && f < H) put(L.obh(jj) + f, v);
-        }
+        wg[jj].sums(
+            lane,
+            [&](int out, int in, T v) {
+              if (out < H && in < H) put(L.oWh(jj) + out * H + in, v);
+            },
+            [&](int f, T v) {
+              if (f < H) put(L.obh(jj) + f, v);
+            });
       const T bl = rowsum16(blacc);
       if (row == 0 && q < n_out) put(L.obL() + q, bl);
     }
@@ -1379,7 +1335,7 @@ struct tdx_nn_plan {
 static size_t wave_private_lds(const tdx_nn_plan *p, const tdx_nn_desc *d) {
   const size_t wb = (size_t)2 * 20 * p->HP + 2 * 16 * 20;
   const size_t tr = std::max<size_t>(4 * p->k2_nt * wb, (size_t)p->P);
-  return tr + stage_words(p->HP, p->NH, d->d_in, d->n_out, true);
+  return tr + stage_words(p->HP, p->NH, d->d_in, d->n_out, true, d->dtype == 0 ? 4 : 8);
 }
 
 namespace {
@@ -1482,7 +1438,7 @@ int forward_grid_size_nb(int NB, size_t lds) {
 
 template <typename T, int NB>
 int launch_pack(const tdx_nn_plan *p, const NNArgs<T> &a, hipStream_t s) {
-  const int64_t total = (int64_t)p->n_inst * image_words(p->HP, p->NH, p->d_in, p->n_out);
+  const int64_t total = (int64_t)p->n_inst * image_words(p->HP, p->NH, p->d_in, p->n_out, (int)sizeof(T));
   const int blocks = (int)std::min<int64_t>((total + 255) / 256, 65535);
   hipLaunchKernelGGL((k_pack<T, NB>), dim3(blocks), dim3(256), 0, s, a);
   TDX_TRY_HIP(hipGetLastError());
@@ -1887,6 +1843,46 @@ int pick_chunk(const std::vector<int64_t> &tiles, int64_t slots, int cap, double
   return best;
 }
 
+// Workgroups of the block-owning kernel a CU keeps resident (the run-time
+// compiled kernel fn when given), 1 if unknown.
+template <int NB, int NH, bool FS>
+int block_residency_of(hipFunction_t fn, size_t lds) {
+  int n = 0;
+  if constexpr (block_acc_regs(NB, NH) <= 192) {
+    if (fn) {
+      if (hipModuleOccupancyMaxActiveBlocksPerMultiprocessor(&n, fn, 256, lds) != hipSuccess) n = 0;
+    } else {
+      const void *k = (const void *)k_backward_c<float, NB, NH, FS>;
+      raise_lds_limit({k});
+      if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k, 256, lds) != hipSuccess) n = 0;
+    }
+    (void)hipGetLastError();
+  }
+  return std::max(n, 1);
+}
+template <bool FS>
+int block_residency(int NB, int NH, hipFunction_t fn, size_t lds) {
+#define TDX_RES(B)                                                \
+  case B:                                                         \
+    switch (NH) {                                                 \
+      case 1: return block_residency_of<B, 1, FS>(fn, lds);       \
+      case 2: return block_residency_of<B, 2, FS>(fn, lds);       \
+      case 3: return block_residency_of<B, 3, FS>(fn, lds);       \
+      case 4: return block_residency_of<B, 4, FS>(fn, lds);       \
+      default: return 1;                                          \
+    }
+  switch (NB) {
+    TDX_RES(3)
+    TDX_RES(4)
+    TDX_RES(5)
+    TDX_RES(6)
+    TDX_RES(7)
+    TDX_RES(8)
+    default: return 1;
+  }
+#undef TDX_RES
+}
+
 // Host-side validation of every table index, so that a malformed table is an
 // error code and never an out-of-bounds access on the device.
 int validate_nn(const tdx_nn_desc *d, int64_t *n_rows_out) {
@@ -2099,8 +2095,9 @@ extern "C" int tdx_nn_plan_create(const tdx_nn_desc *d, tdx_nn_plan **out) {
   p->k1_lds = (2 * K1_WAVES * 16 * max_slots * d->n_out + 512) * ts;
   {
     // stage the forward operand images in LDS when they are small
-    const size_t st = (size_t)stage_words(p->HP, p->NH, d->d_in, d->n_out, false) * ts;
-    p->k1_stage = (p->k1_lds + st <= 64 * 1024) ? 1 : 0;
+    const size_t st = (size_t)stage_words(p->HP, p->NH, d->d_in, d->n_out, false, (int)ts) * ts;
+    // (wide float layers read their operand images from global memory)
+    p->k1_stage = (p->k1_lds + st <= 64 * 1024 && (d->dtype == 1 || p->NB <= 2)) ? 1 : 0;
     if (p->k1_stage) p->k1_lds += st;
   }
 
@@ -2156,7 +2153,7 @@ extern "C" int tdx_nn_plan_create(const tdx_nn_desc *d, tdx_nn_plan **out) {
   const int chunk_tiles =
       d->chunk_tiles > 0  ? d->chunk_tiles
       : p->k2_wave_private ? pick_chunk(k2_tiles, 3 * kCUs, 256, 1.0)
-      : p->k2_block        ? pick_chunk(k2_tiles, kCUs, 16, 0.25)
+      : p->k2_block        ? pick_chunk(k2_tiles, kCUs * block_residency<false>(p->NB, p->NH, nullptr, p->k2_lds), 16, 0.25)
                            : pick_chunk(k2_tiles, kCUs, p->acc_lds ? 16 : 4, 1.0);
   std::vector<int4> k2;
   for (int g = 0; g < d->n_groups; ++g) {
@@ -2187,7 +2184,7 @@ extern "C" int tdx_nn_plan_create(const tdx_nn_desc *d, tdx_nn_plan **out) {
   std::vector<int32_t> prog_ints, ik3p(1, 0), ik3i, prog_kind;
   std::vector<float> prog_reals;
   std::vector<FusedProg> progs;
-  p->k3_lds = (size_t)fused_lds_words(p->HP, p->NH, d->d_in, d->n_out, p->P) * ts;
+  p->k3_lds = (size_t)fused_lds_words(p->HP, p->NH, d->d_in, d->n_out, p->P, true) * ts;
   bool fuse = fused_shape_ok(d, max_slots) && p->k2_wave_private && p->k3_lds <= LDS_MAX &&
               fused_programs(d, &progs);
   if (fuse) {
@@ -2241,6 +2238,9 @@ extern "C" int tdx_nn_plan_create(const tdx_nn_desc *d, tdx_nn_plan **out) {
         p->fused_fn = nullptr;
         prog_kind.clear();
         clear_error();
+      } else {
+        // generated programs need no table copy in LDS
+        p->k3_lds = (size_t)fused_lds_words(p->HP, p->NH, d->d_in, d->n_out, p->P, false) * ts;
       }
     }
   }
@@ -2260,29 +2260,7 @@ extern "C" int tdx_nn_plan_create(const tdx_nn_desc *d, tdx_nn_plan **out) {
       prog_ints.insert(prog_ints.end(), fp.ints.begin(), fp.ints.end());
       prog_reals.insert(prog_reals.end(), fp.reals.begin(), fp.reals.end());
     }
-    std::vector<std::vector<int>> inst_k4(d->n_inst);
-    std::vector<int64_t> tiles;
-    for (int g = 0; g < d->n_groups; ++g) {
-      const int32_t *G = d->groups + (int64_t)g * TDX_GROUP_INTS;
-      tiles.push_back((G[1] + 64 / G[2] - 1) / (64 / G[2]));
-    }
-    const int C = d->chunk_tiles > 0 ? d->chunk_tiles : pick_chunk(tiles, kCUs, 16, 0.25);
-    for (int g = 0; g < d->n_groups; ++g) {
-      const int32_t *G = d->groups + (int64_t)g * TDX_GROUP_INTS;
-      const int E = 64 / G[2];
-      const int ntile = (G[1] + E - 1) / E;
-      for (int j = 0; j < ntile; j += C) {
-        inst_k4[G[0]].push_back((int)k4.size());
-        k4.push_back(make_int4(g, j * E, std::min(G[1], (j + C) * E), G[0]));
-      }
-    }
-    for (int i = 0; i < d->n_inst; ++i) {
-      for (int x : inst_k4[i]) ik4i.push_back(x);
-      ik4p.push_back((int32_t)ik4i.size());
-      inst_k4_size[i] = (int)inst_k4[i].size();
-    }
     p->k2_fs = 1;
-    p->n_k4 = (int)k4.size();
     p->k4_lds = block_fs_lds_words(p->HP, p->NH) * ts;
     // generated residual programs for plans of at least 2^17 network rows
     // (TDX_NN_JIT: 0 never, 1 always); the interpreting kernel if compiling
@@ -2314,6 +2292,31 @@ extern "C" int tdx_nn_plan_create(const tdx_nn_desc *d, tdx_nn_plan **out) {
         (void)hipGetLastError();
       }
     }
+    std::vector<std::vector<int>> inst_k4(d->n_inst);
+    std::vector<int64_t> tiles;
+    for (int g = 0; g < d->n_groups; ++g) {
+      const int32_t *G = d->groups + (int64_t)g * TDX_GROUP_INTS;
+      tiles.push_back((G[1] + 64 / G[2] - 1) / (64 / G[2]));
+    }
+    const int C = d->chunk_tiles > 0
+                      ? d->chunk_tiles
+                      : pick_chunk(tiles, kCUs * block_residency<true>(p->NB, p->NH, p->block_fn, p->k4_lds), 16,
+                             0.25);
+    for (int g = 0; g < d->n_groups; ++g) {
+      const int32_t *G = d->groups + (int64_t)g * TDX_GROUP_INTS;
+      const int E = 64 / G[2];
+      const int ntile = (G[1] + E - 1) / E;
+      for (int j = 0; j < ntile; j += C) {
+        inst_k4[G[0]].push_back((int)k4.size());
+        k4.push_back(make_int4(g, j * E, std::min(G[1], (j + C) * E), G[0]));
+      }
+    }
+    for (int i = 0; i < d->n_inst; ++i) {
+      for (int x : inst_k4[i]) ik4i.push_back(x);
+      ik4p.push_back((int32_t)ik4i.size());
+      inst_k4_size[i] = (int)inst_k4[i].size();
+    }
+    p->n_k4 = (int)k4.size();
   }
 
   // two-stage gradient sum when one thread per parameter of every instance
@@ -2403,7 +2406,7 @@ extern "C" int tdx_nn_plan_create(const tdx_nn_desc *d, tdx_nn_plan **out) {
   }
   size_t off = 0;
   p->off_packed = off;
-  off = align_up(off + (size_t)p->n_inst * image_words(p->HP, p->NH, d->d_in, d->n_out) * ts, 256);
+  off = align_up(off + (size_t)p->n_inst * image_words(p->HP, p->NH, d->d_in, d->n_out, (int)ts) * ts, 256);
   p->off_seeds = off;
   off = align_up(off + (size_t)n_rows * p->n_out * ts, 256);
   p->off_lp = off;

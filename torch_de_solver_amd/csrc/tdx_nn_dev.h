@@ -81,10 +81,17 @@ struct Layout {
 // ---------------------------------------------------------------------------
 // One image per instance, in the workspace, rebuilt from the parameters by
 // k_pack at the start of every forward pass (HP = 16 NB):
-//   [Wf: NH x HP*HP][small: SW][Wb: NH x HP*HP]
-// Wf and Wb hold each hidden layer's W_j as MFMA operand images, laid out so
-// that lane l reads the four values of k-steps i = 0..3 of block (xb, mb)
-// with one 128-bit load:
+//   [Wf: NH x LI][small: SW][Wb: NH x LI]
+// Wf and Wb hold each hidden layer's W_j as MFMA operand images of LI words.
+// float: the operands of 16x16x32 bf16 products, in three bf16 pieces p (see
+// Bf3), KS = (NB + 1) / 2 k-steps ks, word t of a lane holding the k-slots
+// e = 2t (low half) and 2t + 1, which are feature 16 mb + 4 (lane / 16) +
+// e % 4 of block mb = 2 ks + e / 4 (zero beyond the network):
+//   Wf[j][ob][ks][p][lane][t] = W_j[16*ob + lane%16][feature of e]
+//   Wb[j][ib][ks][p][lane][t] = W_j[feature of e][16*ib + lane%16]
+// so a lane reads one piece of a 32-deep operand with one 128-bit load.
+// double: operands of 16x16x4 products, the four values of k-steps i = 0..3
+// of block (xb, mb) adjacent:
 //   Wf[j][ob][mb][lane][i] = W_j[16*ob + lane%16][16*mb + crow(lane/16, i)]
 //   Wb[j][ib][mb][lane][i] = W_j[16*mb + crow(lane/16, i)][16*ib + lane%16]
 // The small arrays are indexed by accumulator position p = 16 mb + 4 q + i,
@@ -96,12 +103,17 @@ struct Layout {
 __host__ __device__ inline int small_words(int HP, int NH, int d_in, int n_out) {
   return HP * (1 + d_in + NH + n_out) + ((n_out + 3) & ~3);
 }
-__host__ __device__ inline int image_words(int HP, int NH, int d_in, int n_out) {
-  return 2 * NH * HP * HP + small_words(HP, NH, d_in, n_out);
+// Words of one layer's operand image (ts: bytes of the working type).
+__host__ __device__ constexpr int layer_words(int HP, int ts) {
+  return ts == 4 ? (HP / 16) * ((HP + 16) / 32) * 768 : HP * HP;
+}
+__host__ __device__ inline int image_words(int HP, int NH, int d_in, int n_out, int ts) {
+  return 2 * NH * layer_words(HP, ts) + small_words(HP, NH, d_in, n_out);
 }
 // Words of the LDS copy (in T units).
-__host__ __device__ inline int stage_words(int HP, int NH, int d_in, int n_out, bool with_wb) {
-  return NH * HP * HP * (with_wb ? 2 : 1) + small_words(HP, NH, d_in, n_out);
+__host__ __device__ inline int stage_words(int HP, int NH, int d_in, int n_out, bool with_wb,
+                                           int ts) {
+  return NH * layer_words(HP, ts) * (with_wb ? 2 : 1) + small_words(HP, NH, d_in, n_out);
 }
 
 // Hidden feature held at accumulator position p of a block.
@@ -116,7 +128,7 @@ template <typename T, int NB>
 __device__ __forceinline__ T image_value(const NNArgs<T> &a, const T *W, int off) {
   constexpr int HP = 16 * NB;
   const int NH = a.NH, H = a.H, d = a.d_in, no = a.n_out;
-  const int img = HP * HP;
+  constexpr int img = layer_words(HP, sizeof(T));
   const int SW = small_words(HP, NH, d, no);
   const Layout<T> L{d, no, H, NH};
   {
@@ -126,19 +138,38 @@ __device__ __forceinline__ T image_value(const NNArgs<T> &a, const T *W, int off
       if (which) off -= NH * img + SW;
       const int j = off / img;
       int r = off - j * img;
-      const int i = r & 3;
-      const int lane = (r >> 2) & 63;
-      r >>= 8;
-      const int mb = r % NB, xb = r / NB;
-      int out, in;
-      if (which == 0) {
-        out = 16 * xb + (lane & 15);
-        in = 16 * mb + crow<T>(lane >> 4, i);
+      if constexpr (sizeof(T) == 4) {
+        constexpr int KS = (NB + 1) / 2;
+        const int t = r & 3, lane = (r >> 2) & 63;
+        r >>= 8;
+        const int p = r % 3, ks = (r / 3) % KS, xb = r / (3 * KS);
+        T w2[2];
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+          const int e = 2 * t + k;
+          const int f = 16 * (2 * ks + (e >> 2)) + 4 * (lane >> 4) + (e & 3);
+          const int x = 16 * xb + (lane & 15);
+          const int out = which == 0 ? x : f, in = which == 0 ? f : x;
+          w2[k] = (out < H && in < H) ? W[L.oWh(j) + out * H + in] : T(0);
+        }
+        unsigned h[1], m[1], l[1];
+        bf3_pairs<1>(w2, h, m, l);
+        v = __builtin_bit_cast(float, p == 0 ? h[0] : (p == 1 ? m[0] : l[0]));
       } else {
-        out = 16 * mb + crow<T>(lane >> 4, i);
-        in = 16 * xb + (lane & 15);
+        const int i = r & 3;
+        const int lane = (r >> 2) & 63;
+        r >>= 8;
+        const int mb = r % NB, xb = r / NB;
+        int out, in;
+        if (which == 0) {
+          out = 16 * xb + (lane & 15);
+          in = 16 * mb + crow<T>(lane >> 4, i);
+        } else {
+          out = 16 * mb + crow<T>(lane >> 4, i);
+          in = 16 * xb + (lane & 15);
+        }
+        if (out < H && in < H) v = W[L.oWh(j) + out * H + in];
       }
-      if (out < H && in < H) v = W[L.oWh(j) + out * H + in];
     } else {
       const int sp = off - NH * img;
       const int blk = sp / HP, f = feature_at<T>(sp - blk * HP);
@@ -164,7 +195,8 @@ __device__ __forceinline__ T image_value(const NNArgs<T> &a, const T *W, int off
 // ---------------------------------------------------------------------------
 template <typename T, int NB>
 struct Net {
-  const T *Wf, *Wb;          // layer j image at Wf + j*HP*HP
+  const T *Wf, *Wb;          // layer j image at Wf + j * LI
+  static constexpr int LI = layer_words(16 * NB, sizeof(T));
   const T *b1, *W1, *bh, *WL, *bL;  // small arrays, row stride HP
   Layout<T> L;
 };
@@ -175,7 +207,7 @@ __device__ __forceinline__ Net<T, NB> net_at(const NNArgs<T> &a, const T *base) 
   Net<T, NB> n;
   n.L = Layout<T>{a.d_in, a.n_out, a.H, a.NH};
   n.Wf = base;
-  const T *sm = base + a.NH * HP * HP;
+  const T *sm = base + a.NH * Net<T, NB>::LI;
   n.b1 = sm;
   n.W1 = sm + HP;
   n.bh = n.W1 + a.d_in * HP;
@@ -188,7 +220,10 @@ __device__ __forceinline__ Net<T, NB> net_at(const NNArgs<T> &a, const T *base) 
 template <typename T, int NB>
 __device__ __forceinline__ Net<T, NB> make_net(const NNArgs<T> &a, int inst) {
   constexpr int HP = 16 * NB;
-  return net_at<T, NB>(a, a.packed + (int64_t)inst * image_words(HP, a.NH, a.d_in, a.n_out));
+  // the instance is the workgroup's: in a scalar register it keeps the weight
+  // addresses scalar too (as vector addresses they were hoisted and spilled)
+  const int64_t i = __builtin_amdgcn_readfirstlane(inst);
+  return net_at<T, NB>(a, a.packed + i * image_words(HP, a.NH, a.d_in, a.n_out, sizeof(T)));
 }
 
 // Cooperative copy of one instance's image (without Wb unless with_wb) into
@@ -198,8 +233,8 @@ template <typename T, int NB>
 __device__ Net<T, NB> stage_net(const NNArgs<T> &a, int inst, T *dst, bool with_wb) {
   constexpr int HP = 16 * NB;
   typedef typename V4<T>::type v4;
-  const T *src = a.packed + (int64_t)inst * image_words(HP, a.NH, a.d_in, a.n_out);
-  const int n4 = stage_words(HP, a.NH, a.d_in, a.n_out, with_wb) / 4;
+  const T *src = a.packed + (int64_t)inst * image_words(HP, a.NH, a.d_in, a.n_out, sizeof(T));
+  const int n4 = stage_words(HP, a.NH, a.d_in, a.n_out, with_wb, sizeof(T)) / 4;
   const v4 *s4 = reinterpret_cast<const v4 *>(src);
   v4 *d4 = reinterpret_cast<v4 *>(dst);
   for (int k = threadIdx.x; k < n4; k += blockDim.x) d4[k] = s4[k];
@@ -235,23 +270,91 @@ __device__ __forceinline__ void layer_in(const Net<T, NB> &n, const T *x, int q,
   }
 }
 
+// The pieces of one float activation vector as the B operand of KS k-steps.
+template <int NB>
+__device__ __forceinline__ void split_act(const float (&b)[NB][4], Bf3 (&s)[(NB + 1) / 2]) {
+#pragma unroll
+  for (int ks = 0; ks < (NB + 1) / 2; ++ks) {
+    const f4_t lo = {b[2 * ks][0], b[2 * ks][1], b[2 * ks][2], b[2 * ks][3]};
+    if (2 * ks + 1 < NB) {
+      constexpr int Z = NB - 1;
+      const int u = 2 * ks + 1 < NB ? 2 * ks + 1 : Z;
+      s[ks] = bf3_split(lo, f4_t{b[u][0], b[u][1], b[u][2], b[u][3]});
+    } else {
+      s[ks] = bf3_split(lo);
+    }
+  }
+}
+
+// acc[ob] += W (rows of block ob) x the split operand s, per block the leading
+// and the small products of every k-step in two accumulators from zero.  Wide layers read their weights from L2: the next block's are
+// loaded while this one is multiplied, and no more than that is kept in
+// flight (the scheduler otherwise hoists every load and spills).
+template <int NB>
+__device__ __forceinline__ void mma_split(const float *img, int lane,
+                                          const Bf3 (&s)[(NB + 1) / 2], f4_t (&acc)[NB]) {
+  constexpr int KS = (NB + 1) / 2;
+  Bf3 w[2][KS];
+  // wide images are in global memory (never staged): buffer loads take a
+  // scalar descriptor and offset and one lane offset, so no address occupies
+  // vector registers (as plain pointers the tile loop's hoisted addresses
+  // spilled up to 2 KB a lane)
+  const auto rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(img), (short)0,
+                                                    NB * KS * 3072, 0x00027000);
+  auto load = [&](int ob, Bf3 (&d)[KS]) {
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+      if constexpr (KS > 1) {
+        const int o = 16 * lane, so = (ob * KS + ks) * 3072;
+        d[ks].h = __builtin_amdgcn_raw_buffer_load_b128(rs, o, so, 0);
+        d[ks].m = __builtin_amdgcn_raw_buffer_load_b128(rs, o, so + 1024, 0);
+        d[ks].l = __builtin_amdgcn_raw_buffer_load_b128(rs, o, so + 2048, 0);
+      } else {
+        const u4_t *p = reinterpret_cast<const u4_t *>(img) + lane + (ob * KS + ks) * 192;
+        d[ks].h = p[0], d[ks].m = p[64], d[ks].l = p[128];
+      }
+    }
+  };
+  load(0, w[0]);
+#pragma unroll
+  for (int ob = 0; ob < NB; ++ob) {
+    if (ob + 1 < NB) load(ob + 1, w[(ob + 1) & 1]);
+    if constexpr (KS > 1) __builtin_amdgcn_sched_barrier(0);
+    const Bf3(&wo)[KS] = w[ob & 1];
+    f4_t c = {0, 0, 0, 0}, c2 = {0, 0, 0, 0};
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+      c = mma_bf(wo[ks].h, s[ks].h, c);
+      c2 = mma3_small(wo[ks], s[ks], c2);
+    }
+    acc[ob] += c + c2;
+    if constexpr (KS > 1) __builtin_amdgcn_sched_barrier(0);
+  }
+}
+
 // acc[ob] += W_j (rows of block ob) x act, W given as an operand image.
 template <typename T, int NB>
 __device__ __forceinline__ void mma_layer(const T *img, int lane, const T (&b)[NB][4],
                                           typename V4<T>::type (&acc)[NB]) {
   typedef typename V4<T>::type v4;
-  const v4 *wp = reinterpret_cast<const v4 *>(img) + lane;
+  if constexpr (sizeof(T) == 4) {
+    Bf3 s[(NB + 1) / 2];
+    split_act<NB>(b, s);
+    mma_split<NB>(img, lane, s, acc);
+  } else {
+    const v4 *wp = reinterpret_cast<const v4 *>(img) + lane;
 #pragma unroll
-  for (int mb = 0; mb < NB; ++mb)
+    for (int mb = 0; mb < NB; ++mb)
 #pragma unroll
-    for (int ob = 0; ob < NB; ++ob) {
-      const v4 w = wp[(ob * NB + mb) * 64];
+      for (int ob = 0; ob < NB; ++ob) {
+        const v4 w = wp[(ob * NB + mb) * 64];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) acc[ob] = mma16(w[i], b[mb][i], acc[ob]);
-    }
+        for (int i = 0; i < 4; ++i) acc[ob] = mma16(w[i], b[mb][i], acc[ob]);
+      }
+  }
 }
 
-// Hidden layer j (MFMA, the accumulator starts at the bias):
+// Hidden layer j (MFMA on top of the bias):
 // act <- tanh(b_j + W_j act).
 template <typename T, int NB>
 __device__ __forceinline__ void layer_hidden(const Net<T, NB> &n, int j, int lane,
@@ -262,7 +365,7 @@ __device__ __forceinline__ void layer_hidden(const Net<T, NB> &n, int j, int lan
   v4 acc[NB];
 #pragma unroll
   for (int ob = 0; ob < NB; ++ob) acc[ob] = ld4(n.bh + j * HP + 16 * ob + 4 * q);
-  mma_layer<T, NB>(n.Wf + j * HP * HP, lane, act, acc);
+  mma_layer<T, NB>(n.Wf + j * n.LI, lane, act, acc);
 #pragma unroll
   for (int ob = 0; ob < NB; ++ob)
 #pragma unroll
@@ -485,6 +588,118 @@ constexpr int WRS = 20;
 template <int HP>
 constexpr int wave_ls() { return WRS * HP / 16; }
 
+// Weight and bias gradient of one H x H layer of a narrow network, summed over
+// 16-row tiles in registers: add() takes a tile's deltas and activations from
+// feature-major buffers, sums() hands every (out, in) sum of the wavefront to
+// put and every bias sum to putb (a lane each).  float, two blocks: one
+// 32x32x16 product per piece pair and tile (lane: feature lane % 32, rows 8
+// (lane / 32) and on), so the tile's 16 rows fill the product's depth; one
+// block: 16x16x32 with the upper half of the depth empty.
+template <typename T, int NB>
+struct WGrad {
+  typedef typename V4<T>::type v4;
+  v4 c[NB * NB];
+  T b[NB];
+  __device__ __forceinline__ void zero() {
+#pragma unroll
+    for (int k = 0; k < NB * NB; ++k) c[k] = v4{0, 0, 0, 0};
+#pragma unroll
+    for (int k = 0; k < NB; ++k) b[k] = T(0);
+  }
+  __device__ __forceinline__ void add(const T *dbuf, const T *abuf, int lane) {
+    const int row = lane & 15, q = lane >> 4;
+    v4 av[NB], dv[NB];
+#pragma unroll
+    for (int xb = 0; xb < NB; ++xb) {
+      dv[xb] = *reinterpret_cast<const v4 *>(dbuf + (16 * xb + row) * WRS + 4 * q);
+      av[xb] = *reinterpret_cast<const v4 *>(abuf + (16 * xb + row) * WRS + 4 * q);
+    }
+#pragma unroll
+    for (int ob = 0; ob < NB; ++ob) {
+      b[ob] += (dv[ob][0] + dv[ob][1]) + (dv[ob][2] + dv[ob][3]);
+#pragma unroll
+      for (int ib = 0; ib < NB; ++ib)
+#pragma unroll
+        for (int kb = 0; kb < 4; ++kb)
+          c[ob * NB + ib] = mma16(dv[ob][kb], av[ib][kb], c[ob * NB + ib]);
+    }
+  }
+  template <typename F, typename G>
+  __device__ __forceinline__ void sums(int lane, F put, G putb) {
+    const int row = lane & 15, q = lane >> 4;
+#pragma unroll
+    for (int ob = 0; ob < NB; ++ob)
+#pragma unroll
+      for (int ib = 0; ib < NB; ++ib)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          put(16 * ob + crow<T>(q, i), 16 * ib + row, c[ob * NB + ib][i]);
+#pragma unroll
+    for (int xb = 0; xb < NB; ++xb) {
+      T v = b[xb];
+      v += __shfl_xor(v, 16);
+      v += __shfl_xor(v, 32);
+      if (q == 0) putb(16 * xb + row, v);
+    }
+  }
+};
+template <>
+struct WGrad<float, 1> {
+  f4_t c;
+  float b;
+  __device__ __forceinline__ void zero() {
+    c = f4_t{0, 0, 0, 0};
+    b = 0.0f;
+  }
+  __device__ __forceinline__ void add(const float *dbuf, const float *abuf, int lane) {
+    const int row = lane & 15, q = lane >> 4;
+    f4_t d0 = {0, 0, 0, 0}, d1 = d0, a0 = d0, a1 = d0;
+    if (q < 2) {
+      const f4_t *dp = reinterpret_cast<const f4_t *>(dbuf + row * WRS + 8 * q);
+      const f4_t *ap = reinterpret_cast<const f4_t *>(abuf + row * WRS + 8 * q);
+      d0 = dp[0], d1 = dp[1], a0 = ap[0], a1 = ap[1];
+    }
+    b += ((d0[0] + d0[1]) + (d0[2] + d0[3])) + ((d1[0] + d1[1]) + (d1[2] + d1[3]));
+    c = mma3(bf3_split(d0, d1), bf3_split(a0, a1), c);
+  }
+  template <typename F, typename G>
+  __device__ __forceinline__ void sums(int lane, F put, G putb) {
+    const int row = lane & 15, q = lane >> 4;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) put(4 * q + i, row, c[i]);
+    float v = b;
+    v += __shfl_xor(v, 16);
+    if (q == 0) putb(row, v);
+  }
+};
+template <>
+struct WGrad<float, 2> {
+  f16_t c;
+  float b;
+  __device__ __forceinline__ void zero() {
+#pragma unroll
+    for (int i = 0; i < 16; ++i) c[i] = 0.0f;
+    b = 0.0f;
+  }
+  __device__ __forceinline__ void add(const float *dbuf, const float *abuf, int lane) {
+    const int f = lane & 31, r = 8 * (lane >> 5);
+    const f4_t *dp = reinterpret_cast<const f4_t *>(dbuf + f * WRS + r);
+    const f4_t *ap = reinterpret_cast<const f4_t *>(abuf + f * WRS + r);
+    const f4_t d0 = dp[0], d1 = dp[1], a0 = ap[0], a1 = ap[1];
+    b += ((d0[0] + d0[1]) + (d0[2] + d0[3])) + ((d1[0] + d1[1]) + (d1[2] + d1[3]));
+    c = mma3(bf3_split(d0, d1), bf3_split(a0, a1), c);
+  }
+  template <typename F, typename G>
+  __device__ __forceinline__ void sums(int lane, F put, G putb) {
+#pragma unroll
+    for (int i = 0; i < 16; ++i)
+      put(8 * (i >> 2) + 4 * (lane >> 5) + (i & 3), lane & 31, c[i]);
+    float v = b;
+    v += __shfl_xor(v, 32);
+    if (lane < 32) putb(lane, v);
+  }
+};
+
 // ---------------------------------------------------------------------------
 // k_fused: forward, residual program, adjoint and weight gradients in one
 // pass (the fused training step of narrow float networks)
@@ -527,9 +742,11 @@ __host__ __device__ constexpr int fused_resid_words() {
 // All LDS words of the fused kernel: buffers, network values (two rounds),
 // the loss values of one block (loss, normalized), the residual policy's
 // area and the staged network image.
-__host__ __device__ inline int fused_lds_words(int HP, int NH, int d_in, int n_out, int P) {
-  return fused_buf_words(HP, P) + 2 * 16 * FUSE_MAX_SLOTS + 128 + fused_resid_words() +
-         stage_words(HP, NH, d_in, n_out, true);
+__host__ __device__ inline int fused_lds_words(int HP, int NH, int d_in, int n_out, int P,
+                                               bool interp) {
+  return fused_buf_words(HP, P) + 2 * 16 * FUSE_MAX_SLOTS + 128 +
+         (interp ? fused_resid_words() : 0) +
+         stage_words(HP, NH, d_in, n_out, true, 4);
 }
 
 // Residual policy of the library's fused kernel: the group's program tables
@@ -537,6 +754,7 @@ __host__ __device__ inline int fused_lds_words(int HP, int NH, int d_in, int n_o
 // per workgroup and interpreted by entry_program; seeds gathered in an LDS
 // row per entry, then returned in registers.
 struct InterpResid {
+  static constexpr int kWords = fused_resid_words();
   const int32_t *pints;
   const float *preals;
   const float *data;
@@ -594,24 +812,18 @@ __device__ __forceinline__ void fused_body(const NNArgs<float> &a, float *smem) 
   T *u_all = smem + fused_buf_words(HP, P);               // [2][16][FUSE_MAX_SLOTS]
   T *lbuf = u_all + 2 * 16 * FUSE_MAX_SLOTS;              // [2][64]
   T *rarea = lbuf + 128;
-  T *stage = rarea + fused_resid_words();
+  T *stage = rarea + R::kWords;
   R resid(a, item.x, n_eq, rarea, w);
   const Net<T, NB> net = stage_net<T, NB>(a, G[0], stage, true);  // ends with a barrier
   const T dl_scale = *a.dloss;
 
   // gradient accumulators, as in the wavefront-private backward (one output
   // and at most two inputs: the first and last layers on the VALU)
-  v4 dwacc[NJ][NB * NB];
-  T bhacc[NJ][NB];
+  WGrad<T, NB> wg[NJ];
   T wlacc[NB][4], w1acc[NB][4][2], b1acc[NB][4];
   T blacc = T(0);
 #pragma unroll
-  for (int j = 0; j < NJ; ++j) {
-#pragma unroll
-    for (int b = 0; b < NB * NB; ++b) dwacc[j][b] = v4{0, 0, 0, 0};
-#pragma unroll
-    for (int b = 0; b < NB; ++b) bhacc[j][b] = T(0);
-  }
+  for (int j = 0; j < NJ; ++j) wg[j].zero();
 #pragma unroll
   for (int b = 0; b < NB; ++b)
 #pragma unroll
@@ -726,31 +938,13 @@ __device__ __forceinline__ void fused_body(const NNArgs<float> &a, float *smem) 
             abuf[f * WRS + row] = act[k][j - 1][mb][i];
           }
         wave_sync();
-        {
-          v4 av[NB], dv[NB];
-#pragma unroll
-          for (int xb = 0; xb < NB; ++xb) {
-            dv[xb] = *reinterpret_cast<const v4 *>(dbuf + (16 * xb + row) * WRS + 4 * q);
-            av[xb] = *reinterpret_cast<const v4 *>(abuf + (16 * xb + row) * WRS + 4 * q);
-          }
-#pragma unroll
-          for (int ob = 0; ob < NB; ++ob) {
-            bhacc[jj][ob] += (dv[ob][0] + dv[ob][1]) + (dv[ob][2] + dv[ob][3]);
-#pragma unroll
-            for (int ib = 0; ib < NB; ++ib) {
-              v4 c = dwacc[jj][ob * NB + ib];
-#pragma unroll
-              for (int kb = 0; kb < 4; ++kb) c = mma16(dv[ob][kb], av[ib][kb], c);
-              dwacc[jj][ob * NB + ib] = c;
-            }
-          }
-        }
+        wg[jj].add(dbuf, abuf, lane);
         wave_sync();
         // delta_{j-1} = (W_jj^T delta_j) * (1 - act_{j-1}^2)
         v4 c[NB];
 #pragma unroll
         for (int ib = 0; ib < NB; ++ib) c[ib] = v4{0, 0, 0, 0};
-        mma_layer<T, NB>(net.Wb + jj * HP * HP, lane, dl, c);
+        mma_layer<T, NB>(net.Wb + jj * net.LI, lane, dl, c);
 #pragma unroll
         for (int ib = 0; ib < NB; ++ib)
 #pragma unroll
@@ -781,19 +975,15 @@ __device__ __forceinline__ void fused_body(const NNArgs<float> &a, float *smem) 
       const bool first = ww == 0;
       auto put = [&](int pos, T v) { cp[pos] = first ? v : cp[pos] + v; };
 #pragma unroll
-      for (int ob = 0; ob < NB; ++ob)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int out = 16 * ob + crow<T>(q, i);
-          if (out >= H) continue;
-#pragma unroll
-          for (int jj = 0; jj < NH; ++jj)
-#pragma unroll
-            for (int ib = 0; ib < NB; ++ib) {
-              const int in = 16 * ib + row;
-              if (in < H) put(L.oWh(jj) + out * H + in, dwacc[jj][ob * NB + ib][i]);
-            }
-        }
+      for (int jj = 0; jj < NH; ++jj)
+        wg[jj].sums(
+            lane,
+            [&](int out, int in, T v) {
+              if (out < H && in < H) put(L.oWh(jj) + out * H + in, v);
+            },
+            [&](int f, T v) {
+              if (f < H) put(L.obh(jj) + f, v);
+            });
 #pragma unroll
       for (int ob = 0; ob < NB; ++ob)
 #pragma unroll
@@ -808,16 +998,6 @@ __device__ __forceinline__ void fused_body(const NNArgs<float> &a, float *smem) 
           if (row == 0 && out < H) put(L.ob1() + out, vb);
           const T vl = rowsum16(wlacc[ob][i]);
           if (row == 0 && out < H) put(L.oWL() + out, vl);
-        }
-#pragma unroll
-      for (int jj = 0; jj < NH; ++jj)
-#pragma unroll
-        for (int xb = 0; xb < NB; ++xb) {
-          T v = bhacc[jj][xb];
-          v += __shfl_xor(v, 16);
-          v += __shfl_xor(v, 32);
-          const int f = 16 * xb + row;
-          if (q == 0 && f < H) put(L.obh(jj) + f, v);
         }
       const T bl = rowsum16(blacc);
       if (row == 0 && q == 0) put(L.obL(), bl);
@@ -845,37 +1025,24 @@ __device__ __forceinline__ void fused_body(const NNArgs<float> &a, float *smem) 
 constexpr int CTRS = 68;  // row stride of the feature-major tile buffers
 
 // acc[ob] += W (rows of block ob) x b where b is this lane's row trow of a
-// feature-major LDS buffer (stride CTRS); one input block at a time, so only
-// that block's four operands and the NB accumulators are live.
-template <typename T, int NB>
-__device__ __forceinline__ void mma_layer_fm(const T *img, int lane, const T *src, int trow,
-                                             typename V4<T>::type (&acc)[NB]) {
-  typedef typename V4<T>::type v4;
+// feature-major LDS buffer (stride CTRS), split once for all output blocks.
+template <int NB>
+__device__ __forceinline__ void mma_layer_fm(const float *img, int lane, const float *src,
+                                             int trow, f4_t (&acc)[NB]) {
   const int q = lane >> 4;
-  const v4 *wp = reinterpret_cast<const v4 *>(img) + lane;
-  // two input blocks per round, the second block's weights loaded with the
-  // first's: their latency is paid once per pair
-  auto block = [&](int mb, const v4 (&w)[NB]) {
-    T b[4];
+  float b[NB][4];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) b[i] = src[(16 * mb + crow<T>(q, i)) * CTRS + trow];
+  for (int mb = 0; mb < NB; ++mb)
 #pragma unroll
-    for (int ob = 0; ob < NB; ++ob)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) acc[ob] = mma16(w[ob][i], b[i], acc[ob]);
-  };
-#pragma unroll 1
-  for (int mb = 0; mb < NB; mb += 2) {
-    v4 wa[NB], wb[NB];
-#pragma unroll
-    for (int ob = 0; ob < NB; ++ob) wa[ob] = wp[(ob * NB + mb) * 64];
-    if (mb + 1 < NB) {
-#pragma unroll
-      for (int ob = 0; ob < NB; ++ob) wb[ob] = wp[(ob * NB + mb + 1) * 64];
-    }
-    block(mb, wa);
-    if (mb + 1 < NB) block(mb + 1, wb);
-  }
+    for (int i = 0; i < 4; ++i) b[mb][i] = src[(16 * mb + 4 * q + i) * CTRS + trow];
+  mma_layer<float, NB>(img, lane, b, acc);
+}
+
+// Eight consecutive rows (r and on) of feature f of a feature-major buffer.
+__device__ __forceinline__ void rows8(const float *buf, int f, int r, f4_t &lo, f4_t &hi) {
+  const f4_t *p = reinterpret_cast<const f4_t *>(buf + f * CTRS + r);
+  lo = p[0];
+  hi = p[1];
 }
 
 __host__ __device__ inline size_t block_lds_words(int HP, int NH) {
@@ -1029,7 +1196,7 @@ __device__ __forceinline__ void block_body(const NNArgs<T> &a, T *smem) {
 #pragma unroll
       for (int ob = 0; ob < NB; ++ob) acc[ob] = ld4(net.bh + (j - 1) * HP + 16 * ob + 4 * q);
       wave_sync();  // the wavefront's own rows of layer j-1 are in LDS
-      mma_layer_fm<T, NB>(net.Wf + (j - 1) * HP * HP, lane, layer_buf(j - 1), trow, acc);
+      mma_layer_fm<NB>(net.Wf + (j - 1) * net.LI, lane, layer_buf(j - 1), trow, acc);
 #pragma unroll
       for (int ob = 0; ob < NB; ++ob)
 #pragma unroll
@@ -1098,13 +1265,11 @@ __device__ __forceinline__ void block_body(const NNArgs<T> &a, T *smem) {
         const int ob = w + 4 * u;
         if (ob < NB) {
 #pragma unroll
-          for (int kk = 0; kk < TR / 16; ++kk) {
-            const v4 av = *reinterpret_cast<const v4 *>(aN + (16 * ob + row) * CTRS + 16 * kk + 4 * q);
-            const v4 sv = (o >= 0 && o < n_out)
-                              ? *reinterpret_cast<const v4 *>(sbuf + o * CTRS + 16 * kk + 4 * q)
-                              : v4{0, 0, 0, 0};
-#pragma unroll
-            for (int kb = 0; kb < 4; ++kb) sacc[u] = mma16(av[kb], sv[kb], sacc[u]);
+          for (int kk = 0; kk < TR / 32; ++kk) {
+            f4_t alo, ahi, slo = {0, 0, 0, 0}, shi = {0, 0, 0, 0};
+            rows8(aN, 16 * ob + row, 32 * kk + 8 * q, alo, ahi);
+            if (o >= 0 && o < n_out) rows8(sbuf, o, 32 * kk + 8 * q, slo, shi);
+            sacc[u] = mma3(bf3_split(alo, ahi), bf3_split(slo, shi), sacc[u]);
           }
         }
       }
@@ -1118,27 +1283,33 @@ __device__ __forceinline__ void block_body(const NNArgs<T> &a, T *smem) {
       T *dbuf = layer_buf(j);  // delta_j over act_j (read for the last time above)
       store_rows(dbuf, dl);
       __syncthreads();
-      // owned blocks of dW_jj over the 64 rows; hidden bias from the delta
-      // operand (each lane holds 4 rows of one feature per row group)
-#pragma unroll
-      for (int u = 0; u < OBW; ++u) {
-        const int ob = w + 4 * u;
-        if (ob < NB) {
-          // row groups outermost (not unrolled): only one group's operands
-          // are live; each block still sums its rows in the same order
+      // owned blocks of dW_jj over the 64 rows, 32 at a time; hidden bias from
+      // the delta operand (each lane holds 8 rows of one feature).  An input
+      // block's activations are split once for all owned output blocks.
 #pragma unroll 1
-          for (int kk = 0; kk < TR / 16; ++kk) {
-            const v4 dv = *reinterpret_cast<const v4 *>(dbuf + (16 * ob + row) * CTRS + 16 * kk + 4 * q);
-            bhacc[jj][u] += (dv[0] + dv[1]) + (dv[2] + dv[3]);
+      for (int kk = 0; kk < TR / 32; ++kk) {
+        const int r8 = 32 * kk + 8 * q;
+        Bf3 ds[OBW];
 #pragma unroll
-            for (int ib = 0; ib < NB; ++ib) {
-              const v4 av = *reinterpret_cast<const v4 *>(ain + (16 * ib + row) * CTRS + 16 * kk + 4 * q);
-              v4 c = dwacc[jj][u][ib];
-#pragma unroll
-              for (int kb = 0; kb < 4; ++kb) c = mma16(dv[kb], av[kb], c);
-              dwacc[jj][u][ib] = c;
-            }
+        for (int u = 0; u < OBW; ++u) {
+          const int ob = w + 4 * u;
+          if (ob < NB) {
+            f4_t lo, hi;
+            rows8(dbuf, 16 * ob + row, r8, lo, hi);
+            bhacc[jj][u] += ((lo[0] + lo[1]) + (lo[2] + lo[3])) +
+                            ((hi[0] + hi[1]) + (hi[2] + hi[3]));
+            ds[u] = bf3_split(lo, hi);
           }
+        }
+#pragma unroll
+        for (int ib = 0; ib < NB; ++ib) {
+          __builtin_amdgcn_sched_barrier(0);
+          f4_t lo, hi;
+          rows8(ain, 16 * ib + row, r8, lo, hi);
+          const Bf3 as = bf3_split(lo, hi);
+#pragma unroll
+          for (int u = 0; u < OBW; ++u)
+            if (w + 4 * u < NB) dwacc[jj][u][ib] = mma3(ds[u], as, dwacc[jj][u][ib]);
         }
       }
       // delta_{j-1} = (W_jj^T delta_j) * (1 - act_{j-1}^2) for this
@@ -1146,7 +1317,7 @@ __device__ __forceinline__ void block_body(const NNArgs<T> &a, T *smem) {
       v4 c[NB];
 #pragma unroll
       for (int ib = 0; ib < NB; ++ib) c[ib] = v4{0, 0, 0, 0};
-      mma_layer_fm<T, NB>(net.Wb + jj * HP * HP, lane, dbuf, trow, c);
+      mma_layer_fm<NB>(net.Wb + jj * net.LI, lane, dbuf, trow, c);
 #pragma unroll
       for (int ib = 0; ib < NB; ++ib)
 #pragma unroll
@@ -1166,13 +1337,12 @@ __device__ __forceinline__ void block_body(const NNArgs<T> &a, T *smem) {
       const int ob = w + 4 * u;
       if (ob < NB) {
 #pragma unroll
-        for (int kk = 0; kk < TR / 16; ++kk) {
-          const v4 dv = *reinterpret_cast<const v4 *>(dbuf + (16 * ob + row) * CTRS + 16 * kk + 4 * q);
-          const v4 xv = row < d_in
-                            ? *reinterpret_cast<const v4 *>(xbuf + row * CTRS + 16 * kk + 4 * q)
-                            : (row == col_b1 ? v4{1, 1, 1, 1} : v4{0, 0, 0, 0});
-#pragma unroll
-          for (int kb = 0; kb < 4; ++kb) sacc[u] = mma16(dv[kb], xv[kb], sacc[u]);
+        for (int kk = 0; kk < TR / 32; ++kk) {
+          f4_t dlo, dhi, xlo = {0, 0, 0, 0}, xhi = {0, 0, 0, 0};
+          rows8(dbuf, 16 * ob + row, 32 * kk + 8 * q, dlo, dhi);
+          if (row < d_in) rows8(xbuf, row, 32 * kk + 8 * q, xlo, xhi);
+          if (row == col_b1) xlo = xhi = f4_t{1, 1, 1, 1};
+          sacc[u] = mma3(bf3_split(dlo, dhi), bf3_split(xlo, xhi), sacc[u]);
         }
       }
     }

@@ -183,6 +183,7 @@ std::string nn_fused_jit_source(const std::vector<std::vector<int32_t>> &keys,
   o << "namespace tdx {\n"
        "// generated residual programs, one per structure (kind)\n"
        "struct GenResid {\n"
+       "  static constexpr int kWords = 0;\n"
        "  const int32_t *I;\n"
        "  const float *R;\n"
        "  const float *data;\n"
