@@ -716,14 +716,19 @@ __global__ __launch_bounds__(AD_THREADS) void k_ad_wreduce(const T *part, int n_
 // per-residual Jacobian (natural-gradient Gram assembly)
 // ---------------------------------------------------------------------------
 // The reference forms J with one torch.autograd.grad per residual
-// (tedeous/optimizers/ngd.py:57-78).  One thread owns one (group, entry):
-// per equation it forms the seeds dr/dU(set, jet, var) of the residual
-// program with dr = 1 (the k_ad_resid seeds), and for every set with a
-// non-zero seed pushes that point's jets through the network and the jet
-// maps' adjoints back, adding seed * dU/dparams into its own column r of
-// jt[P][n_resid].  Per-thread state lives in LDS, thread-fastest:
+// (tedeous/optimizers/ngd.py:57-78).  A workgroup takes E adjacent entries
+// of one group, 256 / E threads each: per equation the seeds dr/dU(set, jet,
+// var) of the residual program with dr = 1 (the k_ad_resid seeds), and for
+// every set with a non-zero seed the point's jets through the network and
+// the jet maps' adjoints back, seed * dU/dparams into the entry's column r
+// of jt[P][n_resid].  An entry's state is in LDS, entry-fastest:
 // pre-activation and activation jets of every hidden layer, two adjoint
-// buffers, the output jets of every set and the seeds.
+// buffers, the output jets of every set and the seeds.  What bounds it: the
+// chain of layers of one entry, a few microseconds each, so an entry's units,
+// jets and parameters are spread over many threads (one thread an entry took
+// 1575 us on 501 points, 1-32-32-2, two equations; now 35 us) and E stays at
+// 4, 16-byte pieces of a row of jt, until there are entries for 512
+// workgroups of more.  Table reads are scalar (the group is the workgroup's).
 template <typename T>
 struct JacArgs {
   int d_in, n_out, H, L, J, n_groups, groups_i, max_sets;
@@ -733,213 +738,273 @@ struct JacArgs {
   Tables tb;
   const int64_t *off_w, *off_b;   // parameter offsets per layer (device)
   T *jt;
-  int64_t n_resid;
+  int64_t n_resid, n_params;
+  int accum;  // add into cleared columns instead of writing them
 };
 
 template <typename T>
-__global__ void k_ad_jac(JacArgs<T> a) {
+__device__ __forceinline__ T ctabr(const T *p, int i) {
+  return ((const __attribute__((address_space(4))) T *)p)[i];
+}
+
+template <typename T>
+__global__ __launch_bounds__(256) void k_ad_jac(JacArgs<T> a, int E) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
   T *smem = reinterpret_cast<T *>(smem_raw);
-  const int B = blockDim.x, t = threadIdx.x;
   const int J = a.J, H = a.H, L = a.L, NL = L - 1, no = a.n_out, din = a.d_in;
-  const int JH = J * H;
-  // LDS per thread (element k at [k * B + t]): Z[NL][J][H] | A[NL][J][H] |
+  const int JH = J * H, t = threadIdx.x & (E - 1), u = threadIdx.x / E, NU = 256 / E;
+  // LDS per entry (element k at [k * E + t]): Z[NL][J][H] | A[NL][J][H] |
   // D0[J][H] | D1[J][H] | U[max_sets][J][no] | S[max_sets][J][no] | X[J][din]
   T *Zs = smem;
-  T *As = Zs + (size_t)NL * JH * B;
-  T *D0 = As + (size_t)NL * JH * B;
-  T *D1 = D0 + (size_t)JH * B;
-  T *Us = D1 + (size_t)JH * B;
-  T *Ss = Us + (size_t)a.max_sets * J * no * B;
-  T *Xs = Ss + (size_t)a.max_sets * J * no * B;
-#define LV(base, k) base[(size_t)(k) * B + t]
-  const int64_t ge = (int64_t)blockIdx.x * B + t;
-  const int64_t total = a.gstart[a.n_groups];
-  if (ge >= total) return;
+  T *As = Zs + (size_t)NL * JH * E;
+  T *D0 = As + (size_t)NL * JH * E;
+  T *D1 = D0 + (size_t)JH * E;
+  T *Us = D1 + (size_t)JH * E;
+  T *Ss = Us + (size_t)a.max_sets * J * no * E;
+  T *Xs = Ss + (size_t)a.max_sets * J * no * E;
+#define LV(base, k) base[(size_t)(k) * E + t]
+  // this workgroup's group and first entry
   int g = 0;
-  while (g + 1 < a.n_groups && a.gstart[g + 1] <= ge) ++g;
-  const int e = (int)(ge - a.gstart[g]);
-  const int32_t *G = a.ints + a.groups_i + TDX_AD_GROUP_INTS * g;
-  const int n_sets = G[1], set_i = G[2], n_eq = G[3], eq_i = G[4];
+  int64_t blk = blockIdx.x, count = 0;
+  for (; g < a.n_groups; ++g) {
+    count = a.gstart[g + 1] - a.gstart[g];
+    const int64_t nb = (count + E - 1) / E;
+    if (blk < nb) break;
+    blk -= nb;
+  }
+  g = __builtin_amdgcn_readfirstlane(g);
+  if (g >= a.n_groups) return;
+  const bool valid = blk * E + t < count;
+  const int e = (int)(valid ? blk * E + t : count - 1);
+  const int G = a.groups_i + TDX_AD_GROUP_INTS * g;
+  const int n_sets = ctab(a.ints, G + 1), set_i = ctab(a.ints, G + 2);
+  const int n_eq = ctab(a.ints, G + 3), eq_i = ctab(a.ints, G + 4);
   const Tables &tb = a.tb;
   const T *W = a.params;
 
   // jets of point pt through the network: Z, A of every hidden layer, and
-  // (with u_out) the output jets
+  // (with u_out) the output jets.  Ends with a workgroup barrier.
   auto forward = [&](int64_t pt, T *u_out) {
-    for (int al = 0; al < J; ++al) {
+    for (int k = u; k < J * din; k += NU) {
+      const int al = k / din, j = k - al * din;
       const int ord = tb.ints[tb.jet_i + 2 * al], ax = tb.ints[tb.jet_i + 2 * al + 1];
-      for (int j = 0; j < din; ++j)
-        LV(Xs, al * din + j) = al == 0 ? a.points[pt * din + j] : (ord == 1 && ax == j ? T(1) : T(0));
+      LV(Xs, k) = al == 0 ? a.points[pt * din + j] : (ord == 1 && ax == j ? T(1) : T(0));
     }
+    __syncthreads();
     for (int l = 0; l < NL; ++l) {
       const int dl = l == 0 ? din : H;
       const T *Wl = W + a.off_w[l], *bl = W + a.off_b[l];
-      T *Z = Zs + (size_t)l * JH * B, *A = As + (size_t)l * JH * B;
-      const T *In = l == 0 ? Xs : As + (size_t)(l - 1) * JH * B;
-      for (int i = 0; i < H; ++i) {
-        for (int al = 0; al < J; ++al) {
-          T z = al == 0 ? bl[i] : T(0);
-          for (int j = 0; j < dl; ++j) z = fma(Wl[i * dl + j], LV(In, al * dl + j), z);
-          LV(Z, al * H + i) = z;
-        }
+      T *Z = Zs + (size_t)l * JH * E, *A = As + (size_t)l * JH * E;
+      const T *In = l == 0 ? Xs : As + (size_t)(l - 1) * JH * E;
+      for (int k = u; k < JH; k += NU) {
+        const int al = k / H, i = k - al * H;
+        T z = al == 0 ? bl[i] : T(0);
+#pragma unroll 8
+        for (int j = 0; j < dl; ++j) z = fma(Wl[i * dl + j], LV(In, al * dl + j), z);
+        LV(Z, k) = z;
+      }
+      __syncthreads();
+      for (int i = u; i < H; i += NU) {
         const TanhDerivs<T> sd = tanh_derivs(LV(Z, i));
         LV(A, i) = sd.s0;
         for (int al = 1; al < J; ++al) {
-          const int k0 = tb.ints[tb.pptr_i + al], k1 = tb.ints[tb.pptr_i + al + 1];
+          const int k0 = ctab(tb.ints, tb.pptr_i + al), k1 = ctab(tb.ints, tb.pptr_i + al + 1);
           T h = T(0);
           for (int k = k0; k < k1; ++k) {
-            const int32_t *pr = tb.ints + tb.part_i + TDX_AD_PART_INTS * k;
-            const int m = pr[0];
+            const int pr = tb.part_i + TDX_AD_PART_INTS * k;
+            const int m = ctab(tb.ints, pr);
             T prod = deriv_n(sd.s1, sd.s2, sd.s3, sd.s4, sd.s5, m);
-            for (int q = 0; q < m; ++q) prod = prod * LV(Z, pr[1 + q] * H + i);
+            for (int q = 0; q < m; ++q) prod = prod * LV(Z, ctab(tb.ints, pr + 1 + q) * H + i);
             h = (k == k0) ? prod : h + prod;
           }
           LV(A, al * H + i) = h;
         }
       }
+      __syncthreads();
     }
     if (u_out) {
       const T *Wl = W + a.off_w[L - 1], *bl = W + a.off_b[L - 1];
-      const T *In = As + (size_t)(NL - 1) * JH * B;
-      for (int o = 0; o < no; ++o)
-        for (int al = 0; al < J; ++al) {
-          T u = al == 0 ? bl[o] : T(0);
-          for (int j = 0; j < H; ++j) u = fma(Wl[o * H + j], LV(In, al * H + j), u);
-          LV(u_out, al * no + o) = u;
-        }
+      const T *In = As + (size_t)(NL - 1) * JH * E;
+      for (int k = u; k < J * no; k += NU) {
+        const int al = k / no, o = k - al * no;
+        T v = al == 0 ? bl[o] : T(0);
+#pragma unroll 8
+        for (int j = 0; j < H; ++j) v = fma(Wl[o * H + j], LV(In, al * H + j), v);
+        LV(u_out, k) = v;
+      }
+      __syncthreads();
     }
   };
 
-  for (int s = 0; s < n_sets; ++s) forward(a.ints[set_i + s] + e, Us + (size_t)s * J * no * B);
+  for (int s = 0; s < n_sets; ++s)
+    forward((int64_t)ctab(a.ints, set_i + s) + e, Us + (size_t)s * J * no * E);
 
   for (int q = 0; q < n_eq; ++q) {
-    const int32_t *E = a.ints + eq_i + TDX_AD_EQ_INTS * q;
-    const int n_terms = E[0], term_i = E[1];
-    if (E[5] < 0) continue;
-    T *col = a.jt + E[5] + e;
-    for (int k = 0; k < n_sets * J * no; ++k) LV(Ss, k) = T(0);
-    auto factor_value = [&](const int32_t *F) {
+    const int Eq = eq_i + TDX_AD_EQ_INTS * q;
+    const int n_terms = ctab(a.ints, Eq), term_i = ctab(a.ints, Eq + 1);
+    const int ro = ctab(a.ints, Eq + 5);
+    if (ro < 0) continue;
+    T *col = a.jt + ro + e;
+    for (int k = u; k < n_sets * J * no; k += NU) LV(Ss, k) = T(0);
+    __syncthreads();
+    auto factor_value = [&](int F) {
+      const int n_st = ctab(a.ints, F), st_i = ctab(a.ints, F + 1), var = ctab(a.ints, F + 2);
       T fv = T(0);
-      for (int k = 0; k < F[0]; ++k) {
-        const int32_t *S = a.ints + F[1] + TDX_AD_STENCIL_INTS * k;
-        const T v = LV(Us, (S[0] * J + S[1]) * no + F[2]);
-        fv = (k == 0) ? a.reals[S[2]] * v : fv + a.reals[S[2]] * v;
+      for (int k = 0; k < n_st; ++k) {
+        const int S = st_i + TDX_AD_STENCIL_INTS * k;
+        const T v = LV(Us, (ctab(a.ints, S) * J + ctab(a.ints, S + 1)) * no + var);
+        const T w = ctabr(a.reals, ctab(a.ints, S + 2));
+        fv = (k == 0) ? w * v : fv + w * v;
       }
       return fv;
     };
-    // dr/dU through every factor of every term
-    for (int tt = 0; tt < n_terms; ++tt) {
-      const int32_t *Tr = a.ints + term_i + TDX_AD_TERM_INTS * tt;
-      const int nf = Tr[0];
-      const T c = Tr[2] == 0 ? a.reals[Tr[3]] : a.data[Tr[3] + e];
-      const bool chain = term_has_chain(a.ints, Tr[1], nf);
-      T fv[AD_MAXF], pw[AD_MAXF], dfv[AD_MAXF];
-      for (int f = 0; f < AD_MAXF; ++f) {
-        fv[f] = T(0);
-        pw[f] = T(1);
-        if (f < nf) {
-          const int32_t *F = a.ints + Tr[1] + TDX_AD_FACTOR_INTS * f;
-          fv[f] = factor_value(F);
-          if (!chain) pw[f] = fpow(F[3], F[4], a.reals, fv[f]);
+    // dr/dU through every factor of every term (one thread an entry)
+    if (u == 0) {
+      for (int tt = 0; tt < n_terms; ++tt) {
+        const int Tr = term_i + TDX_AD_TERM_INTS * tt;
+        const int nf = ctab(a.ints, Tr), fi = ctab(a.ints, Tr + 1);
+        const int cr = ctab(a.ints, Tr + 3);
+        const T c = ctab(a.ints, Tr + 2) == 0 ? ctabr(a.reals, cr) : a.data[cr + e];
+        const bool chain = term_has_chain(a.ints, fi, nf);
+        T fv[AD_MAXF], pw[AD_MAXF], dfv[AD_MAXF];
+#pragma unroll
+        for (int f = 0; f < AD_MAXF; ++f) {
+          fv[f] = T(0);
+          pw[f] = T(1);
+          if (f < nf) {
+            const int F = fi + TDX_AD_FACTOR_INTS * f;
+            fv[f] = factor_value(F);
+            if (!chain) pw[f] = fpow(ctab(a.ints, F + 3), ctab(a.ints, F + 4), a.reals, fv[f]);
+          }
         }
-      }
-      if (chain) (void)chain_term(a.ints, Tr[1], nf, a.reals, fv, dfv);
-      for (int f = 0; f < nf; ++f) {
-        const int32_t *F = a.ints + Tr[1] + TDX_AD_FACTOR_INTS * f;
-        T dv = chain ? c * dfv[f] : c * fdpow(F[3], F[4], a.reals, fv[f]);
-        for (int f2 = 0; f2 < nf && !chain; ++f2)
-          if (f2 != f) dv = dv * pw[f2];
-        for (int k = 0; k < F[0]; ++k) {
-          const int32_t *S = a.ints + F[1] + TDX_AD_STENCIL_INTS * k;
-          LV(Ss, (S[0] * J + S[1]) * no + F[2]) += dv * a.reals[S[2]];
+        if (chain) (void)chain_term(a.ints, fi, nf, a.reals, fv, dfv);
+#pragma unroll
+        for (int f = 0; f < AD_MAXF; ++f) {
+          if (f < nf) {
+            const int F = fi + TDX_AD_FACTOR_INTS * f;
+            T dv;
+            if (chain) {
+              dv = c * dfv[f];
+            } else {
+              dv = c * fdpow(ctab(a.ints, F + 3), ctab(a.ints, F + 4), a.reals, fv[f]);
+#pragma unroll
+              for (int f2 = 0; f2 < AD_MAXF; ++f2)
+                if (f2 != f && f2 < nf) dv = dv * pw[f2];
+            }
+            const int n_st = ctab(a.ints, F), st_i = ctab(a.ints, F + 1);
+            const int var = ctab(a.ints, F + 2);
+            for (int k = 0; k < n_st; ++k) {
+              const int S = st_i + TDX_AD_STENCIL_INTS * k;
+              LV(Ss, (ctab(a.ints, S) * J + ctab(a.ints, S + 1)) * no + var) +=
+                  dv * ctabr(a.reals, ctab(a.ints, S + 2));
+            }
+          }
         }
       }
     }
-    auto add = [&](int64_t pidx, T v) { col[pidx * a.n_resid] += v; };
+    __syncthreads();
+    bool act = false, wrote = a.accum != 0;
+    auto put = [&](int64_t pidx, T v) {
+      if (!valid || !act) return;
+      T &c = col[pidx * a.n_resid];
+      c = wrote ? c + v : v;
+    };
     for (int s = 0; s < n_sets; ++s) {
-      const T *Sd = Ss + (size_t)s * J * no * B;
-      bool any = false;
-      for (int k = 0; k < J * no; ++k) any |= LV(Sd, k) != T(0);
+      const T *Sd = Ss + (size_t)s * J * no * E;
+      act = false;
+      bool any = false;  // of the workgroup's entries
+      for (int k = 0; k < J * no; ++k) act |= LV(Sd, k) != T(0);
+      for (int k = 0; k < J * no * E; ++k) any |= Sd[k] != T(0);
       if (!any) continue;
-      forward(a.ints[set_i + s] + e, nullptr);
+      // with one set its forward state is still in LDS
+      if (n_sets > 1) forward((int64_t)ctab(a.ints, set_i + s) + e, nullptr);
       // output layer: dW[o][j] += sum_al dU[al][o] A[al][j]; dA = W^T dU
       {
         const T *Wl = W + a.off_w[L - 1];
-        const T *Al = As + (size_t)(NL - 1) * JH * B;
-        for (int o = 0; o < no; ++o) {
-          for (int j = 0; j < H; ++j) {
-            T g = T(0);
-            for (int al = 0; al < J; ++al) g = fma(LV(Sd, al * no + o), LV(Al, al * H + j), g);
-            add(a.off_w[L - 1] + o * H + j, g);
-          }
-          add(a.off_b[L - 1] + o, LV(Sd, o));
+        const T *Al = As + (size_t)(NL - 1) * JH * E;
+        const int64_t ow = a.off_w[L - 1], ob = a.off_b[L - 1];
+        for (int k = u; k < no * H; k += NU) {
+          const int o = k / H, j = k - o * H;
+          T gv = T(0);
+          for (int al = 0; al < J; ++al) gv = fma(LV(Sd, al * no + o), LV(Al, al * H + j), gv);
+          put(ow + k, gv);
         }
-        for (int al = 0; al < J; ++al)
-          for (int j = 0; j < H; ++j) {
-            T g = T(0);
-            for (int o = 0; o < no; ++o) g = fma(Wl[o * H + j], LV(Sd, al * no + o), g);
-            LV(D0, al * H + j) = g;
-          }
+        for (int o = u; o < no; o += NU) put(ob + o, LV(Sd, o));
+        for (int k = u; k < JH; k += NU) {
+          const int al = k / H, j = k - al * H;
+          T gv = T(0);
+          for (int o = 0; o < no; ++o) gv = fma(Wl[o * H + j], LV(Sd, al * no + o), gv);
+          LV(D0, k) = gv;
+        }
       }
+      __syncthreads();
       T *dA = D0, *dZ = D1;
       for (int l = NL - 1; l >= 0; --l) {
-        const T *Z = Zs + (size_t)l * JH * B;
+        const T *Z = Zs + (size_t)l * JH * E;
         // adjoint of the tanh jet map (unit i): dZ from dA
-        for (int i = 0; i < H; ++i) {
+        for (int i = u; i < H; i += NU) {
           const TanhDerivs<T> sd = tanh_derivs(LV(Z, i));
           T dz0 = LV(dA, i) * sd.s1;
           for (int al = 1; al < J; ++al) {
             const T dd = LV(dA, al * H + i);
-            const int k0 = tb.ints[tb.pptr_i + al], k1 = tb.ints[tb.pptr_i + al + 1];
+            const int k0 = ctab(tb.ints, tb.pptr_i + al), k1 = ctab(tb.ints, tb.pptr_i + al + 1);
             for (int k = k0; k < k1; ++k) {
-              const int32_t *pr = tb.ints + tb.part_i + TDX_AD_PART_INTS * k;
-              const int m = pr[0];
+              const int pr = tb.part_i + TDX_AD_PART_INTS * k;
+              const int m = ctab(tb.ints, pr);
               T all = deriv_n(sd.s1, sd.s2, sd.s3, sd.s4, sd.s5, m + 1);
-              for (int q2 = 0; q2 < m; ++q2) all = all * LV(Z, pr[1 + q2] * H + i);
+              for (int q2 = 0; q2 < m; ++q2)
+                all = all * LV(Z, ctab(tb.ints, pr + 1 + q2) * H + i);
               dz0 = dz0 + dd * all;
             }
           }
           LV(dZ, i) = dz0;
           for (int b = 1; b < J; ++b) {
             T acc = T(0);
-            const int t0 = tb.occ[tb.tptr_i + b], t1 = tb.occ[tb.tptr_i + b + 1];
+            const int t0 = ctab(tb.occ, tb.tptr_i + b), t1 = ctab(tb.occ, tb.tptr_i + b + 1);
             for (int tt = t0; tt < t1; ++tt) {
-              const int32_t *oc = tb.occ + tb.tent_i + 3 * tt;
-              const int al = oc[0], qq = oc[2];
-              const int32_t *pr = tb.ints + tb.part_i + TDX_AD_PART_INTS * oc[1];
-              const int m = pr[0];
+              const int oc = tb.tent_i + 3 * tt;
+              const int al = ctab(tb.occ, oc), qq = ctab(tb.occ, oc + 2);
+              const int pr = tb.part_i + TDX_AD_PART_INTS * ctab(tb.occ, oc + 1);
+              const int m = ctab(tb.ints, pr);
               T v = LV(dA, al * H + i) * deriv_n(sd.s1, sd.s2, sd.s3, sd.s4, sd.s5, m);
               for (int q2 = 0; q2 < m; ++q2)
-                if (q2 != qq) v = v * LV(Z, pr[1 + q2] * H + i);
+                if (q2 != qq) v = v * LV(Z, ctab(tb.ints, pr + 1 + q2) * H + i);
               acc = acc + v;
             }
             LV(dZ, b * H + i) = acc;
           }
         }
+        __syncthreads();
         // linear layer l: dW[i][j] += sum_al dZ[al][i] In[al][j]; db += dZ[0]
         const int dl = l == 0 ? din : H;
-        const T *In = l == 0 ? Xs : As + (size_t)(l - 1) * JH * B;
+        const T *In = l == 0 ? Xs : As + (size_t)(l - 1) * JH * E;
         const T *Wl = W + a.off_w[l];
-        for (int i = 0; i < H; ++i) {
-          for (int j = 0; j < dl; ++j) {
-            T g = T(0);
-            for (int al = 0; al < J; ++al) g = fma(LV(dZ, al * H + i), LV(In, al * dl + j), g);
-            add(a.off_w[l] + i * dl + j, g);
-          }
-          add(a.off_b[l] + i, LV(dZ, i));
+        const int64_t ow = a.off_w[l], ob = a.off_b[l];
+        for (int k = u; k < H * dl; k += NU) {
+          const int i = k / dl, j = k - i * dl;
+          T gv = T(0);
+          for (int al = 0; al < J; ++al) gv = fma(LV(dZ, al * H + i), LV(In, al * dl + j), gv);
+          put(ow + k, gv);
         }
+        for (int i = u; i < H; i += NU) put(ob + i, LV(dZ, i));
         if (l > 0) {
           // dA of the layer below: W^T dZ
-          for (int al = 0; al < J; ++al)
-            for (int j = 0; j < H; ++j) {
-              T g = T(0);
-              for (int i = 0; i < H; ++i) g = fma(Wl[i * H + j], LV(dZ, al * H + i), g);
-              LV(dA, al * H + j) = g;
-            }
+          for (int k = u; k < JH; k += NU) {
+            const int al = k / H, j = k - al * H;
+            T gv = T(0);
+#pragma unroll 8
+            for (int i = 0; i < H; ++i) gv = fma(Wl[i * H + j], LV(dZ, al * H + i), gv);
+            LV(dA, k) = gv;
+          }
+          __syncthreads();
         }
       }
+      wrote |= act;
+      __syncthreads();
     }
+    // an entry without any seed: its column is zero
+    if (valid && !wrote)
+      for (int64_t k = u; k < a.n_params; k += NU) col[k * a.n_resid] = T(0);
   }
 #undef LV
 }
@@ -1028,6 +1093,10 @@ __global__ __launch_bounds__(256) void k_ad_step_sum(const float *partial, const
 struct tdx_ad_plan {
   int dtype, d_in, n_out, H, L, J;
   int64_t P, n_entries, n_resid, n_params;
+  std::vector<int64_t> group_counts;  // entries of each group
+  // every residual slot belongs to exactly one equation: the Jacobian kernel
+  // writes whole columns (else it adds into cleared ones)
+  bool resid_exact = false;
   int n_groups, groups_i, jet_i, pptr_i, part_i, n_parts, n_occ;
   // causal loss: tolerance, slices and points of group 0 (N = nt K), its
   // equations; workspace for residuals, weights and w * res
@@ -1313,6 +1382,19 @@ extern "C" int tdx_ad_plan_create(const tdx_ad_desc *d, tdx_ad_plan **out) {
   p->J = J;
   p->P = d->n_points;
   p->n_entries = gstart[d->n_groups];
+  {
+    std::vector<int32_t> owners((size_t)std::max<int64_t>(d->n_resid, 0), 0);
+    for (int g = 0; g < d->n_groups; ++g) {
+      const int32_t *G = I + d->groups_i + TDX_AD_GROUP_INTS * g;
+      p->group_counts.push_back(gstart[g + 1] - gstart[g]);
+      for (int q = 0; q < G[3]; ++q) {
+        const int32_t ro = I[G[4] + TDX_AD_EQ_INTS * q + 5];
+        if (ro >= 0)
+          for (int64_t e = 0; e < p->group_counts[g]; ++e) ++owners[(size_t)(ro + e)];
+      }
+    }
+    p->resid_exact = std::all_of(owners.begin(), owners.end(), [](int32_t c) { return c == 1; });
+  }
   p->n_resid = d->n_resid;
   p->max_sets = max_sets;
   p->n_groups = d->n_groups;
@@ -1763,14 +1845,18 @@ int ad_jacobian(const tdx_ad_plan *p, const T *params, T *jt, hipStream_t s) {
   const int NL = p->L - 1, J = p->J, H = p->H, no = p->n_out;
   const size_t words = (size_t)(2 * NL + 2) * J * H + (size_t)2 * p->max_sets * J * no +
                        (size_t)J * p->d_in;
-  int B = 64;
-  while (B > 1 && words * sizeof(T) * B > (160 * 1024)) B >>= 1;
-  TDX_REQUIRE(words * sizeof(T) * B <= (160 * 1024), "network too large for the Jacobian kernel");
+  int E = 4;
+  while (E < 16 && p->n_entries >= (int64_t)2 * E * 512) E <<= 1;
+  while (E > 1 && words * sizeof(T) * E > (160 * 1024)) E >>= 1;
+  TDX_REQUIRE(words * sizeof(T) * E <= (160 * 1024), "network too large for the Jacobian kernel");
   raise_lds_limit({(const void *)k_ad_jac<T>});
-  const int64_t n = p->n_params * p->n_resid;
-  hipLaunchKernelGGL((k_ad_jac_zero<T>), dim3((unsigned)std::min<int64_t>((n + 255) / 256, 65536)),
-                     dim3(256), 0, s, jt, n);
-  TDX_TRY_HIP(hipGetLastError());
+  if (!p->resid_exact) {
+    const int64_t n = p->n_params * p->n_resid;
+    hipLaunchKernelGGL((k_ad_jac_zero<T>),
+                       dim3((unsigned)std::min<int64_t>((n + 255) / 256, 65536)), dim3(256), 0, s,
+                       jt, n);
+    TDX_TRY_HIP(hipGetLastError());
+  }
   JacArgs<T> a;
   a.d_in = p->d_in;
   a.n_out = no;
@@ -1791,8 +1877,12 @@ int ad_jacobian(const tdx_ad_plan *p, const T *params, T *jt, hipStream_t s) {
   a.off_b = a.off_w + p->L;
   a.jt = jt;
   a.n_resid = p->n_resid;
-  const unsigned blocks = (unsigned)((p->n_entries + B - 1) / B);
-  hipLaunchKernelGGL((k_ad_jac<T>), dim3(blocks), dim3(B), words * sizeof(T) * B, s, a);
+  a.n_params = p->n_params;
+  a.accum = p->resid_exact ? 0 : 1;
+  int64_t blocks = 0;
+  for (int64_t c : p->group_counts) blocks += (c + E - 1) / E;
+  hipLaunchKernelGGL((k_ad_jac<T>), dim3((unsigned)blocks), dim3(256), words * sizeof(T) * E, s, a,
+                     E);
   TDX_TRY_HIP(hipGetLastError());
   return TDX_OK;
 }
