@@ -95,6 +95,13 @@ struct MatArgs {
   T *m;
   T *v;
   const T *adam;
+  // plans without a generated kernel: the Adam pass adds the boundary seeds'
+  // sum at a touched point itself (touch_map: index into the touched points
+  // or -1, per grid word; null: k_mat_bc_adj has added them) and forms the
+  // step's scalars (adam null: step_inc and the hyperparameters); the tile
+  // launch advances the step counter
+  const int32_t *touch_map;
+  int64_t *step_inc;
 };
 
 // x / h by division mode DIV: 0 multiplies by the rounded reciprocal inv
@@ -409,7 +416,7 @@ __device__ __forceinline__ void mat_tile_body(const MatArgs<T> &a, T *smem, int 
   // residual, loss and seeds on the tile plus R; each point is read and
   // written by one thread, so a term's seeds overwrite its factor values
   T lsum = T(0), lnsum = T(0);
-  const T dl = ADJ ? *a.dloss : T(0);
+  const T dl = ADJ ? (a.dloss ? *a.dloss : T(1)) : T(0);
   for_box(E1, tl, R0, 3 * R0 + T0, R1, 3 * R1 + T1, [&](int i0, int i1) {
     const int g0 = base0 + i0, g1 = base1 + i1, p = i0 * E1 + i1;
     const bool ing = in_grid(g0, g1);
@@ -569,61 +576,56 @@ __device__ __forceinline__ int xcd_band_tile(int b, int n) {
   return (b & 7) * per + (b >> 3);
 }
 
-template <typename T, int DP, int DIV, bool ADJ>
-__global__ __launch_bounds__(MAT_THREADS) void k_mat_tile(MatArgs<T> a) {
-  extern __shared__ __align__(16) unsigned char smem_raw[];
-  T *smem = reinterpret_cast<T *>(smem_raw);
-  const int tile = a.tile_list ? a.tile_list[blockIdx.x] : xcd_band_tile((int)blockIdx.x, (int)gridDim.x);
-  const int t0 = tile / a.tiles1, t1 = tile - (tile / a.tiles1) * a.tiles1;
-  const int base0 = t0 * a.T0 - 2 * a.R0, base1 = t1 * a.T1 - 2 * a.R1;
-  const bool interior = base0 >= 0 && base0 + a.E0 <= a.n0 && base1 >= 0 && base1 + a.E1 <= a.n1;
-  if (interior)
-    mat_tile_body<T, DP, DIV, ADJ, true>(a, smem, t0, t1);
-  else
-    mat_tile_body<T, DP, DIV, ADJ, false>(a, smem, t0, t1);
-}
-
 // ---------------------------------------------------------------------------
 // boundary entries: pointwise derivative chains straight from HBM
 // ---------------------------------------------------------------------------
-template <typename T, int DIV>
-__device__ T point_chain(const MatArgs<T> &a, const T *plane, int g0, int g1, const int *axes,
-                         int depth) {
-  // D_{axes[depth-1]} ... D_{axes[0]} u at (g0, g1), evaluated recursively
-  if (depth == 0) return plane[(int64_t)g0 * a.n1 + g1];
-  const int ax = axes[depth - 1];
-  const int g = ax == 0 ? g0 : g1;
-  const int n = ax == 0 ? a.n0 : a.n1;
-  const int dp = a.dp;
-  auto at = [&](int off) {
-    const int h0 = ax == 0 ? g0 + off : g0, h1 = ax == 0 ? g1 : g1 + off;
-    return point_chain<T, DIV>(a, plane, h0, h1, axes, depth - 1);
-  };
-  const T *ab = a.coef, *af = a.coef + MMAX_DP;
-  const T h = ax == 0 ? a.h0 : a.h1, ih = ax == 0 ? a.ih0 : a.ih1;
-  const T h2 = ax == 0 ? a.h20 : a.h21, ih2 = ax == 0 ? a.ih20 : a.ih21;
-  if (g < dp - 1) {
-    T f = at(0) * af[0];
-    for (int i = 1; i < dp; ++i) f = f + at(i) * af[i];
-    return qdiv<T, DIV>(f, h, ih);
+// D_{axes[depth-1]} ... D_{axes[0]} u at (g0, g1), D >= depth; the recursion
+// is unrolled (no stack).
+template <typename T, int DIV, int D>
+__device__ __forceinline__ T point_chain(const MatArgs<T> &a, const T *plane, int g0, int g1,
+                                         const int *axes, int depth) {
+  if constexpr (D == 0) {
+    return plane[(int64_t)g0 * a.n1 + g1];
+  } else {
+    if (depth == 0) return plane[(int64_t)g0 * a.n1 + g1];
+    const int ax = axes[depth - 1];
+    const int g = ax == 0 ? g0 : g1;
+    const int n = ax == 0 ? a.n0 : a.n1;
+    const int dp = a.dp;
+    const T *ab = a.coef, *af = a.coef + MMAX_DP;
+    const T h = ax == 0 ? a.h0 : a.h1, ih = ax == 0 ? a.ih0 : a.ih1;
+    const T h2 = ax == 0 ? a.h20 : a.h21, ih2 = ax == 0 ? a.ih20 : a.ih21;
+    const bool first = g < dp - 1, last = !first && g >= n - dp + 1;
+    // backward terms k < dp, then forward ones; an end takes one side
+    T b = T(0), f = T(0);
+#pragma unroll 1
+    for (int k = first ? dp : 0; k < (last ? dp : 2 * dp); ++k) {
+      const bool back = k < dp;
+      const int i = back ? k : k - dp;
+      const int off = back ? i - (dp - 1) : i;
+      const T v = point_chain<T, DIV, D - 1>(a, plane, ax == 0 ? g0 + off : g0,
+                                             ax == 0 ? g1 : g1 + off, axes, depth - 1);
+      const T w = v * (back ? ab[i] : af[i]);
+      if (back)
+        b = i == 0 ? w : b + w;
+      else
+        f = i == 0 ? w : f + w;
+    }
+    if (first) return qdiv<T, DIV>(f, h, ih);
+    if (last) return qdiv<T, DIV>(b, h, ih);
+    return qdiv<T, DIV>(b + f, h2, ih2);
   }
-  T b = at(-(dp - 1)) * ab[0];
-  for (int i = 1; i < dp; ++i) b = b + at(i - (dp - 1)) * ab[i];
-  if (g >= n - dp + 1) return qdiv<T, DIV>(b, h, ih);
-  T f = at(0) * af[0];
-  for (int i = 1; i < dp; ++i) f = f + at(i) * af[i];
-  return qdiv<T, DIV>(b + f, h2, ih2);
 }
 
 // Boundary entries: value, loss partials and (adj) seeds.  ND (full-grid
 // plans): the factor values are the chain fields at the entry's positions
 // (factor k of the entry's operator in field bc_slot[e] + k); otherwise the
 // chains are evaluated at the point (2-D, at most 3 applications).
+// red: 2 x MAT_THREADS words of LDS; blk: the boundary workgroup.
 template <typename T, int DIV, bool ND>
-__global__ __launch_bounds__(MAT_THREADS) void k_mat_bc(MatArgs<T> a, int adj) {
-  __shared__ T red[2 * MAT_THREADS];
+__device__ __forceinline__ void mat_bc_body(const MatArgs<T> &a, T *red, int blk, bool adj) {
   const int tid = threadIdx.x;
-  const int e = blockIdx.x * MAT_THREADS + tid;
+  const int e = blk * MAT_THREADS + tid;
   T lsum = T(0), lnsum = T(0);
   if (e < a.n_bc) {
     const int32_t *Bc = a.ints + a.bc_i + e * TDX_MBC_INTS;
@@ -638,7 +640,7 @@ __global__ __launch_bounds__(MAT_THREADS) void k_mat_bc(MatArgs<T> a, int adj) {
         return a.fields[(int64_t)(slot0 + k) * a.N + pos];
       } else {
         const int g0 = pos / a.n1, g1 = pos - (pos / a.n1) * a.n1;
-        return point_chain<T, DIV>(a, a.u + Fc[0] * a.N, g0, g1, Fc + 5, Fc[4]);
+        return point_chain<T, DIV, 3>(a, a.u + Fc[0] * a.N, g0, g1, Fc + 5, Fc[4]);
       }
     };
     T val = T(0);
@@ -679,7 +681,7 @@ __global__ __launch_bounds__(MAT_THREADS) void k_mat_bc(MatArgs<T> a, int adj) {
     lsum = lam_d * (diff * diff);
     lnsum = invden * (diff * diff);
     if (adj) {
-      const T dr = T(2) * lam_d * diff * (*a.dloss);
+      const T dr = T(2) * lam_d * diff * (a.dloss ? *a.dloss : T(1));
       int sidx = seed_i;
       T robin_w = T(1);
       if (Bc[9] > 0) {
@@ -729,23 +731,56 @@ __global__ __launch_bounds__(MAT_THREADS) void k_mat_bc(MatArgs<T> a, int adj) {
     __syncthreads();
   }
   if (tid == 0) {
-    a.lp[2 * (a.n_tile_wg + blockIdx.x)] = red[0];
-    a.lp[2 * (a.n_tile_wg + blockIdx.x) + 1] = red[MAT_THREADS];
+    a.lp[2 * (a.n_tile_wg + blk)] = red[0];
+    a.lp[2 * (a.n_tile_wg + blk) + 1] = red[MAT_THREADS];
   }
+}
+
+// The boundary entries of a full-grid plan (the others' run in the tile
+// kernel's launch).
+template <typename T, int DIV>
+__global__ __launch_bounds__(MAT_THREADS) void k_mat_bc(MatArgs<T> a, int adj) {
+  __shared__ T red[2 * MAT_THREADS];
+  mat_bc_body<T, DIV, true>(a, red, blockIdx.x, adj != 0);
+}
+
+// The tiles, then the boundary entries' workgroups: they read u alone, and a
+// launch of their own cost its latency again (128 x 128: 11 us beside the
+// tiles' 18).
+template <typename T, int DP, int DIV, bool ADJ>
+__global__ __launch_bounds__(MAT_THREADS) void k_mat_tile(MatArgs<T> a) {
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  T *smem = reinterpret_cast<T *>(smem_raw);
+  if (a.step_inc && blockIdx.x == 0 && threadIdx.x == 0) *a.step_inc += 1;
+  if ((int)blockIdx.x >= a.n_tile_wg) {
+    mat_bc_body<T, DIV, false>(a, smem, (int)blockIdx.x - a.n_tile_wg, ADJ);
+    return;
+  }
+  const int tile = a.tile_list ? a.tile_list[blockIdx.x] : xcd_band_tile((int)blockIdx.x, a.n_tile_wg);
+  const int t0 = tile / a.tiles1, t1 = tile - (tile / a.tiles1) * a.tiles1;
+  const int base0 = t0 * a.T0 - 2 * a.R0, base1 = t1 * a.T1 - 2 * a.R1;
+  const bool interior = base0 >= 0 && base0 + a.E0 <= a.n0 && base1 >= 0 && base1 + a.E1 <= a.n1;
+  if (interior)
+    mat_tile_body<T, DP, DIV, ADJ, true>(a, smem, t0, t1);
+  else
+    mat_tile_body<T, DP, DIV, ADJ, false>(a, smem, t0, t1);
 }
 
 // gradient of the boundary terms: one thread per touched grid point, fixed
 // order over its contributions (no atomics)
 template <typename T>
-__global__ void k_mat_bc_adj(MatArgs<T> a) {
-  const int j = blockIdx.x * blockDim.x + threadIdx.x;
-  if (j >= a.n_touch) return;
+__device__ __forceinline__ T touch_sum(const MatArgs<T> &a, int j) {
   const int32_t *ptr = a.ints + a.bct_ptr_i;
-  const int64_t pos = a.ints[a.bct_pos_i + j];
   T s = T(0);
   for (int k = ptr[j]; k < ptr[j + 1]; ++k)
     s += a.bc_seeds[a.ints[a.bct_seed_i + k]] * a.reals[a.ints[a.bct_w_i + k]];
-  a.grad[pos] += s;
+  return s;
+}
+template <typename T>
+__global__ void k_mat_bc_adj(MatArgs<T> a) {
+  const int j = blockIdx.x * blockDim.x + threadIdx.x;
+  if (j >= a.n_touch) return;
+  a.grad[a.ints[a.bct_pos_i + j]] += touch_sum(a, j);
 }
 
 // Sum of n (loss, normalized loss) pairs: workgroup b of the grid adds the
@@ -806,7 +841,7 @@ __global__ void k_mat_step_prep(T *one, int64_t *step, AdamHyper h, T *out) {
 template <typename T>
 __global__ __launch_bounds__(256) void k_mat_frame_adam(MatArgs<T> a, int r_lo, int r_hi,
                                                         int c_lo, int c_hi, const T *lp,
-                                                        int n_lp, T *loss) {
+                                                        int n_lp, T *loss, AdamHyper h) {
   // with loss: the last workgroup forms the loss pair from the n_lp
   // partial pairs (k_mat_loss in one workgroup) instead of updating points
   if (loss && blockIdx.x == gridDim.x - 1) {
@@ -820,12 +855,20 @@ __global__ __launch_bounds__(256) void k_mat_frame_adam(MatArgs<T> a, int r_lo, 
   const int64_t per = top + bot + (int64_t)(r_hi - r_lo) * wm;
   const int64_t tot = per * a.n_eq;
   AdamScalars<T> sc;
-  sc.w1 = a.adam[0];
-  sc.w2 = a.adam[1];
-  sc.b2 = a.adam[2];
-  sc.step_size = a.adam[3];
-  sc.bc2s = a.adam[4];
-  sc.eps = a.adam[5];
+  if (a.adam) {
+    sc.w1 = a.adam[0];
+    sc.w2 = a.adam[1];
+    sc.b2 = a.adam[2];
+    sc.step_size = a.adam[3];
+    sc.bc2s = a.adam[4];
+    sc.eps = a.adam[5];
+  } else {
+    // the step counter has been advanced by the tile launch
+    __shared__ AdamScalars<T> scs;
+    if (threadIdx.x == 0) scs = adam_scalars<T>(*a.step_inc, h);
+    __syncthreads();
+    sc = scs;
+  }
   const int64_t stride = (int64_t)n_upd * blockDim.x;
   for (int64_t idx = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; idx < tot; idx += stride) {
     const int64_t e = idx / per, k = idx - e * per;
@@ -844,8 +887,12 @@ __global__ __launch_bounds__(256) void k_mat_frame_adam(MatArgs<T> a, int r_lo, 
       col = j < wl ? j : c_hi + (j - wl);
     }
     const int64_t gi = e * a.N + row * n1 + col;
-    T p = a.u[gi], m = a.m[gi], v = a.v[gi];
-    adam_apply(p, a.grad[gi], m, v, sc);
+    T p = a.u[gi], m = a.m[gi], v = a.v[gi], g = a.grad[gi];
+    if (a.touch_map) {
+      const int j = a.touch_map[gi];
+      if (j >= 0) g += touch_sum(a, j);
+    }
+    adam_apply(p, g, m, v, sc);
     a.u_out[gi] = p;
     a.m[gi] = m;
     a.v[gi] = v;
@@ -1024,6 +1071,9 @@ struct tdx_mat_plan {
   int jit_fuse;     // no boundary adjoint touches the rectangle: the fused
                     // step updates it inside the generated kernel
   DevTable gen_list;
+  // small plans without a generated kernel: the fused step in two launches
+  int merged_step = 0;
+  DevTable touch_map;  // per grid word: its touched point's index or -1
   int n_gen_wg;
   size_t off_lp, off_mid, off_seeds, off_one, off_grad, off_adam, ws_bytes;
   double ab[MMAX_DP], af[MMAX_DP];
@@ -1149,6 +1199,8 @@ MatArgs<T> mat_args(const tdx_mat_plan *p, const void *u, void *ws) {
   a.m = nullptr;
   a.v = nullptr;
   a.adam = nullptr;
+  a.touch_map = nullptr;
+  a.step_inc = nullptr;
   return a;
 }
 
@@ -1156,12 +1208,13 @@ template <typename T, int DP, int DIV>
 int mat_tile_launch(const tdx_mat_plan *p, const MatArgs<T> &a, bool adj, hipStream_t s) {
   raise_lds_limit({(const void *)k_mat_tile<T, DP, DIV, true>,
                    (const void *)k_mat_tile<T, DP, DIV, false>});
-  if (p->n_gen_wg == 0) return TDX_OK;
+  const int wg = p->n_gen_wg + p->n_bc_wg;
+  if (wg == 0) return TDX_OK;
   if (adj)
-    hipLaunchKernelGGL((k_mat_tile<T, DP, DIV, true>), dim3(p->n_gen_wg), dim3(MAT_THREADS),
-                       p->tile_lds, s, a);
+    hipLaunchKernelGGL((k_mat_tile<T, DP, DIV, true>), dim3(wg), dim3(MAT_THREADS), p->tile_lds, s,
+                       a);
   else
-    hipLaunchKernelGGL((k_mat_tile<T, DP, DIV, false>), dim3(p->n_gen_wg), dim3(MAT_THREADS),
+    hipLaunchKernelGGL((k_mat_tile<T, DP, DIV, false>), dim3(wg), dim3(MAT_THREADS),
                        p->tile_lds_fwd, s, a);
   TDX_TRY_HIP(hipGetLastError());
   return TDX_OK;
@@ -1205,7 +1258,8 @@ int mat_jit_launch(const tdx_mat_plan *p, const MatArgs<T> &a, bool adj, hipStre
 }
 
 template <typename T, int DIV>
-int mat_run(const tdx_mat_plan *p, MatArgs<T> a, bool adj, T *loss, hipStream_t s) {
+int mat_run(const tdx_mat_plan *p, MatArgs<T> a, bool adj, T *loss, hipStream_t s,
+            const AdamHyper &h) {
   int rc = p->d.dp == 2   ? mat_tile_launch<T, 2, DIV>(p, a, adj, s)
            : p->d.dp == 3 ? mat_tile_launch<T, 3, DIV>(p, a, adj, s)
                           : mat_tile_launch<T, 0, DIV>(p, a, adj, s);
@@ -1214,15 +1268,9 @@ int mat_run(const tdx_mat_plan *p, MatArgs<T> a, bool adj, T *loss, hipStream_t 
     rc = mat_jit_launch<T>(p, a, adj, s);
     if (rc) return rc;
   }
-  if (p->n_bc_wg > 0) {
-    hipLaunchKernelGGL((k_mat_bc<T, DIV, false>), dim3(p->n_bc_wg), dim3(MAT_THREADS), 0, s, a,
-                       adj ? 1 : 0);
+  if (p->n_bc_wg > 0 && adj && p->d.n_touch > 0 && !a.touch_map) {
+    hipLaunchKernelGGL((k_mat_bc_adj<T>), dim3((p->d.n_touch + 255) / 256), dim3(256), 0, s, a);
     TDX_TRY_HIP(hipGetLastError());
-    if (adj && p->d.n_touch > 0) {
-      hipLaunchKernelGGL((k_mat_bc_adj<T>), dim3((p->d.n_touch + 255) / 256), dim3(256), 0, s,
-                         a);
-      TDX_TRY_HIP(hipGetLastError());
-    }
   }
   // loss partial pairs of the step's kernels
   const int var = adj && a.fused && p->jit_fuse ? 2 : adj ? 1 : 0;
@@ -1241,7 +1289,7 @@ int mat_run(const tdx_mat_plan *p, MatArgs<T> a, bool adj, T *loss, hipStream_t 
       const unsigned blocks =
           (unsigned)std::max<int64_t>(1, std::min<int64_t>((tot + 255) / 256, 16384));
       hipLaunchKernelGGL((k_mat_frame_adam<T>), dim3(blocks + (lw ? 1 : 0)), dim3(256), 0, s, a,
-                         r_lo, r_hi, c_lo, c_hi, (const T *)a.lp, n, lw);
+                         r_lo, r_hi, c_lo, c_hi, (const T *)a.lp, n, lw, h);
       TDX_TRY_HIP(hipGetLastError());
       if (lw) loss = nullptr;  // formed
     }
@@ -1310,7 +1358,7 @@ int mat_run_nd(const tdx_mat_plan *p, MatArgs<T> a, bool adj, T *loss, hipStream
                      adj ? 1 : 0);
   TDX_TRY_HIP(hipGetLastError());
   if (p->n_bc_wg > 0) {
-    hipLaunchKernelGGL((k_mat_bc<T, DIV, true>), dim3(p->n_bc_wg), dim3(MAT_THREADS), 0, s, a,
+    hipLaunchKernelGGL((k_mat_bc<T, DIV>), dim3(p->n_bc_wg), dim3(MAT_THREADS), 0, s, a,
                        adj ? 1 : 0);
     TDX_TRY_HIP(hipGetLastError());
   }
@@ -1362,7 +1410,7 @@ int mat_run_nd(const tdx_mat_plan *p, MatArgs<T> a, bool adj, T *loss, hipStream
       b.n1 = N;
       const int64_t tot = gw;
       hipLaunchKernelGGL((k_mat_frame_adam<T>), dim3(nd_blocks(tot)), dim3(256), 0, s, b, 0, 0,
-                         0, 0, (const T *)nullptr, 0, (T *)nullptr);
+                         0, 0, (const T *)nullptr, 0, (T *)nullptr, AdamHyper{0, 0, 0, 0});
       TDX_TRY_HIP(hipGetLastError());
     }
   }
@@ -1383,15 +1431,16 @@ int mat_run_nd(const tdx_mat_plan *p, MatArgs<T> a, bool adj, T *loss, hipStream
 }
 
 template <typename T>
-int mat_dispatch(const tdx_mat_plan *p, MatArgs<T> a, bool adj, T *loss, hipStream_t s) {
+int mat_dispatch(const tdx_mat_plan *p, MatArgs<T> a, bool adj, T *loss, hipStream_t s,
+                 const AdamHyper &h = AdamHyper{0, 0, 0, 0}) {
   if (p->nd) {
     if (p->div_mode == 0) return mat_run_nd<T, 0>(p, a, adj, loss, s);
     if (p->div_mode == 2) return mat_run_nd<T, 2>(p, a, adj, loss, s);
     return mat_run_nd<T, 1>(p, a, adj, loss, s);
   }
-  if (p->div_mode == 0) return mat_run<T, 0>(p, a, adj, loss, s);
-  if (p->div_mode == 2) return mat_run<T, 2>(p, a, adj, loss, s);
-  return mat_run<T, 1>(p, a, adj, loss, s);
+  if (p->div_mode == 0) return mat_run<T, 0>(p, a, adj, loss, s, h);
+  if (p->div_mode == 2) return mat_run<T, 2>(p, a, adj, loss, s, h);
+  return mat_run<T, 1>(p, a, adj, loss, s, h);
 }
 
 }  // namespace
@@ -1898,7 +1947,43 @@ extern "C" int tdx_mat_plan_create(const tdx_mat_desc *d, tdx_mat_plan **out) {
       int e0 = (int)((48 * 1024 - std::min<size_t>(fixed, 32 * 1024)) / ((size_t)p->E1 * words * ts));
       e0 = std::min(e0, d->n0 + 4 * p->R0);
       e0 = e0 / rps * rps;
-      if (e0 - 4 * p->R0 < 8) e0 = min_rows(rps);
+      if (e0 - 4 * p->R0 < 8) {
+        e0 = min_rows(rps);
+      } else {
+        // A workgroup takes about 6 us plus 4 us per sweep of rps rows
+        // whatever its neighbours on the CU do (dependent LDS passes), so
+        // the launch takes max(1, workgroups / resident ones) times that:
+        // small grids want short tiles (128 x 128: 36 rows on 15 workgroups
+        // 57 us, 12 rows on 96 32 us), large ones the tallest that keep few
+        // rounds.  Partial last rounds count half.  With a generated
+        // interior only the edge tiles are launched.
+        const bool edges = d->dtype == 0 && d->specialize >= 0 && N >= (1 << 20) + (1 << 17);
+        double best = 0;
+        const int top = e0;
+        const int T1 = p->E1 - 4 * p->R1, c = (d->n1 + T1 - 1) / T1;
+        for (int r = 4 * p->R0 + rps; r / rps * rps <= top; r += rps) {
+          const int E = r / rps * rps, T0 = E - 4 * p->R0;
+          if (T0 < 1) continue;
+          const int64_t rows = (d->n0 + T0 - 1) / T0;
+          int64_t wg = rows * c;
+          if (edges) {
+            int64_t ir = 0, ic = 0;
+            for (int64_t t = 0; t < rows; ++t)
+              ir += t * T0 >= 2 * p->R0 && t * T0 - 2 * p->R0 + E <= d->n0;
+            for (int64_t t = 0; t < c; ++t)
+              ic += t * T1 >= 2 * p->R1 && t * T1 - 2 * p->R1 + p->E1 <= d->n1;
+            wg -= ir * ic;
+          }
+          const double slots =
+              256.0 * std::max<size_t>(1, std::min<size_t>(8, 160 * 1024 / lds_for(E, p->E1)));
+          const double q = (double)wg / slots;
+          const double cost = std::max(1.0, 0.5 * (q + std::ceil(q))) * (1.5 + (double)E / rps);
+          if (best == 0 || cost < best) {
+            best = cost;
+            e0 = E;
+          }
+        }
+      }
       p->E0 = e0;
       while (lds_for(p->E0, p->E1) > 160 * 1024 && p->E1 > 16 && p->E1 / 2 - 4 * p->R1 >= 8) {
         p->E1 /= 2;
@@ -1964,6 +2049,26 @@ extern "C" int tdx_mat_plan_create(const tdx_mat_desc *d, tdx_mat_plan **out) {
     tdx_mat_plan_destroy(p);
     return rc;
   }
+  // Two-launch step (train_step_to) where launches cost more than the Adam
+  // pass's extra word per point: up to 2^20 grid words (128 x 128: 63 -> 24 us
+  // a step with the smaller tiles); larger grids keep the boundary adjoint's
+  // own launch.  A touched point listed twice keeps it too.
+  if (!p->nd && !p->jit_on && N * d->n_eq <= (1 << 20)) {
+    std::vector<int32_t> map((size_t)(N * d->n_eq), -1);
+    p->merged_step = 1;
+    for (int j = 0; j < d->n_touch; ++j) {
+      int32_t &m = map[(size_t)d->ints[d->bct_pos_i + j]];
+      if (m >= 0) p->merged_step = 0;
+      m = j;
+    }
+    if (p->merged_step && d->n_touch > 0) {
+      rc = p->touch_map.upload(map.data(), map.size() * 4);
+      if (rc) {
+        tdx_mat_plan_destroy(p);
+        return rc;
+      }
+    }
+  }
   p->d.ints = nullptr;
   p->d.reals = nullptr;
   p->d.data = nullptr;
@@ -2010,6 +2115,7 @@ extern "C" void tdx_mat_plan_destroy(tdx_mat_plan *p) {
   p->sc_idx.release();
   p->ints.release();
   p->gen_list.release();
+  p->touch_map.release();
   p->reals.release();
   p->data.release();
   p->fs_tab.release();
@@ -2096,31 +2202,28 @@ extern "C" int tdx_mat_train_step_to(const tdx_mat_plan *p, const void *u_in, vo
   hipStream_t s = (hipStream_t)stream;
   const AdamHyper h{lr, b1, b2, eps};
   char *w = (char *)ws;
-  int rc;
-  if (p->d.dtype == 0) {
-    MatArgs<float> a = mat_args<float>(p, u_in, ws);
-    a.grad = (float *)(w + p->off_grad);
+  auto run = [&](auto tag) -> int {
+    using T = decltype(tag);
+    MatArgs<T> a = mat_args<T>(p, u_in, ws);
+    a.grad = (T *)(w + p->off_grad);
     a.fused = 1;
-    a.u_out = (float *)u_out;
-    a.m = (float *)m;
-    a.v = (float *)v;
-    a.adam = (const float *)(w + p->off_adam);
-    hipLaunchKernelGGL((k_mat_step_prep<float>), dim3(1), dim3(64), 0, s,
-                       (float *)(w + p->off_one), step, h, (float *)(w + p->off_adam));
-    rc = mat_dispatch<float>(p, a, true, (float *)loss, s);
-  } else {
-    MatArgs<double> a = mat_args<double>(p, u_in, ws);
-    a.grad = (double *)(w + p->off_grad);
-    a.fused = 1;
-    a.u_out = (double *)u_out;
-    a.m = (double *)m;
-    a.v = (double *)v;
-    a.adam = (const double *)(w + p->off_adam);
-    hipLaunchKernelGGL((k_mat_step_prep<double>), dim3(1), dim3(64), 0, s,
-                       (double *)(w + p->off_one), step, h, (double *)(w + p->off_adam));
-    rc = mat_dispatch<double>(p, a, true, (double *)loss, s);
-  }
-  return rc;
+    a.u_out = (T *)u_out;
+    a.m = (T *)m;
+    a.v = (T *)v;
+    if (p->merged_step) {
+      // two launches: tiles and boundary entries (unit seed scale, step
+      // counter), then boundary adjoint, Adam and the loss pair
+      a.dloss = nullptr;
+      a.step_inc = step;
+      a.touch_map = p->d.n_touch > 0 ? (const int32_t *)p->touch_map.ptr : nullptr;
+    } else {
+      a.adam = (const T *)(w + p->off_adam);
+      hipLaunchKernelGGL((k_mat_step_prep<T>), dim3(1), dim3(64), 0, s, (T *)(w + p->off_one),
+                         step, h, (T *)(w + p->off_adam));
+    }
+    return mat_dispatch<T>(p, a, true, (T *)loss, s, h);
+  };
+  return p->d.dtype == 0 ? run(0.0f) : run(0.0);
 }
 
 extern "C" int tdx_mat_train_step(const tdx_mat_plan *p, void *u, void *m, void *v,
