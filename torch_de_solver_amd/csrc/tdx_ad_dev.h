@@ -159,6 +159,10 @@ struct ADStepArgs {
   float *lp;          // [items][2]
 };
 
+// Workgroups a CU keeps resident: two for networks of up to four blocks
+// (57 KB of LDS, half the registers), whose waits on LDS, L2 and each other
+// then overlap; wider ones fill the registers with one.
+__host__ __device__ constexpr int ad_step_wgs(int NB) { return NB <= 4 ? 2 : 1; }
 __host__ __device__ inline size_t ad_step_lds_bytes(int HP) {
   return (size_t)(3 * HP * CTRS + (MAXD + 1 + MAXO) * CTRS + 2 * 64 * MAXO + 32) * 4;
 }
@@ -629,34 +633,39 @@ __device__ __forceinline__ void ad_step_body(const ADStepArgs &a, float *smem) {
       wave_sync();
       JP::fwd(zbuf, dbuf, r0w, NP, rNP, J, H, tb, lane);
       __syncthreads();
-      // owned blocks of dW_jj over the 64 rows, 32 at a time (an input
-      // block's activations split once for all owned output blocks); the
-      // bias over value rows
-#pragma unroll 1
-      for (int kk = 0; kk < 2; ++kk) {
-        const int r8 = 32 * kk + 8 * q;
-        f4_t m0, m1;
-        rows8(xbuf, col_b1, r8, m0, m1);
-        Bf3 ds[OBW];
+      // owned blocks of dW_jj over the 64 rows in two steps of 32, as in the
+      // block-owning kernel; the bias over value rows
+      {
+        Bf3 ds[OBW][2];
 #pragma unroll
         for (int u = 0; u < OBW; ++u) {
           const int ob = w + 4 * u;
-          if (ob < NB) {
-            f4_t lo, hi;
+          if (ob >= NB) continue;
+#pragma unroll
+          for (int kk = 0; kk < 2; ++kk) {
+            const int r8 = 32 * kk + 8 * q;
+            f4_t lo, hi, m0, m1;
+            rows8(xbuf, col_b1, r8, m0, m1);
             rows8(abuf, 16 * ob + row, r8, lo, hi);
-            bhacc[jj][u] += ((lo[0] * m0[0] + lo[1] * m0[1]) + (lo[2] * m0[2] + lo[3] * m0[3])) +
-                            ((hi[0] * m1[0] + hi[1] * m1[1]) + (hi[2] * m1[2] + hi[3] * m1[3]));
-            ds[u] = bf3_split(lo, hi);
+            bhacc[jj][u] +=
+                ((lo[0] * m0[0] + lo[1] * m0[1]) + (lo[2] * m0[2] + lo[3] * m0[3])) +
+                ((hi[0] * m1[0] + hi[1] * m1[1]) + (hi[2] * m1[2] + hi[3] * m1[3]));
+            ds[u][kk] = bf3_split(lo, hi);
           }
         }
 #pragma unroll
         for (int ib = 0; ib < NB; ++ib) {
-          f4_t lo, hi;
-          rows8(dbuf, 16 * ib + row, r8, lo, hi);
-          const Bf3 as = bf3_split(lo, hi);
+          __builtin_amdgcn_sched_barrier(0);
+          Bf3 as[2];
+#pragma unroll
+          for (int kk = 0; kk < 2; ++kk) {
+            f4_t lo, hi;
+            rows8(dbuf, 16 * ib + row, 32 * kk + 8 * q, lo, hi);
+            as[kk] = bf3_split(lo, hi);
+          }
 #pragma unroll
           for (int u = 0; u < OBW; ++u)
-            if (w + 4 * u < NB) dwacc[jj][u][ib] = mma3(ds[u], as, dwacc[jj][u][ib]);
+            if (w + 4 * u < NB) dwacc[jj][u][ib] = mma3_pair(ds[u], as, dwacc[jj][u][ib]);
         }
       }
       // dA of layer j - 1 = W_jj^T dZ_j for this wavefront's rows

@@ -126,6 +126,13 @@ __device__ __forceinline__ V mma3(const Bf3 &a, const Bf3 &b, V c) {
   return mma_bf(a.h, b.h, c) + s;
 }
 
+// c + a[0] b[0] + a[1] b[1]: two steps, one sum of small products.
+template <typename V>
+__device__ __forceinline__ V mma3_pair(const Bf3 (&a)[2], const Bf3 (&b)[2], V c) {
+  const V s = mma3_small(a[1], b[1], mma3_small(a[0], b[0], V{}));
+  return mma_bf(a[1].h, b[1].h, mma_bf(a[0].h, b[0].h, c)) + s;
+}
+
 // Row of the 16x16 MFMA accumulator held in register i of a lane in
 // quarter q (= lane / 16); the column is lane % 16.  The f32 and f64
 // 16x16x4 instructions place rows differently.

@@ -801,7 +801,8 @@ k_fused(NNArgs<float> a) {
 // tdx_nn_dev.h) with the interpreted residual program where it forms its
 // own seeds.
 template <typename T, int NB, int NH, bool FS>
-__global__ __launch_bounds__(256) void k_backward_c(NNArgs<T> a) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(block_wgs(NB, NH)))) void
+k_backward_c(NNArgs<T> a) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
   block_body<T, NB, NH, FS, BlockInterp<T>>(a, reinterpret_cast<T *>(smem_raw));
 }

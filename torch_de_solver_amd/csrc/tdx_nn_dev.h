@@ -293,39 +293,39 @@ __device__ __forceinline__ void split_act(const float (&b)[NB][4], Bf3 (&s)[(NB 
 template <int NB>
 __device__ __forceinline__ void mma_split(const float *img, int lane,
                                           const Bf3 (&s)[(NB + 1) / 2], f4_t (&acc)[NB]) {
-  constexpr int KS = (NB + 1) / 2;
-  Bf3 w[2][KS];
+  // operand steps t = ob * KS + ks in a ring, KS steps ahead when wide
+  constexpr int KS = (NB + 1) / 2, NT = NB * KS, AHEAD = KS > 1 ? KS : 1, RING = AHEAD + 1;
+  Bf3 w[RING];
   // wide images are in global memory (never staged): buffer loads take a
   // scalar descriptor and offset and one lane offset, so no address occupies
   // vector registers (as plain pointers the tile loop's hoisted addresses
   // spilled up to 2 KB a lane)
   const auto rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(img), (short)0,
-                                                    NB * KS * 3072, 0x00027000);
-  auto load = [&](int ob, Bf3 (&d)[KS]) {
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
-      if constexpr (KS > 1) {
-        const int o = 16 * lane, so = (ob * KS + ks) * 3072;
-        d[ks].h = __builtin_amdgcn_raw_buffer_load_b128(rs, o, so, 0);
-        d[ks].m = __builtin_amdgcn_raw_buffer_load_b128(rs, o, so + 1024, 0);
-        d[ks].l = __builtin_amdgcn_raw_buffer_load_b128(rs, o, so + 2048, 0);
-      } else {
-        const u4_t *p = reinterpret_cast<const u4_t *>(img) + lane + (ob * KS + ks) * 192;
-        d[ks].h = p[0], d[ks].m = p[64], d[ks].l = p[128];
-      }
+                                                    NT * 3072, 0x00027000);
+  auto load = [&](int t, Bf3 &d) {
+    if constexpr (KS > 1) {
+      const int o = 16 * lane, so = t * 3072;
+      d.h = __builtin_amdgcn_raw_buffer_load_b128(rs, o, so, 0);
+      d.m = __builtin_amdgcn_raw_buffer_load_b128(rs, o, so + 1024, 0);
+      d.l = __builtin_amdgcn_raw_buffer_load_b128(rs, o, so + 2048, 0);
+    } else {
+      const u4_t *p = reinterpret_cast<const u4_t *>(img) + lane + t * 192;
+      d.h = p[0], d.m = p[64], d.l = p[128];
     }
   };
-  load(0, w[0]);
+#pragma unroll
+  for (int t = 0; t < AHEAD; ++t)
+    if (t < NT) load(t, w[t % RING]);
 #pragma unroll
   for (int ob = 0; ob < NB; ++ob) {
-    if (ob + 1 < NB) load(ob + 1, w[(ob + 1) & 1]);
-    if constexpr (KS > 1) __builtin_amdgcn_sched_barrier(0);
-    const Bf3(&wo)[KS] = w[ob & 1];
     f4_t c = {0, 0, 0, 0}, c2 = {0, 0, 0, 0};
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
-      c = mma_bf(wo[ks].h, s[ks].h, c);
-      c2 = mma3_small(wo[ks], s[ks], c2);
+      const int t = ob * KS + ks;
+      if (t + AHEAD < NT) load(t + AHEAD, w[(t + AHEAD) % RING]);
+      if constexpr (KS > 1) __builtin_amdgcn_sched_barrier(0);
+      c = mma_bf(w[t % RING].h, s[ks].h, c);
+      c2 = mma3_small(w[t % RING], s[ks], c2);
     }
     acc[ob] += c + c2;
     if constexpr (KS > 1) __builtin_amdgcn_sched_barrier(0);
@@ -1055,6 +1055,13 @@ __host__ __device__ inline size_t block_fs_lds_words(int HP, int NH) {
   return block_lds_words(HP, NH) + 2 * 64 * MAXO + FUSE_PI + FUSE_PR;
 }
 
+// Workgroups a CU keeps resident: two where LDS (160 KB) and half the
+// registers hold the kernel, whose waits then overlap (KdV 512 x 128 on
+// 2-64x4-1: one 484 us a step, two 366 us).
+__host__ __device__ constexpr int block_wgs(int NB, int NH) {
+  return NB <= 4 && ((NH + 1) * 16 * NB * CTRS + 2000) * 4 <= 80 * 1024 ? 2 : 1;
+}
+
 // Residual policy of the library's block-owning kernel: the group's
 // program tables (a self-contained pair) copied to LDS and interpreted by
 // entry_program.  g < 0: no program (the adjoint of a forward pass).
@@ -1283,33 +1290,39 @@ __device__ __forceinline__ void block_body(const NNArgs<T> &a, T *smem) {
       T *dbuf = layer_buf(j);  // delta_j over act_j (read for the last time above)
       store_rows(dbuf, dl);
       __syncthreads();
-      // owned blocks of dW_jj over the 64 rows, 32 at a time; hidden bias from
-      // the delta operand (each lane holds 8 rows of one feature).  An input
-      // block's activations are split once for all owned output blocks.
-#pragma unroll 1
-      for (int kk = 0; kk < TR / 32; ++kk) {
-        const int r8 = 32 * kk + 8 * q;
-        Bf3 ds[OBW];
+      // owned blocks of dW_jj over the 64 rows in two steps of 32; hidden bias
+      // from the delta operand (each lane holds 8 rows of one feature).  An
+      // input block's activations are split once for all owned output blocks,
+      // and both steps' small products share one sum: the accumulators sit in
+      // the accumulation registers, where adding to them costs moves.
+      {
+        Bf3 ds[OBW][2];
 #pragma unroll
         for (int u = 0; u < OBW; ++u) {
           const int ob = w + 4 * u;
-          if (ob < NB) {
+          if (ob >= NB) continue;
+#pragma unroll
+          for (int kk = 0; kk < 2; ++kk) {
             f4_t lo, hi;
-            rows8(dbuf, 16 * ob + row, r8, lo, hi);
+            rows8(dbuf, 16 * ob + row, 32 * kk + 8 * q, lo, hi);
             bhacc[jj][u] += ((lo[0] + lo[1]) + (lo[2] + lo[3])) +
                             ((hi[0] + hi[1]) + (hi[2] + hi[3]));
-            ds[u] = bf3_split(lo, hi);
+            ds[u][kk] = bf3_split(lo, hi);
           }
         }
 #pragma unroll
         for (int ib = 0; ib < NB; ++ib) {
           __builtin_amdgcn_sched_barrier(0);
-          f4_t lo, hi;
-          rows8(ain, 16 * ib + row, r8, lo, hi);
-          const Bf3 as = bf3_split(lo, hi);
+          Bf3 as[2];
+#pragma unroll
+          for (int kk = 0; kk < 2; ++kk) {
+            f4_t lo, hi;
+            rows8(ain, 16 * ib + row, 32 * kk + 8 * q, lo, hi);
+            as[kk] = bf3_split(lo, hi);
+          }
 #pragma unroll
           for (int u = 0; u < OBW; ++u)
-            if (w + 4 * u < NB) dwacc[jj][u][ib] = mma3(ds[u], as, dwacc[jj][u][ib]);
+            if (w + 4 * u < NB) dwacc[jj][u][ib] = mma3_pair(ds[u], as, dwacc[jj][u][ib]);
         }
       }
       // delta_{j-1} = (W_jj^T delta_j) * (1 - act_{j-1}^2) for this

@@ -255,7 +255,10 @@ std::string nn_block_jit_source(const std::vector<std::vector<int32_t>> &keys,
        "  }\n"
        "};\n"
        "}  // namespace tdx\n"
-       "extern \"C\" __global__ __launch_bounds__(256) void tdx_block_jit(tdx::NNArgs<float> a) {\n"
+       "extern \"C\" __global__ __launch_bounds__(256)\n"
+       "__attribute__((amdgpu_waves_per_eu(tdx::block_wgs("
+    << NB << ", " << NH
+    << ")))) void tdx_block_jit(tdx::NNArgs<float> a) {\n"
        "  extern __shared__ __align__(16) unsigned char smem_raw[];\n"
        "  tdx::block_body<float, "
     << NB << ", " << NH
