@@ -1020,7 +1020,8 @@ __global__ void k_ad_jac_zero(T *jt, int64_t n) {
 // k_ad_step: the fused training step with the jet maps and the residual
 // program interpreted from the plan's tables.
 template <int NB, int NHM>
-__global__ __launch_bounds__(256) void k_ad_step(ADStepArgs a) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ad_step_wgs(NB)))) void
+k_ad_step(ADStepArgs a) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
   ad_step_body<NB, NHM, InterpJets, InterpADResid>(a, reinterpret_cast<float *>(smem_raw));
 }
@@ -1030,20 +1031,23 @@ __global__ __launch_bounds__(256) void k_ad_step(ADStepArgs a) {
 template <int NB>
 __global__ void k_ad_pack(NNArgs<float> a, int64_t *step) {
   constexpr int HP = 16 * NB;
-  if (blockIdx.x == 0 && threadIdx.x == 0) *step += 1;
+  if (step && blockIdx.x == 0 && threadIdx.x == 0) *step += 1;
   const int IMG = image_words(HP, a.NH, a.d_in, a.n_out, 4);
   for (int t = blockIdx.x * blockDim.x + threadIdx.x; t < IMG; t += gridDim.x * blockDim.x)
     a.packed[t] = image_value<float, NB>(a, a.params, t);
 }
 
 // Fixed-order sums of the items' gradient partials and loss pairs, and the
-// Adam update at step *step (already advanced).  Workgroup 0 forms the loss
-// pair; the others one parameter per thread.
+// Adam update at step *step (already advanced), or with grad the gradient
+// times *dloss.  Workgroup 0 forms the loss pair (loss null: not wanted); the
+// others one parameter per thread.
 __global__ __launch_bounds__(256) void k_ad_step_sum(const float *partial, const float *lp,
                                                      int n_items, int64_t P, float *params,
                                                      float *m, float *v, const int64_t *step,
-                                                     AdamHyper h, float *loss) {
+                                                     AdamHyper h, float *loss,
+                                                     const float *dloss, float *grad) {
   if (blockIdx.x == 0) {
+    if (!loss) return;
     __shared__ float r[512];
     float s0 = 0.f, s1 = 0.f;
     for (int k = threadIdx.x; k < n_items; k += 256) {
@@ -1078,6 +1082,10 @@ __global__ __launch_bounds__(256) void k_ad_step_sum(const float *partial, const
   }
   for (; k < n_items; ++k) acc[0] += partial[(int64_t)k * P + p];
   const float g = ((acc[0] + acc[1]) + (acc[2] + acc[3])) + ((acc[4] + acc[5]) + (acc[6] + acc[7]));
+  if (grad) {
+    grad[p] = g * *dloss;
+    return;
+  }
   float pv = params[p], mv = m[p], vv = v[p];
   adam_apply(pv, g, mv, vv, adam_scalars<float>(*step, h));
   params[p] = pv;
@@ -1355,7 +1363,8 @@ AdJitSpec ad_jit_spec(const tdx_ad_desc *d, const std::vector<int32_t> &occ, int
   sp.n_out = d->n_out;
   sp.occ = occ;
   sp.NB = nb;
-  sp.NHM = nhm;
+  // the layers the network has: fewer accumulators than the library's kernel
+  sp.NHM = std::max(1, std::min(nhm, d->n_layers - 2));
   return sp;
 }
 
@@ -1509,13 +1518,14 @@ extern "C" int tdx_ad_plan_create(const tdx_ad_desc *d, tdx_ad_plan **out) {
     }
     const size_t lds = ad_step_lds_bytes(16 * nb);
     if (ok) {
-      // about one work item per compute unit (the kernel runs one
-      // workgroup per compute unit); TDX_AD_TILES sets tiles per item
+      // about one work item per resident workgroup (ad_step_wgs a compute
+      // unit); TDX_AD_TILES sets tiles per item
       int dev = 0, ncu = 256;
       if (hipGetDevice(&dev) != hipSuccess ||
           hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
           ncu < 1)
         ncu = 256;
+      ncu *= ad_step_wgs(nb);
       int64_t tpi = (total_tiles + ncu - 1) / ncu;
       const char *te = std::getenv("TDX_AD_TILES");
       if (te && std::atoi(te) > 0) tpi = std::atoi(te);
@@ -1828,10 +1838,23 @@ extern "C" int tdx_ad_forward(const tdx_ad_plan *p, const void *params, void *lo
   return ad_forward<double>(p, (const double *)params, (double *)loss, (double *)resid, ws, s);
 }
 
+namespace {
+int ad_fused_step(const tdx_ad_plan *p, float *params, float *m, float *v, int64_t *step,
+                  const AdamHyper &h, float *loss, void *ws, hipStream_t s,
+                  const float *dloss = nullptr, float *grad = nullptr);
+}  // namespace
+
 extern "C" int tdx_ad_backward(const tdx_ad_plan *p, const void *params, const void *dloss,
                                void *dparams, void *ws, tdx_stream_t stream) {
   TDX_REQUIRE(p && params && dloss && dparams && ws, "null argument");
   hipStream_t s = (hipStream_t)stream;
+  // the fused step's kernel forms the jets again instead of reading the
+  // layers' arrays, and is still faster than the layer kernels' adjoint with
+  // its products per layer (133 x 91 Poisson, 2-64x3-1: 350 -> 95 us)
+  if (p->fused)
+    return ad_fused_step(p, (float *)const_cast<void *>(params), nullptr, nullptr, nullptr,
+                         AdamHyper{0, 0, 0, 0}, nullptr, ws, s, (const float *)dloss,
+                         (float *)dparams);
   if (p->dtype == 0)
     return ad_backward<float>(p, (const float *)params, (const float *)dloss, (float *)dparams, ws, s);
   return ad_backward<double>(p, (const double *)params, (const double *)dloss, (double *)dparams,
@@ -1925,9 +1948,11 @@ int ad_pack_launch(const NNArgs<float> &nn, int64_t *step, hipStream_t s) {
 }
 
 // The fused training step: three launches (image and step counter, the
-// step kernel, gradient sums with the Adam update and the loss pair).
+// step kernel, gradient sums with the Adam update and the loss pair).  With
+// grad: the gradient times *dloss instead of the update.
 int ad_fused_step(const tdx_ad_plan *p, float *params, float *m, float *v, int64_t *step,
-                  const AdamHyper &h, float *loss, void *ws, hipStream_t s) {
+                  const AdamHyper &h, float *loss, void *ws, hipStream_t s, const float *dloss,
+                  float *grad) {
   NNArgs<float> nn{};
   nn.d_in = p->d_in;
   nn.n_out = p->n_out;
@@ -1963,10 +1988,18 @@ int ad_fused_step(const tdx_ad_plan *p, float *params, float *m, float *v, int64
   a.partial = wsp<float>(ws, p->off_fpart);
   a.lp = wsp<float>(ws, p->off_flp);
   switch (p->f_nb) {
-    case 1: rc = ad_step_launch<1, 4>(p, a, s); break;
-    case 2: rc = ad_step_launch<2, 4>(p, a, s); break;
-    case 3: rc = ad_step_launch<3, 4>(p, a, s); break;
-    case 4: rc = ad_step_launch<4, 4>(p, a, s); break;
+    case 1:
+      rc = nn.NH <= 2 ? ad_step_launch<1, 2>(p, a, s) : ad_step_launch<1, 4>(p, a, s);
+      break;
+    case 2:
+      rc = nn.NH <= 2 ? ad_step_launch<2, 2>(p, a, s) : ad_step_launch<2, 4>(p, a, s);
+      break;
+    case 3:
+      rc = nn.NH <= 2 ? ad_step_launch<3, 2>(p, a, s) : ad_step_launch<3, 4>(p, a, s);
+      break;
+    case 4:
+      rc = nn.NH <= 2 ? ad_step_launch<4, 2>(p, a, s) : ad_step_launch<4, 4>(p, a, s);
+      break;
     case 5: rc = ad_step_launch<5, 4>(p, a, s); break;
     case 6: rc = ad_step_launch<6, 4>(p, a, s); break;
     case 7: rc = ad_step_launch<7, 4>(p, a, s); break;
@@ -1975,7 +2008,7 @@ int ad_fused_step(const tdx_ad_plan *p, float *params, float *m, float *v, int64
   if (rc != TDX_OK) return rc;
   hipLaunchKernelGGL(k_ad_step_sum, dim3((unsigned)(1 + (p->n_params + 255) / 256)), dim3(256), 0,
                      s, (const float *)a.partial, (const float *)a.lp, p->n_fitems,
-                     (int64_t)p->n_params, params, m, v, (const int64_t *)step, h, loss);
+                     (int64_t)p->n_params, params, m, v, (const int64_t *)step, h, loss, dloss, grad);
   TDX_TRY_HIP(hipGetLastError());
   return TDX_OK;
 }

@@ -280,7 +280,10 @@ std::string ad_step_jit_source(const AdJitSpec &sp) {
     o << "    } break;\n";
   }
   o << "    default: break;\n    }\n  }\n};\n}  // namespace tdx\n"
-       "extern \"C\" __global__ __launch_bounds__(256) void tdx_ad_step_jit(tdx::ADStepArgs a) {\n"
+       "extern \"C\" __global__ __launch_bounds__(256)\n"
+       "__attribute__((amdgpu_waves_per_eu(tdx::ad_step_wgs("
+    << sp.NB
+    << ")))) void tdx_ad_step_jit(tdx::ADStepArgs a) {\n"
        "  extern __shared__ __align__(16) unsigned char smem_raw[];\n"
        "  tdx::ad_step_body<"
     << sp.NB << ", " << sp.NHM
