@@ -16,6 +16,10 @@
 
 namespace tdx {
 
+// A plan's workspace with fixed work items and float32 operand images.
+size_t nn_workspace_fixed_bytes(const tdx_nn_plan *p);
+
+
 void set_error(const char *fmt, ...);
 void clear_error();
 

@@ -1267,6 +1267,7 @@ struct tdx_nn_plan;
 static size_t wave_private_lds(const tdx_nn_plan *p, const tdx_nn_desc *d);
 
 struct tdx_nn_plan {
+  size_t ws_fixed = 0;  // workspace with fixed work items (tdx_nn_plan_create)
   int dtype, d_in, n_out, H, n_layers, NH, NB, HP, P, n_inst;
   int n_groups;
   int max_slots;      // largest slot count of a group
@@ -2018,7 +2019,9 @@ bool fused_programs(const tdx_nn_desc *d, std::vector<FusedProg> *out) {
 
 }  // namespace
 
-extern "C" int tdx_nn_plan_create(const tdx_nn_desc *d, tdx_nn_plan **out) {
+// fixed: work items of fixed numbers of tiles (the workspace's gradient
+// partials grow with the items).
+static int nn_plan_create(const tdx_nn_desc *d, tdx_nn_plan **out, bool fixed) {
   TDX_REQUIRE(d && out, "null argument");
   *out = nullptr;
   TDX_REQUIRE(d->dtype == 0 || d->dtype == 1, "dtype must be 0 (f32) or 1 (f64)");
@@ -2153,6 +2156,7 @@ extern "C" int tdx_nn_plan_create(const tdx_nn_desc *d, tdx_nn_plan **out) {
   }
   const int chunk_tiles =
       d->chunk_tiles > 0  ? d->chunk_tiles
+      : fixed              ? (p->k2_wave_private ? 256 : p->k2_block ? 8 : p->acc_lds ? 16 : 4)
       : p->k2_wave_private ? pick_chunk(k2_tiles, 3 * kCUs, 256, 1.0)
       : p->k2_block        ? pick_chunk(k2_tiles, kCUs * block_residency<false>(p->NB, p->NH, nullptr, p->k2_lds), 16, 0.25)
                            : pick_chunk(k2_tiles, kCUs, p->acc_lds ? 16 : 4, 1.0);
@@ -2200,7 +2204,9 @@ extern "C" int tdx_nn_plan_create(const tdx_nn_desc *d, tdx_nn_plan **out) {
     std::vector<int64_t> blocks;
     for (int g = 0; g < d->n_groups; ++g)
       blocks.push_back((d->groups[(int64_t)g * TDX_GROUP_INTS + 1] + 63) / 64);
-    const int C = d->chunk_tiles > 0 ? d->chunk_tiles : pick_chunk(blocks, 4 * kCUs, 4, 0.25);
+    const int C = d->chunk_tiles > 0 ? d->chunk_tiles
+                  : fixed            ? 4
+                                     : pick_chunk(blocks, 4 * kCUs, 4, 0.25);
     for (int g = 0; g < d->n_groups; ++g) {
       const int32_t *G = d->groups + (int64_t)g * TDX_GROUP_INTS;
       const int nblk = (G[1] + 63) / 64;
@@ -2301,6 +2307,7 @@ extern "C" int tdx_nn_plan_create(const tdx_nn_desc *d, tdx_nn_plan **out) {
     }
     const int C = d->chunk_tiles > 0
                       ? d->chunk_tiles
+                  : fixed ? 8
                       : pick_chunk(tiles, kCUs * block_residency<true>(p->NB, p->NH, p->block_fn, p->k4_lds), 16,
                              0.25);
     for (int g = 0; g < d->n_groups; ++g) {
@@ -2451,9 +2458,53 @@ extern "C" int tdx_nn_plan_create(const tdx_nn_desc *d, tdx_nn_plan **out) {
     off = align_up(off + (size_t)p->w_N * p->w_neq * ts, 256);
   }
   p->ws_bytes = off;
+  {
+    // the workspace with fixed work items and float32 operand images, which
+    // the no-allocation entry point's limit is stated in
+    auto items_of = [&](auto tiles_of, int c) {
+      int64_t n = 0;
+      for (int g = 0; g < d->n_groups; ++g)
+        n += (tiles_of(d->groups + (int64_t)g * TDX_GROUP_INTS) + c - 1) / c;
+      return n;
+    };
+    const int c2 = d->chunk_tiles > 0    ? d->chunk_tiles
+                   : p->k2_wave_private ? 256
+                   : p->k2_block        ? 8
+                   : p->acc_lds         ? 16
+                                        : 4;
+    int64_t items = items_of(
+        [&](const int32_t *G) { return ((int64_t)G[1] * G[2] + TR - 1) / TR; }, c2);
+    if (p->fused)
+      items = std::max(items, items_of([](const int32_t *G) { return (int64_t)(G[1] + 63) / 64; },
+                                       d->chunk_tiles > 0 ? d->chunk_tiles : 4));
+    if (p->k2_fs)
+      items = std::max(items, items_of(
+                                  [](const int32_t *G) {
+                                    const int E = 64 / G[2];
+                                    return (int64_t)(G[1] + E - 1) / E;
+                                  },
+                                  d->chunk_tiles > 0 ? d->chunk_tiles : 8));
+    const int64_t now = std::max({p->n_k2, p->n_k3, p->n_k4});
+    const int64_t img = (int64_t)p->n_inst * 2 * p->NH *
+                        (layer_words(p->HP, (int)ts) - p->HP * p->HP) * (int64_t)ts;
+    p->ws_fixed = (size_t)((int64_t)off - (now - items) * p->P * (int64_t)ts - img);
+  }
   *out = p;
   return TDX_OK;
 }
+
+// Plans that a 64 MiB workspace held with fixed work items keep to them where
+// the sized ones would need more (the no-allocation entry point).
+extern "C" int tdx_nn_plan_create(const tdx_nn_desc *d, tdx_nn_plan **out) {
+  const int rc = nn_plan_create(d, out, false);
+  if (rc != TDX_OK || d->chunk_tiles > 0) return rc;
+  constexpr size_t kLimit = size_t(64) << 20;
+  if ((*out)->ws_bytes <= kLimit || (*out)->ws_fixed > kLimit) return rc;
+  tdx_nn_plan_destroy(*out);
+  return nn_plan_create(d, out, true);
+}
+
+size_t tdx::nn_workspace_fixed_bytes(const tdx_nn_plan *p) { return p ? p->ws_fixed : 0; }
 
 extern "C" int tdx_nn_profile(tdx_nn_plan *p, int capacity) {
   TDX_REQUIRE(p && capacity >= 0, "bad argument");

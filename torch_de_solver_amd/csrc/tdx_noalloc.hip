@@ -18,7 +18,11 @@
 
 #include <mutex>
 
-constexpr size_t kScratchBytes = size_t(64) << 20;  // 64 MiB per GPU
+// 80 MiB per GPU: plans whose workspace was at most 64 MiB with float32
+// operand images (kLimit) and those images in three bf16 pieces, half as large
+// again (an instance's image is less than its gradient partials)
+constexpr size_t kScratchBytes = size_t(80) << 20;
+constexpr size_t kLimit = size_t(64) << 20;
 
 static __device__ __align__(256) unsigned char scratch[kScratchBytes];
 
@@ -60,7 +64,7 @@ extern "C" int tdx_nn_train_step_noalloc(const tdx_nn_plan *p, void *params, voi
                                          tdx_stream_t stream) {
   TDX_REQUIRE(p && params && exp_avg && exp_avg_sq && step, "null argument");
   const size_t need = tdx_nn_workspace_bytes(p);
-  TDX_REQUIRE(need <= kScratchBytes,
+  TDX_REQUIRE(need <= kScratchBytes && tdx::nn_workspace_fixed_bytes(p) <= kLimit,
               "the plan needs %zu bytes of workspace; the no-allocation entry point holds "
               "%zu (use tdx_nn_train_step with a caller workspace)",
               need, kScratchBytes);
