@@ -1026,6 +1026,18 @@ k_ad_step(ADStepArgs a) {
   ad_step_body<NB, NHM, InterpJets, InterpADResid>(a, reinterpret_cast<float *>(smem_raw));
 }
 
+// k_ad_loss_pass: the fused step's forward half, for evaluations that want
+// the loss alone: no derivatives stored, no gradient partials, the jet maps
+// and the residual program interpreted.  Bound, like the step, by VALU work
+// and waits at ad_step_wgs(NB) wavefronts per SIMD (133 x 91 points, 2-64x3-1:
+// 61 us).
+template <int NB>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ad_step_wgs(NB)))) void
+k_ad_loss_pass(ADStepArgs a) {
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  ad_step_body<NB, 4, InterpJets, InterpADResid, true>(a, reinterpret_cast<float *>(smem_raw));
+}
+
 // Image of the network for k_ad_step (one instance) and the Adam step
 // counter advanced (the step's Adam update reads the new value).
 template <int NB>
@@ -1829,20 +1841,27 @@ int ad_backward(const tdx_ad_plan *p, const T *params, const T *dloss, T *grad, 
 
 }  // namespace
 
-extern "C" int tdx_ad_forward(const tdx_ad_plan *p, const void *params, void *loss, void *resid,
-                              void *ws, tdx_stream_t stream) {
-  TDX_REQUIRE(p && params && loss && ws, "null argument");
-  hipStream_t s = (hipStream_t)stream;
-  if (p->dtype == 0)
-    return ad_forward<float>(p, (const float *)params, (float *)loss, (float *)resid, ws, s);
-  return ad_forward<double>(p, (const double *)params, (double *)loss, (double *)resid, ws, s);
-}
-
 namespace {
 int ad_fused_step(const tdx_ad_plan *p, float *params, float *m, float *v, int64_t *step,
                   const AdamHyper &h, float *loss, void *ws, hipStream_t s,
                   const float *dloss = nullptr, float *grad = nullptr);
 }  // namespace
+
+extern "C" int tdx_ad_forward(const tdx_ad_plan *p, const void *params, void *loss, void *resid,
+                              void *ws, tdx_stream_t stream) {
+  TDX_REQUIRE(p && params && loss && ws, "null argument");
+  hipStream_t s = (hipStream_t)stream;
+  // the loss alone needs no jets in memory: the fused step's forward half
+  // (its adjoint forms the jets again; 133 x 91 Poisson, 2-64x3-1, evaluate
+  // and backward together: 364 -> 293 us); residuals come from the layer
+  // kernels
+  if (p->fused && !resid)
+    return ad_fused_step(p, (float *)const_cast<void *>(params), nullptr, nullptr, nullptr,
+                         AdamHyper{0, 0, 0, 0}, (float *)loss, ws, s, nullptr, nullptr);
+  if (p->dtype == 0)
+    return ad_forward<float>(p, (const float *)params, (float *)loss, (float *)resid, ws, s);
+  return ad_forward<double>(p, (const double *)params, (double *)loss, (double *)resid, ws, s);
+}
 
 extern "C" int tdx_ad_backward(const tdx_ad_plan *p, const void *params, const void *dloss,
                                void *dparams, void *ws, tdx_stream_t stream) {
@@ -1850,7 +1869,8 @@ extern "C" int tdx_ad_backward(const tdx_ad_plan *p, const void *params, const v
   hipStream_t s = (hipStream_t)stream;
   // the fused step's kernel forms the jets again instead of reading the
   // layers' arrays, and is still faster than the layer kernels' adjoint with
-  // its products per layer (133 x 91 Poisson, 2-64x3-1: 350 -> 95 us)
+  // its products per layer (133 x 91 Poisson, 2-64x3-1, evaluate and backward
+  // together: 482 -> 364 us; the kernel itself 199 us)
   if (p->fused)
     return ad_fused_step(p, (float *)const_cast<void *>(params), nullptr, nullptr, nullptr,
                          AdamHyper{0, 0, 0, 0}, nullptr, ws, s, (const float *)dloss,
@@ -1939,6 +1959,15 @@ int ad_step_launch(const tdx_ad_plan *p, const ADStepArgs &a, hipStream_t s) {
 }
 
 template <int NB>
+int ad_loss_launch(const tdx_ad_plan *p, const ADStepArgs &a, hipStream_t s) {
+  raise_lds_limit({(const void *)k_ad_loss_pass<NB>});
+  hipLaunchKernelGGL((k_ad_loss_pass<NB>), dim3((unsigned)p->n_fitems), dim3(256), p->step_lds, s,
+                     a);
+  TDX_TRY_HIP(hipGetLastError());
+  return TDX_OK;
+}
+
+template <int NB>
 int ad_pack_launch(const NNArgs<float> &nn, int64_t *step, hipStream_t s) {
   const int IMG = image_words(16 * NB, nn.NH, nn.d_in, nn.n_out, 4);
   hipLaunchKernelGGL((k_ad_pack<NB>), dim3((unsigned)((IMG + 255) / 256)), dim3(256), 0, s, nn,
@@ -1987,6 +2016,25 @@ int ad_fused_step(const tdx_ad_plan *p, float *params, float *m, float *v, int64
   a.zs = wsp<float>(ws, p->off_zs);
   a.partial = wsp<float>(ws, p->off_fpart);
   a.lp = wsp<float>(ws, p->off_flp);
+  if (!m && !grad) {
+    // loss only
+    switch (p->f_nb) {
+      case 1: rc = ad_loss_launch<1>(p, a, s); break;
+      case 2: rc = ad_loss_launch<2>(p, a, s); break;
+      case 3: rc = ad_loss_launch<3>(p, a, s); break;
+      case 4: rc = ad_loss_launch<4>(p, a, s); break;
+      case 5: rc = ad_loss_launch<5>(p, a, s); break;
+      case 6: rc = ad_loss_launch<6>(p, a, s); break;
+      case 7: rc = ad_loss_launch<7>(p, a, s); break;
+      default: rc = ad_loss_launch<8>(p, a, s); break;
+    }
+    if (rc != TDX_OK) return rc;
+    hipLaunchKernelGGL(k_ad_step_sum, dim3(1), dim3(256), 0, s, (const float *)a.partial,
+                       (const float *)a.lp, p->n_fitems, (int64_t)0, params, m, v,
+                       (const int64_t *)step, h, loss, dloss, grad);
+    TDX_TRY_HIP(hipGetLastError());
+    return TDX_OK;
+  }
   switch (p->f_nb) {
     case 1:
       rc = nn.NH <= 2 ? ad_step_launch<1, 2>(p, a, s) : ad_step_launch<1, 4>(p, a, s);

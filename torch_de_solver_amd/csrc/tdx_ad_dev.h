@@ -408,7 +408,8 @@ __device__ __forceinline__ void ad_entry(const ADStepArgs &a, const int32_t *G, 
 // or straight-line code generated for the plan's jets); RP: the residual
 // program (interpreted, or generated per group).  Launch: 256 threads,
 // ad_step_lds_bytes of dynamic LDS, one workgroup per work item.
-template <int NB, int NHM, typename JP, typename RP>
+// LOSS: the forward jets, the residual program and the loss pair only.
+template <int NB, int NHM, typename JP, typename RP, bool LOSS = false>
 __device__ __forceinline__ void ad_step_body(const ADStepArgs &a, float *smem) {
   constexpr int HP = 16 * NB;
   constexpr int OBW = (NB + 3) / 4;  // output blocks owned per wavefront
@@ -522,7 +523,7 @@ __device__ __forceinline__ void ad_step_body(const ADStepArgs &a, float *smem) {
 #pragma unroll
       for (int i = 0; i < 4; ++i) z[mb][i] = zz[i];
     }
-    if (NH > 0) zstore(0, z);
+    if (!LOSS && NH > 0) zstore(0, z);
     store_rows(zbuf, z);
     wave_sync();
     JP::fwd(zbuf, abuf, r0w, NP, rNP, J, H, tb, lane);
@@ -539,7 +540,7 @@ __device__ __forceinline__ void ad_step_body(const ADStepArgs &a, float *smem) {
       for (int ob = 0; ob < NB; ++ob)
 #pragma unroll
         for (int i = 0; i < 4; ++i) z[ob][i] = acc[ob][i];
-      if (j < NH) zstore(j, z);
+      if (!LOSS && j < NH) zstore(j, z);
       wave_sync();
       store_rows(zbuf, z);
       wave_sync();
@@ -576,6 +577,7 @@ __device__ __forceinline__ void ad_step_body(const ADStepArgs &a, float *smem) {
       RP::run(a, item.x, (int)(t0 + w * EW + lane), n_out, ubuf + (r0w + lane * SJ) * n_out,
               sdb + (r0w + lane * SJ) * n_out, lsum, lnsum);
     wave_sync();
+    if constexpr (LOSS) continue;
     // seeds: dA of the last layer, the output layer's small terms
     {
       float dl[NB][4];
@@ -706,11 +708,11 @@ __device__ __forceinline__ void ad_step_body(const ADStepArgs &a, float *smem) {
 
   // each wavefront writes the blocks it owns; the output bias and the loss
   // are the only sums over wavefronts (fixed order)
-  float *out = a.partial + (int64_t)blockIdx.x * P;
+  float *out = LOSS ? nullptr : a.partial + (int64_t)blockIdx.x * P;
 #pragma unroll
   for (int u = 0; u < OBW; ++u) {
     const int ob = w + 4 * u;
-    if (ob < NB) {
+    if (!LOSS && ob < NB) {
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const int of = 16 * ob + crow<float>(q, i);
@@ -752,7 +754,7 @@ __device__ __forceinline__ void ad_step_body(const ADStepArgs &a, float *smem) {
     red[17 + 2 * w] = lnsum;
   }
   __syncthreads();
-  if ((int)threadIdx.x < n_out) {
+  if (!LOSS && (int)threadIdx.x < n_out) {
     const int o = threadIdx.x;
     out[L.obL() + o] = ((red[o] + red[4 + o]) + red[8 + o]) + red[12 + o];
   }
