@@ -528,9 +528,12 @@ __device__ __forceinline__ void ad_step_body(const ADStepArgs &a, float *smem) {
     wave_sync();
     JP::fwd(zbuf, abuf, r0w, NP, rNP, J, H, tb, lane);
     wave_sync();
-#pragma unroll
-    for (int j = 1; j <= NHM; ++j) {
-      if (j > NH) break;
+    // (not unrolled, as the adjoint's loop below: a tile runs its code once,
+    // and four layers' copies are more than the instruction cache holds;
+    // rolled, half the accumulators' spills go too.  201 x 201 Poisson,
+    // 2-100x5-1: 1018 -> 927 us a step; 32 x 40, 2-64x5-1: 123 -> 116)
+#pragma unroll 1
+    for (int j = 1; j <= NH; ++j) {
       v4 acc[NB];
 #pragma unroll
       for (int ob = 0; ob < NB; ++ob)
@@ -622,10 +625,8 @@ __device__ __forceinline__ void ad_step_body(const ADStepArgs &a, float *smem) {
     // from here on abuf holds dZ of the current layer (all rows once a
     // barrier has passed), dbuf dA and then A of the layer below
     JP::adj(zbuf, dbuf, abuf, r0w, NP, rNP, J, H, tb, lane);
-#pragma unroll
-    for (int j = NHM; j >= 1; --j) {
-      if (j > NH) continue;
-      const int jj = j - 1;
+#pragma unroll 1
+    for (int j = NH; j >= 1; --j) {
       // A of layer j - 1 again from its pre-activation jets
       {
         float zp[NB][4];
@@ -635,9 +636,12 @@ __device__ __forceinline__ void ad_step_body(const ADStepArgs &a, float *smem) {
       wave_sync();
       JP::fwd(zbuf, dbuf, r0w, NP, rNP, J, H, tb, lane);
       __syncthreads();
-      // owned blocks of dW_jj over the 64 rows in two steps of 32, as in the
-      // block-owning kernel; the bias over value rows
-      {
+      // owned blocks of dW_{j-1} over the 64 rows in two steps of 32, as in the
+      // block-owning kernel; the bias over value rows (a copy of the code per
+      // layer: its accumulators are registers)
+#pragma unroll
+      for (int jj = 0; jj < NHM; ++jj) {
+        if (jj != j - 1) continue;
         Bf3 ds[OBW][2];
 #pragma unroll
         for (int u = 0; u < OBW; ++u) {
@@ -670,11 +674,11 @@ __device__ __forceinline__ void ad_step_body(const ADStepArgs &a, float *smem) {
             if (w + 4 * u < NB) dwacc[jj][u][ib] = mma3_pair(ds[u], as, dwacc[jj][u][ib]);
         }
       }
-      // dA of layer j - 1 = W_jj^T dZ_j for this wavefront's rows
+      // dA of layer j - 1 = W_{j-1}^T dZ_j for this wavefront's rows
       v4 c[NB];
 #pragma unroll
       for (int ib = 0; ib < NB; ++ib) c[ib] = v4{0, 0, 0, 0};
-      mma_layer_fm<NB>(net.Wb + jj * net.LI, lane, abuf, trow, c);
+      mma_layer_fm<NB>(net.Wb + (j - 1) * net.LI, lane, abuf, trow, c);
       __syncthreads();
       {
         float dv[NB][4];
