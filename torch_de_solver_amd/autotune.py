@@ -25,7 +25,9 @@ from typing import Dict, List, Optional, Sequence, Tuple
 
 import torch
 
-NN_CHUNK_CANDIDATES = (1, 2, 4, 8, 16, 32, 64, 128, 256)
+# 0: the plan's own default, which fits the items to the CUs (2-100x4-1 on
+# 256 x 100 points: 0.51 ms a step, the best power of two 0.55)
+NN_CHUNK_CANDIDATES = (0, 1, 2, 4, 8, 16, 32, 64, 128, 256)
 MAT_ROW_CANDIDATES = (4, 8, 12, 16, 20, 28, 36, 44, 60)
 
 _lock = threading.Lock()
