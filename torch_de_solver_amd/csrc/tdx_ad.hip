@@ -1030,7 +1030,7 @@ k_ad_step(ADStepArgs a) {
 // the loss alone: no derivatives stored, no gradient partials, the jet maps
 // and the residual program interpreted.  Bound, like the step, by VALU work
 // and waits at ad_step_wgs(NB) wavefronts per SIMD (133 x 91 points, 2-64x3-1:
-// 61 us).
+// 60 us).
 template <int NB>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ad_step_wgs(NB)))) void
 k_ad_loss_pass(ADStepArgs a) {
@@ -1870,7 +1870,7 @@ extern "C" int tdx_ad_backward(const tdx_ad_plan *p, const void *params, const v
   // the fused step's kernel forms the jets again instead of reading the
   // layers' arrays, and is still faster than the layer kernels' adjoint with
   // its products per layer (133 x 91 Poisson, 2-64x3-1, evaluate and backward
-  // together: 482 -> 364 us; the kernel itself 199 us)
+  // together: 482 -> 364 us; the kernel itself 195 us)
   if (p->fused)
     return ad_fused_step(p, (float *)const_cast<void *>(params), nullptr, nullptr, nullptr,
                          AdamHyper{0, 0, 0, 0}, nullptr, ws, s, (const float *)dloss,
