@@ -13,11 +13,14 @@ two knobs decide how work maps onto the GPU:
 
 ``tune_nn`` / ``tune_mat`` build one plan per candidate, time the dominant
 launches with HIP events after a warm-up, keep the fastest, and cache the
-choice in a JSON file keyed by the plan's shape (``TDX_TUNE_CACHE``, default
-``~/.cache/torch_de_solver_amd/tuning.json``; ``TDX_TUNE_CACHE=off`` keeps
-nothing), so a later plan of the same shape skips the search.
+choice in a JSON file keyed by the plan's shape and the library's build
+(``TDX_TUNE_CACHE``, default ``~/.cache/torch_de_solver_amd/tuning.json``;
+``TDX_TUNE_CACHE=off`` keeps nothing), so a later plan of the same shape skips
+the search.  A choice timed with another build's kernels does not count.
 """
 
+import functools
+import hashlib
 import json
 import os
 import threading
@@ -25,12 +28,28 @@ from typing import Dict, List, Optional, Sequence, Tuple
 
 import torch
 
+from . import native
+
 # 0: the plan's own default, which fits the items to the CUs (2-100x4-1 on
 # 256 x 100 points: 0.51 ms a step, the best power of two 0.55)
 NN_CHUNK_CANDIDATES = (0, 1, 2, 4, 8, 16, 32, 64, 128, 256)
 MAT_ROW_CANDIDATES = (4, 8, 12, 16, 20, 28, 36, 44, 60)
 
 _lock = threading.Lock()
+
+
+@functools.lru_cache(maxsize=None)
+def _digest(path: str) -> str:
+    h = hashlib.sha1()
+    with open(path, 'rb') as f:
+        for block in iter(lambda: f.read(1 << 20), b''):
+            h.update(block)
+    return h.hexdigest()[:16]
+
+
+def _build_key() -> str:
+    """Key part that names the native library's build (its contents)."""
+    return '|lib' + _digest(native.LIB_PATH)
 
 
 def _cache_path() -> Optional[str]:
@@ -102,7 +121,8 @@ def tune_nn(problems, arch, device, params: torch.Tensor,
     copy of ``params``: the fused kernel where the plan has it, else the
     separate forward and adjoint kernels).  Returns (chunk_tiles, report)."""
     from .nn_engine import NNEngine
-    key = nn_key(problems, arch, params.dtype) + f"|tr{tile_rows}|ps{persistent}|step"
+    key = nn_key(problems, arch, params.dtype) + f"|tr{tile_rows}|ps{persistent}|step" + \
+        _build_key()
     if use_cache:
         hit = _load().get(key)
         if hit and hit.get('chunk_tiles') in candidates:
@@ -146,7 +166,7 @@ def tune_mat(prob, device, u: torch.Tensor, exact_div: bool = True,
     from .mat_engine import MatEngine
     if len(prob.shape) < 2 or int(prob.shape[0]) == 1:
         return 0, {'tile_rows': 0, 'ms': {}, 'cached': False}
-    key = mat_key(prob, exact_div)
+    key = mat_key(prob, exact_div) + _build_key()
     if use_cache:
         hit = _load().get(key)
         if hit and hit.get('tile_rows') in candidates:
