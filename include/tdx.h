@@ -222,10 +222,11 @@ int tdx_nn_train_step(const tdx_nn_plan *plan, void *params, void *exp_avg,
 /* No counterpart in the reference: for callers that cannot allocate device
  * memory (code under HIP graph capture, tight serving loops, harnesses that
  * forbid hipMalloc).  tdx_nn_train_step with the workspace taken from a
- * file-scope device array of tdx_noalloc_scratch_bytes() bytes (80 MiB) per
+ * file-scope device array of tdx_noalloc_scratch_bytes() bytes (128 MiB) per
  * GPU instead of a caller buffer; plans whose workspace, with work items of
- * fixed size and float32 network images, exceeds 64 MiB
- * are refused with TDX_EINVAL before anything is launched.  Allocates
+ * fixed size (256 tiles in the wavefront-private adjoint, 8 in the
+ * block-owning one, 4 blocks in the fused step) and float32 network images,
+ * exceeds 64 MiB are refused with TDX_EINVAL before anything is launched.  Allocates
  * nothing (the array's device address is looked up once per device).  All
  * calls on one GPU share that GPU's array: calls that overlap on one GPU
  * (concurrent streams or threads) race; calls in stream order do not. */

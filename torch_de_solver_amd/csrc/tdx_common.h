@@ -16,9 +16,14 @@
 
 namespace tdx {
 
-// A plan's workspace with fixed work items and float32 operand images.
+// The no-allocation entry point takes the plans whose workspace, with work
+// items of fixed size and float32 images, is at most kNoAllocLimit.  Its array
+// holds kNoAllocBytes: the images in bf16 pieces are at most twice the float32
+// ones (layer_words: 33 to 48 units), whatever share of a workspace they are.
+constexpr size_t kNoAllocLimit = size_t(64) << 20;
+constexpr size_t kNoAllocBytes = 2 * kNoAllocLimit;
+// A plan's workspace with fixed work items and float32 images.
 size_t nn_workspace_fixed_bytes(const tdx_nn_plan *p);
-
 
 void set_error(const char *fmt, ...);
 void clear_error();

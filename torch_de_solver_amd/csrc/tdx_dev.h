@@ -33,6 +33,7 @@ __device__ __forceinline__ d4_t mma16(double a, double b, d4_t c) {
 // of sums over K = 32: 3.6e-8 (float32 MFMA 1.03e-7), K = 128: 6e-8 (2.0e-7).
 typedef __bf16 bf8_t __attribute__((ext_vector_type(8)));
 typedef unsigned u4_t __attribute__((ext_vector_type(4)));
+typedef unsigned u2_t __attribute__((ext_vector_type(2)));
 typedef __bf16 bf2_t __attribute__((ext_vector_type(2)));
 typedef float f16_t __attribute__((ext_vector_type(16)));
 

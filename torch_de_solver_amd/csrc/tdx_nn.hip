@@ -1266,8 +1266,18 @@ using namespace tdx;
 struct tdx_nn_plan;
 static size_t wave_private_lds(const tdx_nn_plan *p, const tdx_nn_desc *d);
 
-struct tdx_nn_plan {
-  size_t ws_fixed = 0;  // workspace with fixed work items (tdx_nn_plan_create)
+// Workspace layout (byte offsets) and size.
+struct NNWorkspace {
+  size_t off_packed = 0, off_seeds = 0, off_lp = 0, off_partial = 0, off_one = 0, off_red = 0;
+  // causal loss: residuals, weights and w * res; weak form: residuals, the
+  // runs' sums and the points' seed multipliers
+  size_t off_resid = 0, off_cw = 0, off_cwr = 0, off_wR = 0, off_wm = 0;
+  size_t ws_bytes = 0;
+};
+
+struct tdx_nn_plan : NNWorkspace {
+  // bytes of the workspace with work items of fixed size and float32 images
+  size_t ws_fixed = 0;
   int dtype, d_in, n_out, H, n_layers, NH, NB, HP, P, n_inst;
   int n_groups;
   int max_slots;      // largest slot count of a group
@@ -1298,7 +1308,6 @@ struct tdx_nn_plan {
   // their list (instance i: items s * n_inst + i) and workspace offset
   int red_slices = 1;
   DevTable ik5p, ik5i;
-  size_t off_red = 0;
   // training step of wide float networks: the block-owning backward forms
   // its own seeds (FS work items: tiles of whole entries)
   int k2_fs = 0;
@@ -1311,20 +1320,15 @@ struct tdx_nn_plan {
   int acc_lds;
   size_t k1_lds, k2_lds;
   DevTable groups, ints, reals, data, k1_items, k2_items, ik1p, ik1i, ik2p, ik2i;
-  // workspace layout (byte offsets)
-  size_t off_packed, off_seeds, off_lp, off_partial, off_one, ws_bytes;
   // causal loss: tolerance, slices, points of group 0 (N = nt * K), its
-  // equations and slots; workspace for residuals, weights and w * res
+  // equations and slots
   int causal = 0;
   double causal_tol = 0;
   int c_nt = 0, c_K = 0, c_N = 0, c_neq = 0, c_slots = 0;
-  size_t off_resid = 0, off_cw = 0, off_cwr = 0;
   // weak form: levels (0 none), runs, group 0's points and equations, table
-  // offsets (data: c_i, x_g, lambda_eq; ints: run starts); workspace for
-  // the runs' sums and the points' seed multipliers
+  // offsets (data: c_i, x_g, lambda_eq; ints: run starts)
   int weak = 0, w_G = 0, w_N = 0, w_neq = 0;
   int64_t w_d = 0, w_i = 0;
-  size_t off_wR = 0, off_wm = 0;
   // optional launch timing: event pairs per kernel kind
   int prof_cap = 0;
   int prof_n[TDX_NN_KERNEL_KINDS] = {0};
@@ -2019,6 +2023,40 @@ bool fused_programs(const tdx_nn_desc *d, std::vector<FusedProg> *out) {
 
 }  // namespace
 
+// Workspace of a plan (its shapes and loss set) with images of img words an
+// instance, n_k4 seed-forming and n_items largest list of gradient work items
+// and a gradient sum of `slices` slices an instance.
+static NNWorkspace nn_layout(const tdx_nn_plan &p, int img, int64_t n_k4, int64_t n_items,
+                             int slices) {
+  const size_t ts = p.dtype == 0 ? 4 : 8;
+  NNWorkspace w;
+  size_t off = 0;
+  auto take = [&](size_t words) {
+    const size_t at = off;
+    off = align_up(off + words * ts, 256);
+    return at;
+  };
+  w.off_packed = take((size_t)p.n_inst * img);
+  w.off_seeds = take((size_t)p.n_rows * p.n_out);
+  w.off_lp = take((size_t)std::max<int64_t>(p.n_k1, n_k4) * 2);
+  w.off_partial = take((size_t)n_items * p.P);
+  w.off_one = take(1);
+  w.off_red = off;
+  if (slices > 1) take((size_t)slices * p.n_inst * p.P);
+  if (p.causal) {
+    w.off_resid = take((size_t)std::max<int64_t>(p.n_resid, 1));
+    w.off_cw = take((size_t)p.c_N);
+    w.off_cwr = take((size_t)p.c_N);
+  }
+  if (p.weak) {
+    w.off_resid = take((size_t)std::max<int64_t>(p.n_resid, 1));
+    w.off_wR = take((size_t)p.w_G * p.w_neq);
+    w.off_wm = take((size_t)p.w_N * p.w_neq);
+  }
+  w.ws_bytes = off;
+  return w;
+}
+
 // fixed: work items of fixed numbers of tiles (the workspace's gradient
 // partials grow with the items).
 static int nn_plan_create(const tdx_nn_desc *d, tdx_nn_plan **out, bool fixed) {
@@ -2332,15 +2370,18 @@ static int nn_plan_create(const tdx_nn_desc *d, tdx_nn_plan **out, bool fixed) {
   // at least 8 work items per slice (an instance of few items is summed in
   // one pass: a second launch would cost more than it saves)
   std::vector<int32_t> ik5p, ik5i;
-  {
+  auto slices_of = [&](int64_t max_items) {
     const int64_t np = (int64_t)d->n_inst * p->P;
+    const int sl = (int)std::min<int64_t>({64, ((1 << 20) + np - 1) / np, max_items / 8});
+    return np < (1 << 19) && sl >= 2 ? sl : 1;
+  };
+  {
     int max_items = 0;
     for (int i = 0; i < d->n_inst; ++i)
       max_items = std::max({max_items, (int)inst_k2[i].size(), (int)inst_k3[i].size(),
                             (int)inst_k4_size[i]});
-    const int sl = (int)std::min<int64_t>({64, ((1 << 20) + np - 1) / np, max_items / 8});
-    if (np < (1 << 19) && sl >= 2) {
-      p->red_slices = sl;
+    p->red_slices = slices_of(max_items);
+    if (p->red_slices > 1) {
       for (int i = 0; i <= d->n_inst; ++i) ik5p.push_back(i * p->red_slices);
       for (int i = 0; i < d->n_inst; ++i)
         for (int sl = 0; sl < p->red_slices; ++sl) ik5i.push_back(sl * d->n_inst + i);
@@ -2412,19 +2453,6 @@ static int nn_plan_create(const tdx_nn_desc *d, tdx_nn_plan **out, bool fixed) {
     tdx_nn_plan_destroy(p);
     return r2;
   }
-  size_t off = 0;
-  p->off_packed = off;
-  off = align_up(off + (size_t)p->n_inst * image_words(p->HP, p->NH, d->d_in, d->n_out, (int)ts) * ts, 256);
-  p->off_seeds = off;
-  off = align_up(off + (size_t)n_rows * p->n_out * ts, 256);
-  p->off_lp = off;
-  off = align_up(off + (size_t)std::max(p->n_k1, p->n_k4) * 2 * ts, 256);
-  p->off_partial = off;
-  off = align_up(off + (size_t)std::max({p->n_k2, p->n_k3, p->n_k4}) * p->P * ts, 256);
-  p->off_one = off;
-  off = align_up(off + ts, 256);
-  p->off_red = off;
-  if (p->red_slices > 1) off = align_up(off + (size_t)p->red_slices * p->n_inst * p->P * ts, 256);
   if (d->causal_tol != 0.0) {
     const int32_t *G0 = d->groups;
     p->causal = 1;
@@ -2434,12 +2462,6 @@ static int nn_plan_create(const tdx_nn_desc *d, tdx_nn_plan **out, bool fixed) {
     p->c_neq = G0[5];
     p->c_nt = d->causal_nt;
     p->c_K = p->c_N / std::max(1, p->c_nt);
-    p->off_resid = off;
-    off = align_up(off + (size_t)std::max<int64_t>(d->n_resid, 1) * ts, 256);
-    p->off_cw = off;
-    off = align_up(off + (size_t)p->c_N * ts, 256);
-    p->off_cwr = off;
-    off = align_up(off + (size_t)p->c_N * ts, 256);
   }
   if (d->weak_levels != 0) {
     const int32_t *G0 = d->groups;
@@ -2450,56 +2472,41 @@ static int nn_plan_create(const tdx_nn_desc *d, tdx_nn_plan **out, bool fixed) {
     p->c_slots = G0[2];
     p->w_d = d->weak_d;
     p->w_i = d->weak_i;
-    p->off_resid = off;
-    off = align_up(off + (size_t)std::max<int64_t>(d->n_resid, 1) * ts, 256);
-    p->off_wR = off;
-    off = align_up(off + (size_t)p->w_G * p->w_neq * ts, 256);
-    p->off_wm = off;
-    off = align_up(off + (size_t)p->w_N * p->w_neq * ts, 256);
   }
-  p->ws_bytes = off;
+  const int img = image_words(p->HP, p->NH, d->d_in, d->n_out, (int)ts);
+  *static_cast<NNWorkspace *>(p) = nn_layout(*p, img, p->n_k4, std::max({p->n_k2, p->n_k3, p->n_k4}),
+                                             p->red_slices);
   {
-    // the workspace with fixed work items and float32 operand images, which
-    // the no-allocation entry point's limit is stated in
-    auto items_of = [&](auto tiles_of, int c) {
-      int64_t n = 0;
-      for (int g = 0; g < d->n_groups; ++g)
-        n += (tiles_of(d->groups + (int64_t)g * TDX_GROUP_INTS) + c - 1) / c;
-      return n;
-    };
-    const int c2 = d->chunk_tiles > 0    ? d->chunk_tiles
-                   : p->k2_wave_private ? 256
-                   : p->k2_block        ? 8
-                   : p->acc_lds         ? 16
-                                        : 4;
-    int64_t items = items_of(
-        [&](const int32_t *G) { return ((int64_t)G[1] * G[2] + TR - 1) / TR; }, c2);
-    if (p->fused)
-      items = std::max(items, items_of([](const int32_t *G) { return (int64_t)(G[1] + 63) / 64; },
-                                       d->chunk_tiles > 0 ? d->chunk_tiles : 4));
-    if (p->k2_fs)
-      items = std::max(items, items_of(
-                                  [](const int32_t *G) {
-                                    const int E = 64 / G[2];
-                                    return (int64_t)(G[1] + E - 1) / E;
-                                  },
-                                  d->chunk_tiles > 0 ? d->chunk_tiles : 8));
-    const int64_t now = std::max({p->n_k2, p->n_k3, p->n_k4});
-    const int64_t img = (int64_t)p->n_inst * 2 * p->NH *
-                        (layer_words(p->HP, (int)ts) - p->HP * p->HP) * (int64_t)ts;
-    p->ws_fixed = (size_t)((int64_t)off - (now - items) * p->P * (int64_t)ts - img);
+    // the same with work items of fixed size and float32 images, which the
+    // no-allocation entry point's limit is stated in
+    std::vector<int64_t> i2(d->n_inst, 0), i3(d->n_inst, 0), i4(d->n_inst, 0);
+    auto chunk_of = [&](int c) { return d->chunk_tiles > 0 ? d->chunk_tiles : c; };
+    auto items_of = [](int64_t tiles, int c) { return (tiles + c - 1) / c; };
+    const int c2 = chunk_of(p->k2_wave_private ? 256 : p->k2_block ? 8 : p->acc_lds ? 16 : 4);
+    int64_t n2 = 0, n3 = 0, n4 = 0, most = 0;
+    for (int g = 0; g < d->n_groups; ++g) {
+      const int32_t *G = d->groups + (int64_t)g * TDX_GROUP_INTS;
+      i2[G[0]] += items_of(((int64_t)G[1] * G[2] + TR - 1) / TR, c2);
+      if (p->fused) i3[G[0]] += items_of(((int64_t)G[1] + 63) / 64, chunk_of(4));
+      if (p->k2_fs) i4[G[0]] += items_of(((int64_t)G[1] + 64 / G[2] - 1) / (64 / G[2]), chunk_of(8));
+    }
+    for (int i = 0; i < d->n_inst; ++i) {
+      n2 += i2[i], n3 += i3[i], n4 += i4[i];
+      most = std::max({most, i2[i], i3[i], i4[i]});
+    }
+    const int img32 = img - 2 * p->NH * (layer_words(p->HP, (int)ts) - p->HP * p->HP);
+    p->ws_fixed = nn_layout(*p, img32, n4, std::max({n2, n3, n4}), slices_of(most)).ws_bytes;
   }
   *out = p;
   return TDX_OK;
 }
 
-// Plans that a 64 MiB workspace held with fixed work items keep to them where
-// the sized ones would need more (the no-allocation entry point).
+// Plans that the no-allocation entry point takes keep to fixed work items
+// where the sized ones would need more than its array.
 extern "C" int tdx_nn_plan_create(const tdx_nn_desc *d, tdx_nn_plan **out) {
   const int rc = nn_plan_create(d, out, false);
   if (rc != TDX_OK || d->chunk_tiles > 0) return rc;
-  constexpr size_t kLimit = size_t(64) << 20;
-  if ((*out)->ws_bytes <= kLimit || (*out)->ws_fixed > kLimit) return rc;
+  if ((*out)->ws_bytes <= kNoAllocBytes || (*out)->ws_fixed > kNoAllocLimit) return rc;
   tdx_nn_plan_destroy(*out);
   return nn_plan_create(d, out, true);
 }

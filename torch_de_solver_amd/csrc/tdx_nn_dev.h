@@ -89,7 +89,10 @@ struct Layout {
 // e % 4 of block mb = 2 ks + e / 4 (zero beyond the network):
 //   Wf[j][ob][ks][p][lane][t] = W_j[16*ob + lane%16][feature of e]
 //   Wb[j][ib][ks][p][lane][t] = W_j[feature of e][16*ib + lane%16]
-// so a lane reads one piece of a 32-deep operand with one 128-bit load.
+// so a lane reads one piece of a 32-deep operand with one 128-bit load.  At an
+// odd NB the last step's upper half is stored zeros; NB = 1 stores the lower
+// half alone (t = 0, 1; 64-bit loads).  An image is so 1.5 times the float32
+// matrix at even NB and NB = 1, at most twice at the others.
 // double: operands of 16x16x4 products, the four values of k-steps i = 0..3
 // of block (xb, mb) adjacent:
 //   Wf[j][ob][mb][lane][i] = W_j[16*ob + lane%16][16*mb + crow(lane/16, i)]
@@ -105,7 +108,7 @@ __host__ __device__ inline int small_words(int HP, int NH, int d_in, int n_out) 
 }
 // Words of one layer's operand image (ts: bytes of the working type).
 __host__ __device__ constexpr int layer_words(int HP, int ts) {
-  return ts == 4 ? (HP / 16) * ((HP + 16) / 32) * 768 : HP * HP;
+  return ts == 8 ? HP * HP : HP == 16 ? 384 : (HP / 16) * ((HP + 16) / 32) * 768;
 }
 __host__ __device__ inline int image_words(int HP, int NH, int d_in, int n_out, int ts) {
   return 2 * NH * layer_words(HP, ts) + small_words(HP, NH, d_in, n_out);
@@ -139,9 +142,9 @@ __device__ __forceinline__ T image_value(const NNArgs<T> &a, const T *W, int off
       const int j = off / img;
       int r = off - j * img;
       if constexpr (sizeof(T) == 4) {
-        constexpr int KS = (NB + 1) / 2;
-        const int t = r & 3, lane = (r >> 2) & 63;
-        r >>= 8;
+        constexpr int KS = (NB + 1) / 2, TB = NB == 1 ? 1 : 2;  // 2^TB words a lane
+        const int t = r & ((1 << TB) - 1), lane = (r >> TB) & 63;
+        r >>= TB + 6;
         const int p = r % 3, ks = (r / 3) % KS, xb = r / (3 * KS);
         T w2[2];
 #pragma unroll
@@ -308,6 +311,10 @@ __device__ __forceinline__ void mma_split(const float *img, int lane,
       d.h = __builtin_amdgcn_raw_buffer_load_b128(rs, o, so, 0);
       d.m = __builtin_amdgcn_raw_buffer_load_b128(rs, o, so + 1024, 0);
       d.l = __builtin_amdgcn_raw_buffer_load_b128(rs, o, so + 2048, 0);
+    } else if constexpr (NB == 1) {
+      const u2_t *p = reinterpret_cast<const u2_t *>(img) + lane;
+      const u2_t h = p[0], m = p[64], l = p[128];
+      d = Bf3{u4_t{h[0], h[1], 0, 0}, u4_t{m[0], m[1], 0, 0}, u4_t{l[0], l[1], 0, 0}};
     } else {
       const u4_t *p = reinterpret_cast<const u4_t *>(img) + lane + t * 192;
       d.h = p[0], d.m = p[64], d.l = p[128];

@@ -18,13 +18,7 @@
 
 #include <mutex>
 
-// 80 MiB per GPU: plans whose workspace was at most 64 MiB with float32
-// operand images (kLimit) and those images in three bf16 pieces, half as large
-// again (an instance's image is less than its gradient partials)
-constexpr size_t kScratchBytes = size_t(80) << 20;
-constexpr size_t kLimit = size_t(64) << 20;
-
-static __device__ __align__(256) unsigned char scratch[kScratchBytes];
+static __device__ __align__(256) unsigned char scratch[tdx::kNoAllocBytes];
 
 namespace {
 
@@ -56,18 +50,23 @@ void *scratch_address() {
 
 }  // namespace
 
-extern "C" size_t tdx_noalloc_scratch_bytes(void) { return kScratchBytes; }
+extern "C" size_t tdx_noalloc_scratch_bytes(void) { return tdx::kNoAllocBytes; }
 
 extern "C" int tdx_nn_train_step_noalloc(const tdx_nn_plan *p, void *params, void *exp_avg,
                                          void *exp_avg_sq, int64_t *step, double lr,
                                          double beta1, double beta2, double eps, void *loss,
                                          tdx_stream_t stream) {
   TDX_REQUIRE(p && params && exp_avg && exp_avg_sq && step, "null argument");
-  const size_t need = tdx_nn_workspace_bytes(p);
-  TDX_REQUIRE(need <= kScratchBytes && tdx::nn_workspace_fixed_bytes(p) <= kLimit,
+  const size_t fixed = tdx::nn_workspace_fixed_bytes(p), need = tdx_nn_workspace_bytes(p);
+  TDX_REQUIRE(fixed <= tdx::kNoAllocLimit,
+              "the plan's workspace, with fixed work items and float32 images, takes %zu bytes; "
+              "the no-allocation entry point serves up to %zu (use tdx_nn_train_step with a "
+              "caller workspace)",
+              fixed, tdx::kNoAllocLimit);
+  TDX_REQUIRE(need <= tdx::kNoAllocBytes,
               "the plan needs %zu bytes of workspace; the no-allocation entry point holds "
               "%zu (use tdx_nn_train_step with a caller workspace)",
-              need, kScratchBytes);
+              need, tdx::kNoAllocBytes);
   void *ws = scratch_address();
   if (!ws) return TDX_ELAUNCH;
   return tdx_nn_train_step(p, params, exp_avg, exp_avg_sq, step, lr, beta1, beta2, eps, loss,
