@@ -226,7 +226,9 @@ int tdx_nn_train_step(const tdx_nn_plan *plan, void *params, void *exp_avg,
  * GPU instead of a caller buffer; plans whose workspace, with work items of
  * fixed size (256 tiles in the wavefront-private adjoint, 8 in the
  * block-owning one, 4 blocks in the fused step) and float32 network images,
- * exceeds 64 MiB are refused with TDX_EINVAL before anything is launched.  Allocates
+ * exceeds 64 MiB are refused with TDX_EINVAL before anything is launched.  A
+ * plan whose own work items need more than the array runs fixed ones here (the
+ * gradient's sums in another order than tdx_nn_train_step's).  Allocates
  * nothing (the array's device address is looked up once per device).  All
  * calls on one GPU share that GPU's array: calls that overlap on one GPU
  * (concurrent streams or threads) race; calls in stream order do not. */

@@ -78,3 +78,37 @@ def test_noalloc_takes_sweeps_up_to_the_limit(width, hidden):
     assert b'serves up to 67108864' in native.lib().tdx_last_error()
     torch.cuda.synchronize()
     assert int(st[3]) == 0
+
+
+def test_plans_keep_their_work_items_beside_the_noalloc_ones():
+    """float64, 2-128x6-1: the work items that fill the device need more than
+    the no-allocation array, four tiles an item do not.  A caller with a
+    workspace gets the former; the no-allocation call runs the latter, the bits
+    of a plan that asks for them."""
+    lib = native.lib()
+    d, eq, b, _ = problems.burgers_nn(api, nx=22, nt=24, dtype='float64')
+    prob = compile_nn(d.build('NN'), eq.equation_lst, b.build(d.variable_dict), 1,
+                      lambda_operator=1, lambda_bound=10)
+    arch = _arch(128, 6)
+    eng, four = NNEngine([prob], arch, DEV), NNEngine([prob], arch, DEV, chunk_tiles=4)
+    cap = int(lib.tdx_noalloc_scratch_bytes())
+    assert int(lib.tdx_nn_workspace_bytes(eng._plan)) > cap
+    assert int(lib.tdx_nn_workspace_bytes(four._plan)) <= LIMIT
+    a, b, c = ([t if t.dtype == torch.int64 else t.double() for t in _state(eng)]
+               for _ in range(3))
+    eng.profile(8)
+    for _ in range(2):
+        native.check(_noalloc(eng, a))
+        four.train_step(b[0], b[1], b[2], b[3], 1e-3, 0.9, 0.999, 1e-8, b[4])
+        eng.train_step(c[0], c[1], c[2], c[3], 1e-3, 0.9, 0.999, 1e-8, c[4])
+    torch.cuda.synchronize()
+    # launch timing counts both entry points' launches
+    assert {n for _, n in eng.profile_read().values()} == {4}
+    eng.profile(0)
+    for x, y in zip(a, b):
+        assert torch.equal(x, y)
+    # the same sums in another order: each of P gradients a few 1e-15 apart,
+    # Adam's first steps of 1e-3 divide by sqrt(v) + 1e-8
+    assert torch.equal(a[4], c[4]) or torch.allclose(a[4], c[4], rtol=1e-9)
+    assert float((a[0] - c[0]).abs().max()) <= 2 * 2 * 1e-3
+    assert float(((a[1] - c[1]).norm() / c[1].norm())) <= 1e-9

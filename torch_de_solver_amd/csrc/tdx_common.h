@@ -24,6 +24,9 @@ constexpr size_t kNoAllocLimit = size_t(64) << 20;
 constexpr size_t kNoAllocBytes = 2 * kNoAllocLimit;
 // A plan's workspace with fixed work items and float32 images.
 size_t nn_workspace_fixed_bytes(const tdx_nn_plan *p);
+// The plan that the no-allocation entry point runs: p, or p's problem with
+// fixed work items where p's own need more than kNoAllocBytes.
+const tdx_nn_plan *nn_noalloc_plan(const tdx_nn_plan *p);
 
 void set_error(const char *fmt, ...);
 void clear_error();
@@ -45,10 +48,17 @@ void clear_error();
     }                                                                        \
   } while (0)
 
-// Device copy of an immutable host table, owned by a plan.
+// Device copy of an immutable host table, owned by a plan (or borrowed from
+// one that outlives its reader).
 struct DevTable {
   void *ptr = nullptr;
   size_t bytes = 0;
+  bool borrowed = false;
+  void borrow(const DevTable &o) {
+    ptr = o.ptr;
+    bytes = o.bytes;
+    borrowed = true;
+  }
   int upload(const void *host, size_t n) {
     bytes = n;
     if (n == 0) return TDX_OK;
@@ -63,7 +73,7 @@ struct DevTable {
     return TDX_OK;
   }
   void release() {
-    if (ptr) (void)hipFree(ptr);
+    if (ptr && !borrowed) (void)hipFree(ptr);
     ptr = nullptr;
   }
 };

@@ -1278,6 +1278,11 @@ struct NNWorkspace {
 struct tdx_nn_plan : NNWorkspace {
   // bytes of the workspace with work items of fixed size and float32 images
   size_t ws_fixed = 0;
+  // the same problem with fixed work items, for the no-allocation entry point
+  // (null: this plan fits its array); that plan's tables and launch timing are
+  // this one's
+  tdx_nn_plan *fixed_items = nullptr;
+  const tdx_nn_plan *fixed_of = nullptr;
   int dtype, d_in, n_out, H, n_layers, NH, NB, HP, P, n_inst;
   int n_groups;
   int max_slots;      // largest slot count of a group
@@ -1351,7 +1356,8 @@ struct ProfScope {
   int kind;
   hipStream_t s;
   hipEvent_t stop = nullptr;
-  ProfScope(const tdx_nn_plan *pc, int k, hipStream_t st) : p(const_cast<tdx_nn_plan *>(pc)), kind(k), s(st) {
+  ProfScope(const tdx_nn_plan *pc, int k, hipStream_t st)
+      : p(const_cast<tdx_nn_plan *>(pc->fixed_of ? pc->fixed_of : pc)), kind(k), s(st) {
     if (p->prof_cap > 0 && p->prof_n[kind] < p->prof_cap) {
       const int i = p->prof_n[kind]++;
       (void)hipEventRecord(p->prof_ev[kind][2 * i], s);
@@ -2057,9 +2063,10 @@ static NNWorkspace nn_layout(const tdx_nn_plan &p, int img, int64_t n_k4, int64_
   return w;
 }
 
-// fixed: work items of fixed numbers of tiles (the workspace's gradient
-// partials grow with the items).
-static int nn_plan_create(const tdx_nn_desc *d, tdx_nn_plan **out, bool fixed) {
+// of: not null for the plan with work items of fixed numbers of tiles (fewer
+// gradient partials) that shares the tables of `of`, which has the same desc.
+static int nn_plan_create(const tdx_nn_desc *d, tdx_nn_plan **out, const tdx_nn_plan *of) {
+  const bool fixed = of != nullptr;
   TDX_REQUIRE(d && out, "null argument");
   *out = nullptr;
   TDX_REQUIRE(d->dtype == 0 || d->dtype == 1, "dtype must be 0 (f32) or 1 (f64)");
@@ -2102,6 +2109,7 @@ static int nn_plan_create(const tdx_nn_desc *d, tdx_nn_plan **out, bool fixed) {
                   "weak form: group 0's residuals must lead the residual output");
   }
   tdx_nn_plan *p = new tdx_nn_plan();
+  p->fixed_of = of;
   p->dtype = d->dtype;
   p->d_in = d->d_in;
   p->n_out = d->n_out;
@@ -2388,38 +2396,43 @@ static int nn_plan_create(const tdx_nn_desc *d, tdx_nn_plan **out, bool fixed) {
     }
   }
 
+  auto shared = [&](DevTable tdx_nn_plan::*t, const void *src, size_t n) -> int {
+    if (!of) return (p->*t).upload(src, n);
+    (p->*t).borrow(of->*t);
+    return TDX_OK;
+  };
   int r2 = TDX_OK;
   if (!r2 && p->red_slices > 1) r2 = p->ik5p.upload(ik5p.data(), ik5p.size() * 4);
   if (!r2 && p->red_slices > 1) r2 = p->ik5i.upload(ik5i.data(), ik5i.size() * 4);
-  if (!r2) r2 = p->groups.upload(d->groups, (size_t)d->n_groups * TDX_GROUP_INTS * 4);
-  if (!r2) r2 = p->ints.upload(d->ints, (size_t)std::max<int64_t>(d->n_ints, 1) * 4);
-  if (!r2) r2 = p->reals.upload(d->reals, (size_t)d->n_reals * ts);
-  if (!r2) r2 = p->data.upload(d->data, (size_t)d->n_data * ts);
-  if (!r2) r2 = p->k1_items.upload(k1.data(), k1.size() * sizeof(int2));
+  if (!r2) r2 = shared(&tdx_nn_plan::groups, d->groups, (size_t)d->n_groups * TDX_GROUP_INTS * 4);
+  if (!r2) r2 = shared(&tdx_nn_plan::ints, d->ints, (size_t)std::max<int64_t>(d->n_ints, 1) * 4);
+  if (!r2) r2 = shared(&tdx_nn_plan::reals, d->reals, (size_t)d->n_reals * ts);
+  if (!r2) r2 = shared(&tdx_nn_plan::data, d->data, (size_t)d->n_data * ts);
+  if (!r2) r2 = shared(&tdx_nn_plan::k1_items, k1.data(), k1.size() * sizeof(int2));
   if (!r2) r2 = p->k2_items.upload(k2.data(), k2.size() * sizeof(int4));
-  if (!r2) r2 = p->ik1p.upload(ik1p.data(), ik1p.size() * 4);
-  if (!r2) r2 = p->ik1i.upload(ik1i.data(), ik1i.size() * 4);
+  if (!r2) r2 = shared(&tdx_nn_plan::ik1p, ik1p.data(), ik1p.size() * 4);
+  if (!r2) r2 = shared(&tdx_nn_plan::ik1i, ik1i.data(), ik1i.size() * 4);
   if (!r2) r2 = p->ik2p.upload(ik2p.data(), ik2p.size() * 4);
   if (!r2) r2 = p->ik2i.upload(ik2i.data(), ik2i.size() * 4);
   if (!r2 && p->k2_fs) {
     r2 = p->k4_items.upload(k4.data(), k4.size() * sizeof(int4));
     if (!r2) r2 = p->ik4p.upload(ik4p.data(), ik4p.size() * 4);
     if (!r2) r2 = p->ik4i.upload(ik4i.data(), ik4i.size() * 4);
-    if (!r2) r2 = p->prog_idx.upload(prog_idx.data(), prog_idx.size() * sizeof(int4));
-    if (!r2) r2 = p->prog_ints.upload(prog_ints.data(), prog_ints.size() * 4);
-    if (!r2) r2 = p->prog_reals.upload(prog_reals.data(), prog_reals.size() * 4);
+    if (!r2) r2 = shared(&tdx_nn_plan::prog_idx, prog_idx.data(), prog_idx.size() * sizeof(int4));
+    if (!r2) r2 = shared(&tdx_nn_plan::prog_ints, prog_ints.data(), prog_ints.size() * 4);
+    if (!r2) r2 = shared(&tdx_nn_plan::prog_reals, prog_reals.data(), prog_reals.size() * 4);
     if (!r2 && !prog_kind.empty())
-      r2 = p->prog_kind.upload(prog_kind.data(), prog_kind.size() * 4);
+      r2 = shared(&tdx_nn_plan::prog_kind, prog_kind.data(), prog_kind.size() * 4);
   }
   if (!r2 && p->fused) {
     r2 = p->k3_items.upload(k3.data(), k3.size() * sizeof(int4));
     if (!r2) r2 = p->ik3p.upload(ik3p.data(), ik3p.size() * 4);
     if (!r2) r2 = p->ik3i.upload(ik3i.data(), ik3i.size() * 4);
-    if (!r2) r2 = p->prog_idx.upload(prog_idx.data(), prog_idx.size() * sizeof(int4));
-    if (!r2) r2 = p->prog_ints.upload(prog_ints.data(), prog_ints.size() * 4);
-    if (!r2) r2 = p->prog_reals.upload(prog_reals.data(), prog_reals.size() * 4);
+    if (!r2) r2 = shared(&tdx_nn_plan::prog_idx, prog_idx.data(), prog_idx.size() * sizeof(int4));
+    if (!r2) r2 = shared(&tdx_nn_plan::prog_ints, prog_ints.data(), prog_ints.size() * 4);
+    if (!r2) r2 = shared(&tdx_nn_plan::prog_reals, prog_reals.data(), prog_reals.size() * 4);
     if (!r2 && !prog_kind.empty())
-      r2 = p->prog_kind.upload(prog_kind.data(), prog_kind.size() * 4);
+      r2 = shared(&tdx_nn_plan::prog_kind, prog_kind.data(), prog_kind.size() * 4);
   }
   if (!r2 && p->persist) {
     // persistent forward: as many workgroups as the device keeps resident,
@@ -2501,16 +2514,22 @@ static int nn_plan_create(const tdx_nn_desc *d, tdx_nn_plan **out, bool fixed) {
   return TDX_OK;
 }
 
-// Plans that the no-allocation entry point takes keep to fixed work items
-// where the sized ones would need more than its array.
+// A plan whose sized work items need more than the no-allocation entry
+// point's array, and fixed ones do not, carries a second list of items for that
+// entry point alone; without one (no device memory for its lists) that entry
+// point refuses the plan.
 extern "C" int tdx_nn_plan_create(const tdx_nn_desc *d, tdx_nn_plan **out) {
-  const int rc = nn_plan_create(d, out, false);
+  const int rc = nn_plan_create(d, out, nullptr);
   if (rc != TDX_OK || d->chunk_tiles > 0) return rc;
-  if ((*out)->ws_bytes <= kNoAllocBytes || (*out)->ws_fixed > kNoAllocLimit) return rc;
-  tdx_nn_plan_destroy(*out);
-  return nn_plan_create(d, out, true);
+  tdx_nn_plan *p = *out;
+  if (p->ws_bytes <= kNoAllocBytes || p->ws_fixed > kNoAllocLimit) return rc;
+  if (nn_plan_create(d, &p->fixed_items, p) != TDX_OK) clear_error();
+  return TDX_OK;
 }
 
+const tdx_nn_plan *tdx::nn_noalloc_plan(const tdx_nn_plan *p) {
+  return p->fixed_items ? p->fixed_items : p;
+}
 size_t tdx::nn_workspace_fixed_bytes(const tdx_nn_plan *p) { return p ? p->ws_fixed : 0; }
 
 extern "C" int tdx_nn_profile(tdx_nn_plan *p, int capacity) {
@@ -2549,6 +2568,7 @@ extern "C" int tdx_nn_profile_read(tdx_nn_plan *p, double *ms, int *count) {
 
 extern "C" void tdx_nn_plan_destroy(tdx_nn_plan *p) {
   if (!p) return;
+  tdx_nn_plan_destroy(p->fixed_items);
   (void)tdx_nn_profile(p, 0);
   DevTable *t[] = {&p->groups,   &p->ints,     &p->reals,     &p->data,     &p->k1_items,
                    &p->k2_items, &p->ik1p,     &p->ik1i,      &p->ik2p,     &p->ik2i,

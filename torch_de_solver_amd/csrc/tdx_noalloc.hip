@@ -57,12 +57,14 @@ extern "C" int tdx_nn_train_step_noalloc(const tdx_nn_plan *p, void *params, voi
                                          double beta1, double beta2, double eps, void *loss,
                                          tdx_stream_t stream) {
   TDX_REQUIRE(p && params && exp_avg && exp_avg_sq && step, "null argument");
-  const size_t fixed = tdx::nn_workspace_fixed_bytes(p), need = tdx_nn_workspace_bytes(p);
+  const size_t fixed = tdx::nn_workspace_fixed_bytes(p);
   TDX_REQUIRE(fixed <= tdx::kNoAllocLimit,
               "the plan's workspace, with fixed work items and float32 images, takes %zu bytes; "
               "the no-allocation entry point serves up to %zu (use tdx_nn_train_step with a "
               "caller workspace)",
               fixed, tdx::kNoAllocLimit);
+  p = tdx::nn_noalloc_plan(p);
+  const size_t need = tdx_nn_workspace_bytes(p);
   TDX_REQUIRE(need <= tdx::kNoAllocBytes,
               "the plan needs %zu bytes of workspace; the no-allocation entry point holds "
               "%zu (use tdx_nn_train_step with a caller workspace)",
