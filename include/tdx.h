@@ -145,8 +145,8 @@ typedef struct tdx_nn_desc {
    * on them and forms its own seeds (three launches; chunk_tiles counts
    * such tiles, default 8).  Otherwise, and with -1, separate forward and
    * adjoint kernels, one workgroup per work item.  1: separate kernels with the
-   * persistent forward: when the network's forward image fits in LDS
-   * and the plan has no causal or weak-form loss, the forward kernel runs
+   * persistent forward: when the network's forward image fits in LDS (160 KB
+   * with the kernel's own words, float images in bf16 pieces) and the plan has no causal or weak-form loss, the forward kernel runs
    * as a grid of CUs x resident workgroups, each walking a contiguous range
    * of equal cost of the (instance, entry tile) work items and gathering
    * its instance's network into LDS from the parameters when the instance

@@ -63,15 +63,37 @@ __global__ void k_pack(NNArgs<T> a) {
   }
 }
 
-// The same LDS copy as stage_net, gathered from the instance's parameters
-// (no packed image in global memory needed).  Ends with a workgroup
+// The layer images (which: 0 Wf, 1 Wb) of the instance with parameters W, by
+// the whole workgroup.  float: a thread forms the three pieces of a pair at
+// once.
+template <typename T, int NB>
+__device__ __forceinline__ void gather_layers(const NNArgs<T> &a, const T *W, int which, T *dst) {
+  constexpr int LI = Net<T, NB>::LI;
+  if constexpr (sizeof(T) == 4) {
+    for (int k = threadIdx.x; k < a.NH * (LI / 3); k += blockDim.x) {
+      const int j = k / (LI / 3);
+      int at;
+      const Bits3 b = image_pair<NB>(a, W, which, j, k - j * (LI / 3), at);
+      float *to = dst + j * LI + at;
+      to[0] = __builtin_bit_cast(float, b.h);
+      to[kPieceWords<NB>] = __builtin_bit_cast(float, b.m);
+      to[2 * kPieceWords<NB>] = __builtin_bit_cast(float, b.l);
+    }
+  } else {
+    const int off = which ? a.NH * LI + small_words(16 * NB, a.NH, a.d_in, a.n_out) : 0;
+    for (int k = threadIdx.x; k < a.NH * LI; k += blockDim.x)
+      dst[k] = image_value<T, NB>(a, W, off + k);
+  }
+}
+
+// The same LDS copy as stage_net (without Wb), gathered from the instance's
+// parameters (no packed image in global memory needed).  Ends with a workgroup
 // barrier.
 template <typename T, int NB>
-__device__ void gather_image(const NNArgs<T> &a, int inst, T *dst, bool with_wb) {
-  constexpr int HP = 16 * NB;
-  const T *W = a.params + (int64_t)inst * a.P;
-  const int n = stage_words(HP, a.NH, a.d_in, a.n_out, with_wb, sizeof(T));
-  for (int k = threadIdx.x; k < n; k += blockDim.x) dst[k] = image_value<T, NB>(a, W, k);
+__device__ void gather_image(const NNArgs<T> &a, const T *W, T *dst) {
+  const int n = a.NH * Net<T, NB>::LI, sw = small_words(16 * NB, a.NH, a.d_in, a.n_out);
+  gather_layers<T, NB>(a, W, 0, dst);
+  for (int k = threadIdx.x; k < sw; k += blockDim.x) dst[n + k] = image_value<T, NB>(a, W, n + k);
   __syncthreads();
 }
 
@@ -110,8 +132,8 @@ __device__ __forceinline__ T *forward_stage_area(const NNArgs<T> &a, T *smem) {
 // One forward work item (64 entries of one group): network at every slot,
 // residual program, loss partials (lp[2 it], lp[2 it + 1]) and seeds.
 template <typename T, int NB, bool STAGE>
-__device__ __forceinline__ void forward_item(const NNArgs<T> &a, int it, const Net<T, NB> &net,
-                                             T *smem) {
+__device__ __forceinline__ void forward_item(const NNArgs<T> &a, int it,
+                                             const Net<T, NB, STAGE> &net, T *smem) {
   const int2 item = a.k1_items[it];
   const int32_t *G = a.groups + item.x * TDX_GROUP_INTS;
   const int n_entries = G[1], n_slots = G[2];
@@ -143,10 +165,10 @@ __device__ __forceinline__ void forward_item(const NNArgs<T> &a, int it, const N
       x[k] = (k < a.d_in) ? a.data[base + (int64_t)ec * a.d_in + k] +
                                 a.reals[slot_off_r + s * a.d_in + k]
                           : T(0);
-    layer_in<T, NB>(net, x, q, act);
-    for (int j = 0; j < a.NH; ++j) layer_hidden<T, NB>(net, j, lane, act);
+    layer_in(net, x, q, act);
+    for (int j = 0; j < a.NH; ++j) layer_hidden(net, j, lane, act);
     for (int o = 0; o < a.n_out; ++o) {
-      const T u = layer_out<T, NB>(net, o, q, act);
+      const T u = layer_out(net, o, q, act);
       if (q == 0) u_lds[s * a.n_out + o] = u;
       if (a.u_out && q == 0 && valid)
         a.u_out[(row_base + (int64_t)s * n_entries + e) * a.n_out + o] = u;
@@ -216,25 +238,26 @@ __global__ __launch_bounds__(256) void k_forward(NNArgs<T> a) {
     const int lo = a.k1_bounds[blockIdx.x], hi = a.k1_bounds[blockIdx.x + 1];
     int cur = -1;
     T *stage = forward_stage_area(a, smem);
-    const Net<T, NB> net = net_at<T, NB>(a, stage);
+    const Net<T, NB, STAGE> net = net_at<T, NB, STAGE>(a, stage);
     for (int it = lo; it < hi; ++it) {
       const int inst = a.groups[a.k1_items[it].x * TDX_GROUP_INTS];
       __syncthreads();
       if (!a.u_in && inst != cur) {
-        gather_image<T, NB>(a, inst, stage, false);
+        const T *W = a.params + (int64_t)inst * a.P;
+        gather_image<T, NB>(a, W, stage);
         cur = inst;
         if (it == a.inst_k1_idx[a.inst_k1_ptr[inst]]) {
           constexpr int HP = 16 * NB;
-          const int IMG = image_words(HP, a.NH, a.d_in, a.n_out, sizeof(T));
-          const T *W = a.params + (int64_t)inst * a.P;
-          T *dst = a.packed + (int64_t)inst * IMG;
-          for (int k = threadIdx.x; k < IMG; k += blockDim.x) dst[k] = image_value<T, NB>(a, W, k);
+          T *dst = a.packed + (int64_t)inst * image_words(HP, a.NH, a.d_in, a.n_out, sizeof(T));
+          const int n = stage_words(HP, a.NH, a.d_in, a.n_out, false, sizeof(T));
+          for (int k = threadIdx.x; k < n; k += blockDim.x) dst[k] = stage[k];
+          gather_layers<T, NB>(a, W, 1, dst + n);
         }
       }
       forward_item<T, NB, STAGE>(a, it, net, smem);
     }
   } else {
-    Net<T, NB> net;
+    Net<T, NB, STAGE> net;
     if (!a.u_in) {
       const int inst = a.groups[a.k1_items[blockIdx.x].x * TDX_GROUP_INTS];
       if constexpr (STAGE)
@@ -310,9 +333,9 @@ __global__ __launch_bounds__(256) void k_backward(NNArgs<T> a) {
 
     // forward recompute, activations to LDS
     T act[NB][4];
-    layer_in<T, NB>(net, x, q, act);
+    layer_in(net, x, q, act);
     for (int j = 0; j <= a.NH; ++j) {
-      if (j > 0) layer_hidden<T, NB>(net, j - 1, lane, act);
+      if (j > 0) layer_hidden(net, j - 1, lane, act);
       T *dstl = act_l + ((int64_t)j * TR + trow) * LS;
 #pragma unroll
       for (int mb = 0; mb < NB; ++mb)
@@ -471,7 +494,7 @@ __device__ __forceinline__ int backward_w_buffer_words(int NW, int P) {
 // wavefront-private backward: its gradient partial goes to partial[it].
 template <typename T, int NB, int NH, int NT>
 __device__ __forceinline__ void backward_w_item(const NNArgs<T> &a, int it,
-                                                const Net<T, NB> &net, T *smem) {
+                                                const Net<T, NB, true> &net, T *smem) {
   constexpr int HP = 16 * NB;
   constexpr int FB = WRS * HP;  // words of one feature-major buffer
   typedef typename V4<T>::type v4;
@@ -570,7 +593,7 @@ __device__ __forceinline__ void backward_w_item(const NNArgs<T> &a, int it,
     // forward recompute, every activation kept
     T act[NH + 1][NT][NB][4];
 #pragma unroll
-    for (int t = 0; t < NT; ++t) layer_in<T, NB>(net, x[t], q, act[0][t]);
+    for (int t = 0; t < NT; ++t) layer_in(net, x[t], q, act[0][t]);
 #pragma unroll
     for (int j = 1; j <= NH; ++j) {
       v4 acc[NT][NB];
@@ -785,7 +808,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(
   extern __shared__ __align__(16) unsigned char smem_raw[];
   T *smem = reinterpret_cast<T *>(smem_raw);
   T *stage = smem + backward_w_buffer_words<NB, NT>(blockDim.x >> 6, a.P);
-  const Net<T, NB> net = stage_net<T, NB>(a, a.k2_items[blockIdx.x].w, stage, true);
+  const auto net = stage_net<T, NB>(a, a.k2_items[blockIdx.x].w, stage, true);
   backward_w_item<T, NB, NH, NT>(a, blockIdx.x, net, smem);
 }
 
@@ -1464,6 +1487,7 @@ int launch_forward_kernel(const tdx_nn_plan *p, const NNArgs<T> &a, hipStream_t 
     raise_lds_limit({(const void *)k_forward<T, NB, true, true>});
     hipLaunchKernelGGL((k_forward<T, NB, true, true>), dim3(p->g1), dim3(256), p->k1_lds, s, a);
   } else if (p->k1_stage) {
+    raise_lds_limit({(const void *)k_forward<T, NB, true, false>});
     hipLaunchKernelGGL((k_forward<T, NB, true, false>), dim3(p->n_k1), dim3(256), p->k1_lds, s,
                        a);
   } else {
@@ -2143,11 +2167,17 @@ static int nn_plan_create(const tdx_nn_desc *d, tdx_nn_plan **out, const tdx_nn_
     max_slots = std::max(max_slots, (int)d->groups[(int64_t)g * TDX_GROUP_INTS + 2]);
   p->max_slots = max_slots;
   p->k1_lds = (2 * K1_WAVES * 16 * max_slots * d->n_out + 512) * ts;
+  const bool persist = d->persistent > 0 && d->causal_tol == 0.0 && d->weak_levels == 0;
   {
-    // stage the forward operand images in LDS when they are small
+    // Stage the forward operand images in LDS: what leaves room for a second
+    // workgroup on a CU (64 KB), and all that fits (160 KB) where the grid is
+    // one workgroup a CU or less, or persistent.  A forward pass, global images
+    // against staged ones: 256 x 100 points, 2-48x2-1 43 -> 41 us, 2-80x2-1
+    // 63 -> 55, 2-100x2-1 (81 KB) 85 -> 109; 40 x 30 points (18 workgroups),
+    // 2-48x4-1 53 -> 48, 2-100x2-1 67 -> 56.
     const size_t st = (size_t)stage_words(p->HP, p->NH, d->d_in, d->n_out, false, (int)ts) * ts;
-    // (wide float layers read their operand images from global memory)
-    p->k1_stage = (p->k1_lds + st <= 64 * 1024 && (d->dtype == 1 || p->NB <= 2)) ? 1 : 0;
+    const size_t limit = persist || k1.size() <= (size_t)kCUs ? 160 * 1024 : 64 * 1024;
+    p->k1_stage = p->k1_lds + st <= limit ? 1 : 0;
     if (p->k1_stage) p->k1_lds += st;
   }
 
@@ -2192,8 +2222,7 @@ static int nn_plan_create(const tdx_nn_desc *d, tdx_nn_plan **out, const tdx_nn_
     p->acc_lds = 1;
     p->k2_lds = block_lds_words(p->HP, p->NH) * ts;
   }
-  p->persist = (d->persistent > 0 && p->k1_stage && d->causal_tol == 0.0 &&
-                d->weak_levels == 0) ? 1 : 0;
+  p->persist = persist && p->k1_stage ? 1 : 0;
   const int TR = 16 * p->k2_waves;
   std::vector<int64_t> k2_tiles;
   for (int g = 0; g < d->n_groups; ++g) {

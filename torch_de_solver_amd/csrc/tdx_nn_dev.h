@@ -125,6 +125,36 @@ __device__ __forceinline__ int feature_at(int p) {
   return (p & ~15) + crow<T>((p & 15) >> 2, p & 3);
 }
 
+// Pair q of layer j's float image (which: 0 Wf, 1 Wb) from the parameters W:
+// its three pieces, piece p at word at + p * kPieceWords of the layer.
+struct Bits3 {
+  unsigned h, m, l;
+};
+template <int NB>
+constexpr int kPieceWords = NB == 1 ? 128 : 256;
+template <int NB>
+__device__ __forceinline__ Bits3 image_pair(const NNArgs<float> &a, const float *W, int which,
+                                            int j, int q, int &at) {
+  constexpr int KS = (NB + 1) / 2, PW = kPieceWords<NB>, LW = PW / 64;  // words a lane
+  const int H = a.H;
+  const Layout<float> L{a.d_in, a.n_out, H, a.NH};
+  const int t = q % LW, lane = (q / LW) & 63, step = q / PW;
+  const int ks = step % KS, xb = step / KS;
+  at = step * 3 * PW + lane * LW + t;
+  float w2[2];
+#pragma unroll
+  for (int k = 0; k < 2; ++k) {
+    const int e = 2 * t + k;
+    const int f = 16 * (2 * ks + (e >> 2)) + 4 * (lane >> 4) + (e & 3);
+    const int x = 16 * xb + (lane & 15);
+    const int out = which == 0 ? x : f, in = which == 0 ? f : x;
+    w2[k] = (out < H && in < H) ? W[L.oWh(j) + out * H + in] : 0.f;
+  }
+  unsigned h[1], m[1], l[1];
+  bf3_pairs<1>(w2, h, m, l);
+  return Bits3{h[0], m[0], l[0]};
+}
+
 // Word `off` of an instance's packed image, from its parameters W (torch
 // layout).
 template <typename T, int NB>
@@ -142,22 +172,11 @@ __device__ __forceinline__ T image_value(const NNArgs<T> &a, const T *W, int off
       const int j = off / img;
       int r = off - j * img;
       if constexpr (sizeof(T) == 4) {
-        constexpr int KS = (NB + 1) / 2, TB = NB == 1 ? 1 : 2;  // 2^TB words a lane
-        const int t = r & ((1 << TB) - 1), lane = (r >> TB) & 63;
-        r >>= TB + 6;
-        const int p = r % 3, ks = (r / 3) % KS, xb = r / (3 * KS);
-        T w2[2];
-#pragma unroll
-        for (int k = 0; k < 2; ++k) {
-          const int e = 2 * t + k;
-          const int f = 16 * (2 * ks + (e >> 2)) + 4 * (lane >> 4) + (e & 3);
-          const int x = 16 * xb + (lane & 15);
-          const int out = which == 0 ? x : f, in = which == 0 ? f : x;
-          w2[k] = (out < H && in < H) ? W[L.oWh(j) + out * H + in] : T(0);
-        }
-        unsigned h[1], m[1], l[1];
-        bf3_pairs<1>(w2, h, m, l);
-        v = __builtin_bit_cast(float, p == 0 ? h[0] : (p == 1 ? m[0] : l[0]));
+        constexpr int PW = kPieceWords<NB>;
+        const int p = r / PW % 3;
+        int at;
+        const Bits3 b = image_pair<NB>(a, W, which, j, r / (3 * PW) * PW + r % PW, at);
+        v = __builtin_bit_cast(float, p == 0 ? b.h : (p == 1 ? b.m : b.l));
       } else {
         const int i = r & 3;
         const int lane = (r >> 2) & 63;
@@ -196,7 +215,9 @@ __device__ __forceinline__ T image_value(const NNArgs<T> &a, const T *W, int off
 // ---------------------------------------------------------------------------
 // network view: the packed image in global memory or its copy in LDS
 // ---------------------------------------------------------------------------
-template <typename T, int NB>
+// S: a copy in LDS (float layers of several k-steps read a global image by
+// buffer loads).
+template <typename T, int NB, bool S = false>
 struct Net {
   const T *Wf, *Wb;          // layer j image at Wf + j * LI
   static constexpr int LI = layer_words(16 * NB, sizeof(T));
@@ -204,10 +225,10 @@ struct Net {
   Layout<T> L;
 };
 
-template <typename T, int NB>
-__device__ __forceinline__ Net<T, NB> net_at(const NNArgs<T> &a, const T *base) {
+template <typename T, int NB, bool S = false>
+__device__ __forceinline__ Net<T, NB, S> net_at(const NNArgs<T> &a, const T *base) {
   constexpr int HP = 16 * NB;
-  Net<T, NB> n;
+  Net<T, NB, S> n;
   n.L = Layout<T>{a.d_in, a.n_out, a.H, a.NH};
   n.Wf = base;
   const T *sm = base + a.NH * Net<T, NB>::LI;
@@ -233,16 +254,29 @@ __device__ __forceinline__ Net<T, NB> make_net(const NNArgs<T> &a, int inst) {
 // LDS at `dst`; returns the network view on the copy.  Ends with a
 // workgroup barrier.
 template <typename T, int NB>
-__device__ Net<T, NB> stage_net(const NNArgs<T> &a, int inst, T *dst, bool with_wb) {
+__device__ Net<T, NB, true> stage_net(const NNArgs<T> &a, int inst, T *dst, bool with_wb) {
   constexpr int HP = 16 * NB;
   typedef typename V4<T>::type v4;
   const T *src = a.packed + (int64_t)inst * image_words(HP, a.NH, a.d_in, a.n_out, sizeof(T));
   const int n4 = stage_words(HP, a.NH, a.d_in, a.n_out, with_wb, sizeof(T)) / 4;
   const v4 *s4 = reinterpret_cast<const v4 *>(src);
   v4 *d4 = reinterpret_cast<v4 *>(dst);
-  for (int k = threadIdx.x; k < n4; k += blockDim.x) d4[k] = s4[k];
+  // eight loads in flight: the copy is a latency of L2 or more per round
+  for (int k0 = threadIdx.x; k0 < n4; k0 += 8 * blockDim.x) {
+    v4 v[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int k = k0 + i * blockDim.x;
+      v[i] = s4[k < n4 ? k : k0];
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int k = k0 + i * blockDim.x;
+      if (k < n4) d4[k] = v[i];
+    }
+  }
   __syncthreads();
-  return net_at<T, NB>(a, dst);
+  return net_at<T, NB, true>(a, dst);
 }
 
 // Four consecutive values of a small array at accumulator position p.
@@ -252,8 +286,8 @@ __device__ __forceinline__ typename V4<T>::type ld4(const T *p) {
 }
 
 // Layer 1 (VALU): act[mb][i] = tanh(b1[f] + sum_a x[a] W1[f][a]).
-template <typename T, int NB>
-__device__ __forceinline__ void layer_in(const Net<T, NB> &n, const T *x, int q,
+template <typename T, int NB, bool S>
+__device__ __forceinline__ void layer_in(const Net<T, NB, S> &n, const T *x, int q,
                                          T (&act)[NB][4]) {
   constexpr int HP = 16 * NB;
   typedef typename V4<T>::type v4;
@@ -290,23 +324,23 @@ __device__ __forceinline__ void split_act(const float (&b)[NB][4], Bf3 (&s)[(NB 
 }
 
 // acc[ob] += W (rows of block ob) x the split operand s, per block the leading
-// and the small products of every k-step in two accumulators from zero.  Wide layers read their weights from L2: the next block's are
-// loaded while this one is multiplied, and no more than that is kept in
-// flight (the scheduler otherwise hoists every load and spills).
-template <int NB>
+// and the small products of every k-step in two accumulators from zero.  Wide
+// layers read their weights from L2 (S: from LDS): the next block's are loaded
+// while this one is multiplied, and no more than that is kept in flight (the
+// scheduler otherwise hoists every load and spills).
+template <int NB, bool S>
 __device__ __forceinline__ void mma_split(const float *img, int lane,
                                           const Bf3 (&s)[(NB + 1) / 2], f4_t (&acc)[NB]) {
   // operand steps t = ob * KS + ks in a ring, KS steps ahead when wide
   constexpr int KS = (NB + 1) / 2, NT = NB * KS, AHEAD = KS > 1 ? KS : 1, RING = AHEAD + 1;
   Bf3 w[RING];
-  // wide images are in global memory (never staged): buffer loads take a
-  // scalar descriptor and offset and one lane offset, so no address occupies
-  // vector registers (as plain pointers the tile loop's hoisted addresses
-  // spilled up to 2 KB a lane)
+  // wide images in global memory: buffer loads take a scalar descriptor and
+  // offset and one lane offset, so no address occupies vector registers (as
+  // plain pointers the tile loop's hoisted addresses spilled up to 2 KB a lane)
   const auto rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(img), (short)0,
                                                     NT * 3072, 0x00027000);
   auto load = [&](int t, Bf3 &d) {
-    if constexpr (KS > 1) {
+    if constexpr (KS > 1 && !S) {
       const int o = 16 * lane, so = t * 3072;
       d.h = __builtin_amdgcn_raw_buffer_load_b128(rs, o, so, 0);
       d.m = __builtin_amdgcn_raw_buffer_load_b128(rs, o, so + 1024, 0);
@@ -340,14 +374,14 @@ __device__ __forceinline__ void mma_split(const float *img, int lane,
 }
 
 // acc[ob] += W_j (rows of block ob) x act, W given as an operand image.
-template <typename T, int NB>
+template <typename T, int NB, bool S = false>
 __device__ __forceinline__ void mma_layer(const T *img, int lane, const T (&b)[NB][4],
                                           typename V4<T>::type (&acc)[NB]) {
   typedef typename V4<T>::type v4;
   if constexpr (sizeof(T) == 4) {
     Bf3 s[(NB + 1) / 2];
     split_act<NB>(b, s);
-    mma_split<NB>(img, lane, s, acc);
+    mma_split<NB, S>(img, lane, s, acc);
   } else {
     const v4 *wp = reinterpret_cast<const v4 *>(img) + lane;
 #pragma unroll
@@ -363,8 +397,8 @@ __device__ __forceinline__ void mma_layer(const T *img, int lane, const T (&b)[N
 
 // Hidden layer j (MFMA on top of the bias):
 // act <- tanh(b_j + W_j act).
-template <typename T, int NB>
-__device__ __forceinline__ void layer_hidden(const Net<T, NB> &n, int j, int lane,
+template <typename T, int NB, bool S>
+__device__ __forceinline__ void layer_hidden(const Net<T, NB, S> &n, int j, int lane,
                                              T (&act)[NB][4]) {
   constexpr int HP = 16 * NB;
   typedef typename V4<T>::type v4;
@@ -372,7 +406,7 @@ __device__ __forceinline__ void layer_hidden(const Net<T, NB> &n, int j, int lan
   v4 acc[NB];
 #pragma unroll
   for (int ob = 0; ob < NB; ++ob) acc[ob] = ld4(n.bh + j * HP + 16 * ob + 4 * q);
-  mma_layer<T, NB>(n.Wf + j * n.LI, lane, act, acc);
+  mma_layer<T, NB, S>(n.Wf + j * n.LI, lane, act, acc);
 #pragma unroll
   for (int ob = 0; ob < NB; ++ob)
 #pragma unroll
@@ -380,8 +414,8 @@ __device__ __forceinline__ void layer_hidden(const Net<T, NB> &n, int j, int lan
 }
 
 // Output layer (VALU + cross-quarter shuffle): u[o] for the lane's row.
-template <typename T, int NB>
-__device__ __forceinline__ T layer_out(const Net<T, NB> &n, int o, int q,
+template <typename T, int NB, bool S>
+__device__ __forceinline__ T layer_out(const Net<T, NB, S> &n, int o, int q,
                                        const T (&act)[NB][4]) {
   constexpr int HP = 16 * NB;
   typedef typename V4<T>::type v4;
@@ -821,7 +855,7 @@ __device__ __forceinline__ void fused_body(const NNArgs<float> &a, float *smem) 
   T *rarea = lbuf + 128;
   T *stage = rarea + R::kWords;
   R resid(a, item.x, n_eq, rarea, w);
-  const Net<T, NB> net = stage_net<T, NB>(a, G[0], stage, true);  // ends with a barrier
+  const auto net = stage_net<T, NB>(a, G[0], stage, true);  // ends with a barrier
   const T dl_scale = *a.dloss;
 
   // gradient accumulators, as in the wavefront-private backward (one output
@@ -870,16 +904,16 @@ __device__ __forceinline__ void fused_body(const NNArgs<float> &a, float *smem) 
                              : T(0);
         x[k][0] = xs[0];
         x[k][1] = xs[1];
-        layer_in<T, NB>(net, xs, q, act[k][0]);
+        layer_in(net, xs, q, act[k][0]);
 #pragma unroll
         for (int j = 1; j <= NH; ++j) {
 #pragma unroll
           for (int mb = 0; mb < NB; ++mb)
 #pragma unroll
             for (int i = 0; i < 4; ++i) act[k][j][mb][i] = act[k][j - 1][mb][i];
-          layer_hidden<T, NB>(net, j - 1, lane, act[k][j]);
+          layer_hidden(net, j - 1, lane, act[k][j]);
         }
-        const T u = layer_out<T, NB>(net, 0, q, act[k][NH]);
+        const T u = layer_out(net, 0, q, act[k][NH]);
         if (q == 0) ub[row * FUSE_MAX_SLOTS + s] = u;
       }
     }
@@ -1202,7 +1236,7 @@ __device__ __forceinline__ void block_body(const NNArgs<T> &a, T *smem) {
 
     // forward recompute of this wavefront's 16 rows, every layer to LDS
     T act[NB][4];
-    layer_in<T, NB>(net, x, q, act);
+    layer_in(net, x, q, act);
     store_rows(layer_buf(0), act);
 #pragma unroll 1
     for (int j = 1; j <= NH; ++j) {
@@ -1224,7 +1258,7 @@ __device__ __forceinline__ void block_body(const NNArgs<T> &a, T *smem) {
 #pragma unroll
       for (int o = 0; o < MAXO; ++o)
         if (o < n_out) {
-          const T u = layer_out<T, NB>(net, o, q, act);
+          const T u = layer_out(net, o, q, act);
           if (q == 0) ubuf[trow * n_out + o] = u;
         }
       __syncthreads();
