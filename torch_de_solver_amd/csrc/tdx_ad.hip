@@ -1020,10 +1020,10 @@ __global__ void k_ad_jac_zero(T *jt, int64_t n) {
 // k_ad_step: the fused training step with the jet maps and the residual
 // program interpreted from the plan's tables.
 template <int NB, int NHM>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ad_step_wgs(NB)))) void
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ad_step_waves(NB)))) void
 k_ad_step(ADStepArgs a) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
-  ad_step_body<NB, NHM, InterpJets, InterpADResid>(a, reinterpret_cast<float *>(smem_raw));
+  ad_step_body<NB, NHM, InterpJets<NB>, InterpADResid>(a, reinterpret_cast<float *>(smem_raw));
 }
 
 // k_ad_loss_pass: the fused step's forward half, for evaluations that want
@@ -1035,7 +1035,7 @@ template <int NB>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ad_step_wgs(NB)))) void
 k_ad_loss_pass(ADStepArgs a) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
-  ad_step_body<NB, 4, InterpJets, InterpADResid, true>(a, reinterpret_cast<float *>(smem_raw));
+  ad_step_body<NB, 4, InterpJets<NB>, InterpADResid, true>(a, reinterpret_cast<float *>(smem_raw));
 }
 
 // Image of the network for k_ad_step (one instance) and the Adam step

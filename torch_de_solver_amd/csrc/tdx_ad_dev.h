@@ -167,11 +167,23 @@ __host__ __device__ inline size_t ad_step_lds_bytes(int HP) {
   return (size_t)(3 * HP * CTRS + (MAXD + 1 + MAXO) * CTRS + 2 * 64 * MAXO + 32) * 4;
 }
 
+// Wavefronts per SIMD that the interpreted step kernel is compiled for.  Up to
+// two blocks its registers leave room for two without being told so, and told
+// so the scheduler lengthens the jet maps, most of such a step (32 x 40 points,
+// one tile a workgroup, 2-32x2-1: 6.7k -> 7.9k cycles a forward map).
+__host__ __device__ constexpr int ad_step_waves(int NB) { return NB <= 2 ? 1 : ad_step_wgs(NB); }
+
 // Activation jets h of the wavefront's NP points from their pre-activation
-// jets z (feature-major, rows r0 + p J + alpha).  Each lane takes ADF_R
-// (point, unit) items at once, so the table reads (uniform) are issued once
-// for all of them and their LDS reads overlap.
+// jets z (feature-major, rows r0 + p J + alpha).  Each lane takes R (point,
+// unit) items at once, so the table reads (uniform) are issued once for all of
+// them and their LDS reads overlap.  R is 5 (three points of 100 units), and
+// ad_small_r(NB) where that holds all of a narrow network's items: the slots
+// beyond them cost their instructions (32 x 40 points, three points a
+// wavefront, cycles a forward and an adjoint map: 32 units 8.0k, 16.5k with
+// five, 4.1k, 9.5k with two; 64 units 8.1k, 16.6k with five, 5.7k, 12k with
+// three).
 constexpr int ADF_R = 5;
+__host__ __device__ constexpr int ad_small_r(int NB) { return NB <= 2 ? 2 : NB <= 4 ? 3 : ADF_R; }
 
 // Reads of the plan's read-only tables at wavefront-uniform indices, through
 // the constant address space: scalar loads, which do not wait behind LDS
@@ -183,10 +195,11 @@ __device__ __forceinline__ float ctabf(const float *p, int i) {
   return ((const __attribute__((address_space(4))) float *)p)[i];
 }
 
+template <int R>
 __device__ __forceinline__ void ad_items(int kb, int n, int NP, float rNP, int r0, int J,
-                                         int (&off)[ADF_R], bool (&ok)[ADF_R]) {
+                                         int (&off)[R], bool (&ok)[R]) {
 #pragma unroll
-  for (int r = 0; r < ADF_R; ++r) {
+  for (int r = 0; r < R; ++r) {
     const int k = kb + 64 * r;
     ok[r] = k < n;
     const int kk = ok[r] ? k : kb;
@@ -195,41 +208,42 @@ __device__ __forceinline__ void ad_items(int kb, int n, int NP, float rNP, int r
   }
 }
 
+template <int R>
 __device__ __forceinline__ void ad_jet_fwd(const float *zb, float *hb, int r0, int NP, float rNP,
                                            int J, int H, const Tables &tb, int lane) {
   const int n = NP * H;
-  for (int kb = lane; kb < n; kb += 64 * ADF_R) {
-    int off[ADF_R];
-    bool ok[ADF_R];
-    ad_items(kb, n, NP, rNP, r0, J, off, ok);
-    TanhDerivs<float> s[ADF_R];
+  for (int kb = lane; kb < n; kb += 64 * R) {
+    int off[R];
+    bool ok[R];
+    ad_items<R>(kb, n, NP, rNP, r0, J, off, ok);
+    TanhDerivs<float> s[R];
 #pragma unroll
-    for (int r = 0; r < ADF_R; ++r) s[r] = tanh_derivs(zb[off[r]]);
+    for (int r = 0; r < R; ++r) s[r] = tanh_derivs(zb[off[r]]);
 #pragma unroll
-    for (int r = 0; r < ADF_R; ++r)
+    for (int r = 0; r < R; ++r)
       if (ok[r]) hb[off[r]] = s[r].s0;
     for (int al = 1; al < J; ++al) {
       const int k0 = ctab(tb.ints, tb.pptr_i + al), k1 = ctab(tb.ints, tb.pptr_i + al + 1);
-      float v[ADF_R];
+      float v[R];
       for (int kp = k0; kp < k1; ++kp) {
         const int pr = tb.part_i + TDX_AD_PART_INTS * kp;
         const int m = ctab(tb.ints, pr);
-        float prod[ADF_R];
+        float prod[R];
 #pragma unroll
-        for (int r = 0; r < ADF_R; ++r)
+        for (int r = 0; r < R; ++r)
           prod[r] = deriv_n(s[r].s1, s[r].s2, s[r].s3, s[r].s4, s[r].s5, m);
 #pragma unroll
         for (int qq = 0; qq < TDX_AD_MAX_ORDER; ++qq)
           if (qq < m) {
             const int bq = ctab(tb.ints, pr + 1 + qq);
 #pragma unroll
-            for (int r = 0; r < ADF_R; ++r) prod[r] = prod[r] * zb[off[r] + bq];
+            for (int r = 0; r < R; ++r) prod[r] = prod[r] * zb[off[r] + bq];
           }
 #pragma unroll
-        for (int r = 0; r < ADF_R; ++r) v[r] = (kp == k0) ? prod[r] : v[r] + prod[r];
+        for (int r = 0; r < R; ++r) v[r] = (kp == k0) ? prod[r] : v[r] + prod[r];
       }
 #pragma unroll
-      for (int r = 0; r < ADF_R; ++r)
+      for (int r = 0; r < R; ++r)
         if (ok[r]) hb[off[r] + al] = v[r];
     }
   }
@@ -237,74 +251,75 @@ __device__ __forceinline__ void ad_jet_fwd(const float *zb, float *hb, int r0, i
 
 // The jet map's adjoint for the wavefront's NP points: dL/dz into dzb from
 // dL/dh in dab and the pre-activation jets zb (k_ad_bwd's arithmetic, in
-// its order), ADF_R items per lane at once.
+// its order), R items per lane at once.
+template <int R>
 __device__ __forceinline__ void ad_jet_adj(const float *zb, const float *dab, float *dzb, int r0,
                                            int NP, float rNP, int J, int H, const Tables &tb,
                                            int lane) {
   const int n = NP * H;
-  for (int kb = lane; kb < n; kb += 64 * ADF_R) {
-    int off[ADF_R];
-    bool ok[ADF_R];
-    ad_items(kb, n, NP, rNP, r0, J, off, ok);
-    TanhDerivs<float> s[ADF_R];
-    float dz0[ADF_R];
+  for (int kb = lane; kb < n; kb += 64 * R) {
+    int off[R];
+    bool ok[R];
+    ad_items<R>(kb, n, NP, rNP, r0, J, off, ok);
+    TanhDerivs<float> s[R];
+    float dz0[R];
 #pragma unroll
-    for (int r = 0; r < ADF_R; ++r) {
+    for (int r = 0; r < R; ++r) {
       s[r] = tanh_derivs(zb[off[r]]);
       dz0[r] = dab[off[r]] * s[r].s1;
     }
     for (int al = 1; al < J; ++al) {
-      float da[ADF_R];
+      float da[R];
 #pragma unroll
-      for (int r = 0; r < ADF_R; ++r) da[r] = dab[off[r] + al];
+      for (int r = 0; r < R; ++r) da[r] = dab[off[r] + al];
       const int k0 = ctab(tb.ints, tb.pptr_i + al), k1 = ctab(tb.ints, tb.pptr_i + al + 1);
       for (int kp = k0; kp < k1; ++kp) {
         const int pr = tb.part_i + TDX_AD_PART_INTS * kp;
         const int m = ctab(tb.ints, pr);
-        float all[ADF_R];
+        float all[R];
 #pragma unroll
-        for (int r = 0; r < ADF_R; ++r)
+        for (int r = 0; r < R; ++r)
           all[r] = deriv_n(s[r].s1, s[r].s2, s[r].s3, s[r].s4, s[r].s5, m + 1);
 #pragma unroll
         for (int qq = 0; qq < TDX_AD_MAX_ORDER; ++qq)
           if (qq < m) {
             const int bq = ctab(tb.ints, pr + 1 + qq);
 #pragma unroll
-            for (int r = 0; r < ADF_R; ++r) all[r] = all[r] * zb[off[r] + bq];
+            for (int r = 0; r < R; ++r) all[r] = all[r] * zb[off[r] + bq];
           }
 #pragma unroll
-        for (int r = 0; r < ADF_R; ++r) dz0[r] = dz0[r] + da[r] * all[r];
+        for (int r = 0; r < R; ++r) dz0[r] = dz0[r] + da[r] * all[r];
       }
     }
 #pragma unroll
-    for (int r = 0; r < ADF_R; ++r)
+    for (int r = 0; r < R; ++r)
       if (ok[r]) dzb[off[r]] = dz0[r];
     for (int b = 1; b < J; ++b) {
-      float acc[ADF_R];
+      float acc[R];
 #pragma unroll
-      for (int r = 0; r < ADF_R; ++r) acc[r] = 0.f;
+      for (int r = 0; r < R; ++r) acc[r] = 0.f;
       const int t0 = ctab(tb.occ, tb.tptr_i + b), t1 = ctab(tb.occ, tb.tptr_i + b + 1);
       for (int t = t0; t < t1; ++t) {
         const int oc = tb.tent_i + 3 * t;
         const int al = ctab(tb.occ, oc), qo = ctab(tb.occ, oc + 2);
         const int pr = tb.part_i + TDX_AD_PART_INTS * ctab(tb.occ, oc + 1);
         const int m = ctab(tb.ints, pr);
-        float v[ADF_R];
+        float v[R];
 #pragma unroll
-        for (int r = 0; r < ADF_R; ++r)
+        for (int r = 0; r < R; ++r)
           v[r] = dab[off[r] + al] * deriv_n(s[r].s1, s[r].s2, s[r].s3, s[r].s4, s[r].s5, m);
 #pragma unroll
         for (int q2 = 0; q2 < TDX_AD_MAX_ORDER; ++q2)
           if (q2 < m && q2 != qo) {
             const int bq = ctab(tb.ints, pr + 1 + q2);
 #pragma unroll
-            for (int r = 0; r < ADF_R; ++r) v[r] = v[r] * zb[off[r] + bq];
+            for (int r = 0; r < R; ++r) v[r] = v[r] * zb[off[r] + bq];
           }
 #pragma unroll
-        for (int r = 0; r < ADF_R; ++r) acc[r] = acc[r] + v[r];
+        for (int r = 0; r < R; ++r) acc[r] = acc[r] + v[r];
       }
 #pragma unroll
-      for (int r = 0; r < ADF_R; ++r)
+      for (int r = 0; r < R; ++r)
         if (ok[r]) dzb[off[r] + b] = acc[r];
     }
   }
@@ -770,15 +785,23 @@ __device__ __forceinline__ void ad_step_body(const ADStepArgs &a, float *smem) {
 
 // Policies of the library's kernel: the jet maps and the residual program
 // interpreted from the plan's tables.
+template <int NB>
 struct InterpJets {
+  static constexpr int R = ad_small_r(NB);
   static __device__ __forceinline__ void fwd(const float *zb, float *hb, int r0, int NP, float rNP,
                                              int J, int H, const Tables &tb, int lane) {
-    ad_jet_fwd(zb, hb, r0, NP, rNP, J, H, tb, lane);
+    if (R == ADF_R || NP * H > 64 * R)
+      ad_jet_fwd<ADF_R>(zb, hb, r0, NP, rNP, J, H, tb, lane);
+    else
+      ad_jet_fwd<R>(zb, hb, r0, NP, rNP, J, H, tb, lane);
   }
   static __device__ __forceinline__ void adj(const float *zb, const float *dab, float *dzb, int r0,
                                              int NP, float rNP, int J, int H, const Tables &tb,
                                              int lane) {
-    ad_jet_adj(zb, dab, dzb, r0, NP, rNP, J, H, tb, lane);
+    if (R == ADF_R || NP * H > 64 * R)
+      ad_jet_adj<ADF_R>(zb, dab, dzb, r0, NP, rNP, J, H, tb, lane);
+    else
+      ad_jet_adj<R>(zb, dab, dzb, r0, NP, rNP, J, H, tb, lane);
   }
 };
 struct InterpADResid {
