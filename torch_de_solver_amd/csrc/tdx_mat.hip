@@ -1551,6 +1551,25 @@ bool jit_spec_from_desc(const tdx_mat_desc *d, int div_mode, JitSpec *sp, std::s
   return true;
 }
 
+// Tiles of a tiling whose halo lies inside the grid: [a0, b0) x [a1, b1).
+struct InteriorTiles {
+  int a0, b0, a1, b1;
+  int64_t count() const { return b0 > a0 && b1 > a1 ? (int64_t)(b0 - a0) * (b1 - a1) : 0; }
+  int64_t points(int T0, int T1) const { return count() * T0 * T1; }
+};
+InteriorTiles interior_tiles(const tdx_mat_desc *d, int T0, int T1, int R0, int R1) {
+  // tile t along an axis is interior when t*T >= 2R and t*T + T + 2R <= n
+  auto first = [](int T, int R) { return (2 * R + T - 1) / T; };
+  auto end = [](int n, int T, int R) { return n - T - 2 * R >= 0 ? (n - T - 2 * R) / T + 1 : 0; };
+  return InteriorTiles{first(T0, R0), end(d->n0, T0, R0), first(T1, R1), end(d->n1, T1, R1)};
+}
+// Whether an interior of that many points is given a generated kernel (if one
+// can be had): 2^20 points, or any when asked for.
+bool generates_interior(const tdx_mat_desc *d, int64_t points) {
+  return d->dtype == 0 && d->n0 > 1 && d->n2 == 1 && d->specialize >= 0 && points > 0 &&
+         (d->specialize > 0 || points >= (1LL << 20));
+}
+
 // Sets up the specialized interior kernel of a float 2-D plan (see the
 // specialize field of tdx_mat_desc): the interior tiles of the plan's tiling
 // -- those whose halo lies inside the grid, so every stencil they apply or
@@ -1558,16 +1577,11 @@ bool jit_spec_from_desc(const tdx_mat_desc *d, int div_mode, JitSpec *sp, std::s
 // generated kernel evaluates; the general kernel keeps the other tiles.
 // Returns an error only when specialization was required (specialize = 1).
 int mat_specialize(tdx_mat_plan *p, const tdx_mat_desc *d) {
-  if (d->dtype != 0 || d->n0 == 1 || d->n2 != 1 || d->specialize < 0) return TDX_OK;
   const bool required = d->specialize > 0;
   const int T0 = p->T0, T1 = p->T1, R0 = p->R0, R1 = p->R1;
-  // tile t along an axis is interior when t*T >= 2R and t*T + T + 2R <= n
-  const int ta0 = (2 * R0 + T0 - 1) / T0, ta1 = (2 * R1 + T1 - 1) / T1;
-  const int tb0 = d->n0 - T0 - 2 * R0 >= 0 ? (d->n0 - T0 - 2 * R0) / T0 + 1 : 0;
-  const int tb1 = d->n1 - T1 - 2 * R1 >= 0 ? (d->n1 - T1 - 2 * R1) / T1 + 1 : 0;
-  if (tb0 <= ta0 || tb1 <= ta1) return TDX_OK;
-  const int64_t pts = (int64_t)(tb0 - ta0) * T0 * (tb1 - ta1) * T1;
-  if (!required && pts < (1LL << 20)) return TDX_OK;
+  const InteriorTiles in = interior_tiles(d, T0, T1, R0, R1);
+  if (!generates_interior(d, in.points(T0, T1))) return TDX_OK;
+  const int ta0 = in.a0, tb0 = in.b0, ta1 = in.a1, tb1 = in.b1;
   JitSpec sp;
   std::string why;
   if (!jit_spec_from_desc(d, p->div_mode, &sp, &why)) {
@@ -1928,7 +1942,44 @@ extern "C" int tdx_mat_plan_create(const tdx_mat_desc *d, tdx_mat_plan **out) {
     return MAT_THREADS >> p->tpr_log;  // tile rows per sweep of the workgroup
   };
   auto min_rows = [&](int rps) { return (4 * p->R0 + 8 + rps - 1) / rps * rps; };
+  // Tile rows of a 2-D grid by a model of the launch (generated: an interior
+  // large enough gets a kernel of its own).  A workgroup takes about 6 us plus
+  // 4 us per sweep of rps rows whatever its neighbours on the CU do (dependent
+  // LDS passes), so the launch takes max(1, workgroups / resident ones) times
+  // that: small grids want short tiles (128 x 128: 36 rows on 15 workgroups
+  // 57 us, 12 rows on 96 32 us), large ones the tallest that keep few rounds.
+  // Partial last rounds count half.  With a generated interior only the edge
+  // tiles are launched.
+  auto model_rows = [&](int rps, bool generated) {
+    int e0 = (int)((48 * 1024 - std::min<size_t>(fixed, 32 * 1024)) / ((size_t)p->E1 * words * ts));
+    e0 = std::min(e0, d->n0 + 4 * p->R0);
+    e0 = e0 / rps * rps;
+    if (e0 - 4 * p->R0 < 8) return min_rows(rps);
+    double best = 0;
+    const int top = e0;
+    const int T1 = p->E1 - 4 * p->R1, c = (d->n1 + T1 - 1) / T1;
+    for (int r = 4 * p->R0 + rps; r / rps * rps <= top; r += rps) {
+      const int E = r / rps * rps, T0 = E - 4 * p->R0;
+      if (T0 < 1) continue;
+      int64_t wg = (int64_t)((d->n0 + T0 - 1) / T0) * c;
+      if (generated) {
+        const InteriorTiles in = interior_tiles(d, T0, T1, p->R0, p->R1);
+        if (generates_interior(d, in.points(T0, T1))) wg -= in.count();
+      }
+      const double slots =
+          256.0 * std::max<size_t>(1, std::min<size_t>(8, 160 * 1024 / lds_for(E, p->E1)));
+      const double q = (double)wg / slots;
+      const double cost = std::max(1.0, 0.5 * (q + std::ceil(q))) * (1.5 + (double)E / rps);
+      if (best == 0 || cost < best) {
+        best = cost;
+        e0 = E;
+      }
+    }
+    return e0;
+  };
   p->nd = (d->n2 > 1 || maxc > 3) ? 1 : 0;
+  bool by_model = false;
+  int rps = 0;
   if (p->nd) {
     p->E0 = p->E1 = 1;
   } else if (d->n0 == 1) {
@@ -1939,77 +1990,42 @@ extern "C" int tdx_mat_plan_create(const tdx_mat_desc *d, tdx_mat_plan **out) {
   } else {
     p->E1 = 64;
     while (p->E1 - 4 * p->R1 < 32) p->E1 *= 2;
-    int rps = set_tpr();
+    rps = set_tpr();
     if (d->tile_rows > 0) {
       // requested output rows, rounded up so the tile rows fill whole sweeps
       p->E0 = (4 * p->R0 + d->tile_rows + rps - 1) / rps * rps;
     } else {
-      int e0 = (int)((48 * 1024 - std::min<size_t>(fixed, 32 * 1024)) / ((size_t)p->E1 * words * ts));
-      e0 = std::min(e0, d->n0 + 4 * p->R0);
-      e0 = e0 / rps * rps;
-      if (e0 - 4 * p->R0 < 8) {
-        e0 = min_rows(rps);
-      } else {
-        // A workgroup takes about 6 us plus 4 us per sweep of rps rows
-        // whatever its neighbours on the CU do (dependent LDS passes), so
-        // the launch takes max(1, workgroups / resident ones) times that:
-        // small grids want short tiles (128 x 128: 36 rows on 15 workgroups
-        // 57 us, 12 rows on 96 32 us), large ones the tallest that keep few
-        // rounds.  Partial last rounds count half.  With a generated
-        // interior only the edge tiles are launched.
-        const bool edges = d->dtype == 0 && d->specialize >= 0 && N >= (1 << 20) + (1 << 17);
-        double best = 0;
-        const int top = e0;
-        const int T1 = p->E1 - 4 * p->R1, c = (d->n1 + T1 - 1) / T1;
-        for (int r = 4 * p->R0 + rps; r / rps * rps <= top; r += rps) {
-          const int E = r / rps * rps, T0 = E - 4 * p->R0;
-          if (T0 < 1) continue;
-          const int64_t rows = (d->n0 + T0 - 1) / T0;
-          int64_t wg = rows * c;
-          if (edges) {
-            int64_t ir = 0, ic = 0;
-            for (int64_t t = 0; t < rows; ++t)
-              ir += t * T0 >= 2 * p->R0 && t * T0 - 2 * p->R0 + E <= d->n0;
-            for (int64_t t = 0; t < c; ++t)
-              ic += t * T1 >= 2 * p->R1 && t * T1 - 2 * p->R1 + p->E1 <= d->n1;
-            wg -= ir * ic;
-          }
-          const double slots =
-              256.0 * std::max<size_t>(1, std::min<size_t>(8, 160 * 1024 / lds_for(E, p->E1)));
-          const double q = (double)wg / slots;
-          const double cost = std::max(1.0, 0.5 * (q + std::ceil(q))) * (1.5 + (double)E / rps);
-          if (best == 0 || cost < best) {
-            best = cost;
-            e0 = E;
-          }
-        }
-      }
-      p->E0 = e0;
+      by_model = true;
+      p->E0 = model_rows(rps, true);
       while (lds_for(p->E0, p->E1) > 160 * 1024 && p->E1 > 16 && p->E1 / 2 - 4 * p->R1 >= 8) {
         p->E1 /= 2;
         rps = set_tpr();
         p->E0 = min_rows(rps);
+        by_model = false;
       }
     }
   }
-  p->T0 = p->E0 - 4 * p->R0;
-  p->T1 = p->E1 - 4 * p->R1;
-  // a reach that no LDS tile holds: the full-grid passes serve the plan
-  if (!p->nd && (p->T0 < 1 || p->T1 < 1 || lds_for(p->E0, p->E1) > 160 * 1024)) p->nd = 1;
-  if (p->nd) {
-    p->E0 = p->E1 = p->T0 = p->T1 = 1;
-    p->R0 = p->R1 = 0;
-  }
+  auto set_tiles = [&]() {
+    p->T0 = p->E0 - 4 * p->R0;
+    p->T1 = p->E1 - 4 * p->R1;
+    // a reach that no LDS tile holds: the full-grid passes serve the plan
+    if (!p->nd && (p->T0 < 1 || p->T1 < 1 || lds_for(p->E0, p->E1) > 160 * 1024)) p->nd = 1;
+    if (p->nd) {
+      p->E0 = p->E1 = p->T0 = p->T1 = 1;
+      p->R0 = p->R1 = 0;
+    }
+    p->tile_lds = lds_for(p->E0, p->E1);
+    p->tile_lds_fwd = p->tile_lds;
+    p->tiles0 = (d->n0 + p->T0 - 1) / p->T0;
+    p->tiles1 = (d->n1 + p->T1 - 1) / p->T1;
+    p->n_tile_wg = p->tiles0 * p->tiles1;
+    p->n_gen_wg = p->n_tile_wg;
+  };
+  set_tiles();
   p->div_mode = plan_div_mode(d);
-  p->tile_lds = lds_for(p->E0, p->E1);
-  p->tile_lds_fwd = p->tile_lds;
-  p->tiles0 = (d->n0 + p->T0 - 1) / p->T0;
-  p->tiles1 = (d->n1 + p->T1 - 1) / p->T1;
-  p->n_tile_wg = p->tiles0 * p->tiles1;
   p->n_bc_wg = (d->n_bc + MAT_THREADS - 1) / MAT_THREADS;
   p->jit_on = 0;
   p->jit_fuse = 0;
-  p->n_gen_wg = p->n_tile_wg;
 
   // stencil coefficients and their transposed products, in T
   std::vector<double> coef(MCOEF_N, 0.0);
@@ -2048,6 +2064,12 @@ extern "C" int tdx_mat_plan_create(const tdx_mat_desc *d, tdx_mat_plan **out) {
   if (rc) {
     tdx_mat_plan_destroy(p);
     return rc;
+  }
+  // no generated interior after all (the program, its compilation or spills):
+  // the height for the whole grid
+  if (by_model && !p->nd && !p->jit_on) {
+    p->E0 = model_rows(rps, false);
+    set_tiles();
   }
   // Two-launch step (train_step_to) where launches cost more than the Adam
   // pass's extra word per point: up to 2^20 grid words (128 x 128: 63 -> 24 us
