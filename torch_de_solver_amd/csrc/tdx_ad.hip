@@ -1532,12 +1532,7 @@ extern "C" int tdx_ad_plan_create(const tdx_ad_desc *d, tdx_ad_plan **out) {
     if (ok) {
       // about one work item per resident workgroup (ad_step_wgs a compute
       // unit); TDX_AD_TILES sets tiles per item
-      int dev = 0, ncu = 256;
-      if (hipGetDevice(&dev) != hipSuccess ||
-          hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-          ncu < 1)
-        ncu = 256;
-      ncu *= ad_step_wgs(nb);
+      const int ncu = device_cus() * ad_step_wgs(nb);
       int64_t tpi = (total_tiles + ncu - 1) / ncu;
       const char *te = std::getenv("TDX_AD_TILES");
       if (te && std::atoi(te) > 0) tpi = std::atoi(te);

@@ -1621,11 +1621,7 @@ int mat_specialize(tdx_mat_plan *p, const tdx_mat_desc *d) {
   // long as a band plus its halo and pipeline rows, so the band height that
   // minimizes rounds x (rows + 4 R0 + 8) is taken (on a 16384^2 grid the
   // model orders the band heights 64..1024 as the measured times do).
-  int dev = 0, cus = 0;
-  (void)hipGetDevice(&dev);
-  if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-      cus <= 0)
-    cus = 256;
+  const int cus = device_cus();
   const hipFunction_t fns[3] = {p->jit.fn_fwd, p->jit.fn_adj, p->jit.fn_step};
   p->j_waves_max = 0;
   for (int var = 0; var < 3; ++var) {
@@ -1950,6 +1946,7 @@ extern "C" int tdx_mat_plan_create(const tdx_mat_desc *d, tdx_mat_plan **out) {
   // 57 us, 12 rows on 96 32 us), large ones the tallest that keep few rounds.
   // Partial last rounds count half.  With a generated interior only the edge
   // tiles are launched.
+  const int cus = device_cus();
   auto model_rows = [&](int rps, bool generated) {
     int e0 = (int)((48 * 1024 - std::min<size_t>(fixed, 32 * 1024)) / ((size_t)p->E1 * words * ts));
     e0 = std::min(e0, d->n0 + 4 * p->R0);
@@ -1967,7 +1964,7 @@ extern "C" int tdx_mat_plan_create(const tdx_mat_desc *d, tdx_mat_plan **out) {
         if (generates_interior(d, in.points(T0, T1))) wg -= in.count();
       }
       const double slots =
-          256.0 * std::max<size_t>(1, std::min<size_t>(8, 160 * 1024 / lds_for(E, p->E1)));
+          (double)cus * std::max<size_t>(1, std::min<size_t>(8, 160 * 1024 / lds_for(E, p->E1)));
       const double q = (double)wg / slots;
       const double cost = std::max(1.0, 0.5 * (q + std::ceil(q))) * (1.5 + (double)E / rps);
       if (best == 0 || cost < best) {

@@ -1849,7 +1849,7 @@ int nn_dispatch(const tdx_nn_plan *p, int op, const void *params, void *params_m
 
 // Tiles per work item for a launch whose workgroups walk items of up to
 // `cap` tiles of one group.  tiles: tiles of each group; slots: workgroups
-// resident on the device at once (256 CUs); overhead: an item's fixed cost
+// resident on the device at once; overhead: an item's fixed cost
 // (staging, the final sums, its gradient partial) in tiles.  The launch
 // takes about ceil(items / slots) rounds of `chunk` tiles each, so the chunk
 // with the smallest rounds * (chunk + overhead) is taken, the larger one of
@@ -1861,7 +1861,6 @@ int nn_dispatch(const tdx_nn_plan *p, int op, const void *params, void *params_m
 // 100 points on 1-100x2-1 192 -> 38 us a step (2 items before), Burgers
 // 256 x 100 on 2-100x4-1 755 -> 526 us (346 items of 8 tiles took two rounds
 // of 256; now 252 of 11 take one), KdV 512 x 128 489 -> 429 us.
-constexpr int kCUs = 256;
 int pick_chunk(const std::vector<int64_t> &tiles, int64_t slots, int cap, double overhead) {
   int best = cap;
   double best_cost = 0;
@@ -2149,6 +2148,7 @@ static int nn_plan_create(const tdx_nn_desc *d, tdx_nn_plan **out, const tdx_nn_
   const int H = p->H;
   p->P = H * d->d_in + H + p->NH * (H * H + H) + d->n_out * H + d->n_out;
   const size_t ts = d->dtype == 0 ? 4 : 8;
+  const int cus = device_cus();
 
   // forward work: 64 entries per workgroup
   std::vector<int2> k1;
@@ -2176,7 +2176,7 @@ static int nn_plan_create(const tdx_nn_desc *d, tdx_nn_plan **out, const tdx_nn_
     // 63 -> 55, 2-100x2-1 (81 KB) 85 -> 109; 40 x 30 points (18 workgroups),
     // 2-48x4-1 53 -> 48, 2-100x2-1 67 -> 56.
     const size_t st = (size_t)stage_words(p->HP, p->NH, d->d_in, d->n_out, false, (int)ts) * ts;
-    const size_t limit = persist || k1.size() <= (size_t)kCUs ? 160 * 1024 : 64 * 1024;
+    const size_t limit = persist || k1.size() <= (size_t)cus ? 160 * 1024 : 64 * 1024;
     p->k1_stage = p->k1_lds + st <= limit ? 1 : 0;
     if (p->k1_stage) p->k1_lds += st;
   }
@@ -2232,9 +2232,9 @@ static int nn_plan_create(const tdx_nn_desc *d, tdx_nn_plan **out, const tdx_nn_
   const int chunk_tiles =
       d->chunk_tiles > 0  ? d->chunk_tiles
       : fixed              ? (p->k2_wave_private ? 256 : p->k2_block ? 8 : p->acc_lds ? 16 : 4)
-      : p->k2_wave_private ? pick_chunk(k2_tiles, 3 * kCUs, 256, 1.0)
-      : p->k2_block        ? pick_chunk(k2_tiles, kCUs * block_residency<false>(p->NB, p->NH, nullptr, p->k2_lds), 16, 0.25)
-                           : pick_chunk(k2_tiles, kCUs, p->acc_lds ? 16 : 4, 1.0);
+      : p->k2_wave_private ? pick_chunk(k2_tiles, 3 * cus, 256, 1.0)
+      : p->k2_block        ? pick_chunk(k2_tiles, cus * block_residency<false>(p->NB, p->NH, nullptr, p->k2_lds), 16, 0.25)
+                           : pick_chunk(k2_tiles, cus, p->acc_lds ? 16 : 4, 1.0);
   std::vector<int4> k2;
   for (int g = 0; g < d->n_groups; ++g) {
     const int32_t *G = d->groups + (int64_t)g * TDX_GROUP_INTS;
@@ -2281,7 +2281,7 @@ static int nn_plan_create(const tdx_nn_desc *d, tdx_nn_plan **out, const tdx_nn_
       blocks.push_back((d->groups[(int64_t)g * TDX_GROUP_INTS + 1] + 63) / 64);
     const int C = d->chunk_tiles > 0 ? d->chunk_tiles
                   : fixed            ? 4
-                                     : pick_chunk(blocks, 4 * kCUs, 4, 0.25);
+                                     : pick_chunk(blocks, 4 * cus, 4, 0.25);
     for (int g = 0; g < d->n_groups; ++g) {
       const int32_t *G = d->groups + (int64_t)g * TDX_GROUP_INTS;
       const int nblk = (G[1] + 63) / 64;
@@ -2383,7 +2383,7 @@ static int nn_plan_create(const tdx_nn_desc *d, tdx_nn_plan **out, const tdx_nn_
     const int C = d->chunk_tiles > 0
                       ? d->chunk_tiles
                   : fixed ? 8
-                      : pick_chunk(tiles, kCUs * block_residency<true>(p->NB, p->NH, p->block_fn, p->k4_lds), 16,
+                      : pick_chunk(tiles, cus * block_residency<true>(p->NB, p->NH, p->block_fn, p->k4_lds), 16,
                              0.25);
     for (int g = 0; g < d->n_groups; ++g) {
       const int32_t *G = d->groups + (int64_t)g * TDX_GROUP_INTS;
