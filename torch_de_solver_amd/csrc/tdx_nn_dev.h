@@ -150,8 +150,31 @@ __device__ __forceinline__ Bits3 image_pair(const NNArgs<float> &a, const float 
     const int out = which == 0 ? x : f, in = which == 0 ? f : x;
     w2[k] = (out < H && in < H) ? W[L.oWh(j) + out * H + in] : 0.f;
   }
+  // weights that round to infinity in bf16, after the others (their remainder
+  // would be NaN): a finite one as the largest bf16 and its exact remainder, an
+  // infinite one as the last piece alone, which meets only the leading piece of
+  // the other factor, so the product is float32's
+  float over[2] = {0.f, 0.f};
+#pragma unroll
+  for (int k = 0; k < 2; ++k)
+    if (fabsf(w2[k]) >= 0x1.FFp127f) over[k] = w2[k], w2[k] = 0.f;
   unsigned h[1], m[1], l[1];
   bf3_pairs<1>(w2, h, m, l);
+#pragma unroll
+  for (int k = 0; k < 2; ++k)
+    if (over[k] != 0.f) {
+      const unsigned sign = __builtin_bit_cast(unsigned, over[k]) >> 31 << 15;
+      if (fabsf(over[k]) == __builtin_inff()) {
+        l[0] |= (0x7F80u | sign) << (16 * k);
+      } else {
+        const float rest[2] = {over[k] - copysignf(0x1.FEp127f, over[k]), 0.f};
+        unsigned rh[1], rm[1], rl[1];
+        bf3_pairs<1>(rest, rh, rm, rl);
+        h[0] |= (0x7F7Fu | sign) << (16 * k);
+        m[0] |= (rh[0] & 0xFFFFu) << (16 * k);
+        l[0] |= (rm[0] & 0xFFFFu) << (16 * k);
+      }
+    }
   return Bits3{h[0], m[0], l[0]};
 }
 
