@@ -221,8 +221,9 @@ class ADEngine:
         self.n_params = int(lib.tdx_ad_param_count(handle))
         nbytes = int(lib.tdx_ad_workspace_bytes(handle))
         self.workspace = torch.empty(max(nbytes, 1), dtype=torch.uint8, device=device)
-        # forward passes so far: the adjoint reads the jets and seeds of the
-        # latest one, so a backward checks that it belongs to its forward
+        # forward passes so far: the layer kernels' adjoint reads the jets and
+        # seeds of the latest one, so a backward checks that it belongs to its
+        # forward (the fused kernel's forms its own)
         self.fwd_gen = 0
 
     def __del__(self):
@@ -316,7 +317,7 @@ class ADResidualLoss(torch.autograd.Function):
     def backward(ctx, grad_out: torch.Tensor):
         (p,) = ctx.saved_tensors
         eng: ADEngine = ctx.engine
-        if eng.fwd_gen != ctx.gen:
+        if eng.fwd_gen != ctx.gen and eng.step_kernel == 'layers':
             # another forward pass ran since this node's: restore its jets
             # and seeds before the adjoint
             eng.forward(p, torch.empty(2, dtype=eng.dtype, device=eng.device))
