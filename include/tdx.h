@@ -88,6 +88,12 @@ const char *tdx_last_error(void);
 #define TDX_FACTOR_INTS 6
 #define TDX_STENCIL_INTS 2
 
+/* float32 networks: the products of hidden layers are sums of six bf16 piece
+ * products of each pair of values, in float32 accumulators.  Hidden weights are
+ * exact in the pieces from 2^-110 to the largest float32, and infinite ones act
+ * as in float32.  An activation jet, delta or seed that is infinite, or rounds
+ * to infinity in bf16 (3.39e38 and more), gives NaN in the sums that it enters,
+ * where float32 products may give an infinity. */
 typedef struct tdx_nn_desc {
   int dtype;
   int d_in, n_out, width, n_layers;
@@ -104,9 +110,10 @@ typedef struct tdx_nn_desc {
   int tile_rows;    /* backward tile rows (0: default; -1: workgroup-cooperative kernel;
                        32: two 16-row tiles per wavefront iteration of the
                        wavefront-private kernel (float), otherwise one) */
-  int chunk_tiles;  /* work per gradient work item (0: default): 64-row tiles of the
-                       separate adjoint kernel, or 64-entry blocks of the fused
-                       training-step kernel (default 4) */
+  int chunk_tiles;  /* work per gradient work item: 64-row tiles of the separate
+                       adjoint kernel, or 64-entry blocks of the fused training-step
+                       kernel (0: sized so that the items fill the device in few,
+                       whole rounds) */
   /* Causal loss (tedeous/losses.py:137-182), one instance: tol != 0 replaces
    * the operator term of group 0's equations (loss and normalized weights 0,
    * seed weight 1/N) by mean(w * res), res[p] = sum_eq r_eq[p]^2 over the
@@ -143,7 +150,7 @@ typedef struct tdx_nn_desc {
    * kernel too: their block-owning adjoint, which evaluates the network
    * again anyway, takes tiles of whole entries, runs the residual program
    * on them and forms its own seeds (three launches; chunk_tiles counts
-   * such tiles, default 8).  Otherwise, and with -1, separate forward and
+   * such tiles).  Otherwise, and with -1, separate forward and
    * adjoint kernels, one workgroup per work item.  1: separate kernels with the
    * persistent forward: when the network's forward image fits in LDS (160 KB
    * with the kernel's own words, float images in bf16 pieces) and the plan has no causal or weak-form loss, the forward kernel runs
@@ -542,8 +549,8 @@ int tdx_ad_jacobian(const tdx_ad_plan *plan, const void *params, void *jt,
  * the layer kernels of tdx_ad_forward/tdx_ad_backward and tdx_adam.  The
  * two differ in the order of the float sums only.  Environment:
  * TDX_AD_FUSED=0 keeps the layer kernels; TDX_AD_TILES sets the tiles per
- * work item of the fused kernel (default: about one item per compute
- * unit).  Replaces Closure._closure (tedeous/optimizers/closure.py:49-64)
+ * work item of the fused kernel (default: about one item per workgroup that
+ * the device keeps resident, two per compute unit up to 64 hidden units).  Replaces Closure._closure (tedeous/optimizers/closure.py:49-64)
  * with loss.backward() through Derivative_autograd
  * (tedeous/derivative.py:61-132). */
 int tdx_ad_train_step(const tdx_ad_plan *plan, void *params, void *exp_avg,

@@ -3,8 +3,8 @@ network (odd ones leave half a k-step empty), its edges, and one to three
 H x H layers, against the separate kernels and torch's float64 backward of
 the same seeds (the bounds of test_fused_gpu._compare: network values and
 losses the same in every kernel, gradients within four times the error of
-torch's own float32 backward); and values over the whole exponent range
-through a layer against float64.
+torch's own float32 backward); and weights of 2^-60 to 2^20 in one layer
+against float64 (beyond bf16's range: test_large_weights_gpu.py).
 """
 import numpy as np
 import pytest

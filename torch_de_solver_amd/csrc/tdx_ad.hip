@@ -1028,9 +1028,11 @@ k_ad_step(ADStepArgs a) {
 
 // k_ad_loss_pass: the fused step's forward half, for evaluations that want
 // the loss alone: no derivatives stored, no gradient partials, the jet maps
-// and the residual program interpreted.  Bound, like the step, by VALU work
-// and waits at ad_step_wgs(NB) wavefronts per SIMD (133 x 91 points, 2-64x3-1:
-// 60 us).
+// and the residual program interpreted, also where the step's are generated.
+// Bound, like the step, by VALU work and waits at ad_step_wgs(NB) wavefronts
+// per SIMD.  An evaluation by the layer kernels and by this one: 133 x 91
+// points 2-64x3-1 131, 59 us, 2-100x5-1 312, 171; 201 x 201 2-32x2-1 106, 79,
+// 2-64x3-1 249, 120, 2-100x5-1 775, 453, 2-128x4-1 750, 545.
 template <int NB>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ad_step_wgs(NB)))) void
 k_ad_loss_pass(ADStepArgs a) {
@@ -1847,9 +1849,8 @@ extern "C" int tdx_ad_forward(const tdx_ad_plan *p, const void *params, void *lo
   TDX_REQUIRE(p && params && loss && ws, "null argument");
   hipStream_t s = (hipStream_t)stream;
   // the loss alone needs no jets in memory: the fused step's forward half
-  // (its adjoint forms the jets again; 133 x 91 Poisson, 2-64x3-1, evaluate
-  // and backward together: 364 -> 293 us); residuals come from the layer
-  // kernels
+  // (its adjoint forms the jets again; k_ad_loss_pass has both sides' times);
+  // residuals come from the layer kernels
   if (p->fused && !resid)
     return ad_fused_step(p, (float *)const_cast<void *>(params), nullptr, nullptr, nullptr,
                          AdamHyper{0, 0, 0, 0}, (float *)loss, ws, s, nullptr, nullptr);
@@ -1864,8 +1865,9 @@ extern "C" int tdx_ad_backward(const tdx_ad_plan *p, const void *params, const v
   hipStream_t s = (hipStream_t)stream;
   // the fused step's kernel forms the jets again instead of reading the
   // layers' arrays, and is still faster than the layer kernels' adjoint with
-  // its products per layer (133 x 91 Poisson, 2-64x3-1, evaluate and backward
-  // together: 482 -> 364 us; the kernel itself 195 us)
+  // its products per layer (evaluate and backward together, layer kernels and
+  // fused: 133 x 91 points 2-64x3-1 463, 239 us, 2-100x5-1 1112, 834; 201 x 201
+  // 2-100x5-1 2562, 1382)
   if (p->fused)
     return ad_fused_step(p, (float *)const_cast<void *>(params), nullptr, nullptr, nullptr,
                          AdamHyper{0, 0, 0, 0}, nullptr, ws, s, (const float *)dloss,

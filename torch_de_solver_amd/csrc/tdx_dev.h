@@ -46,8 +46,9 @@ struct Bf3 {
 // The remainder x - h is a dot product of the packed pieces with (-1, 0) or
 // (0, -1) on top of x: exact, and one instruction where unpacking and
 // subtracting are two.  Stage by stage over the pairs, so that the dot
-// products' latencies overlap.  An infinite or NaN value makes its remainder,
-// and its pair partner's, NaN.
+// products' latencies overlap.  An infinite or NaN value, or one that rounds to
+// infinity, makes its remainder, and its pair partner's, NaN (image_pair takes
+// such weights out first).
 template <int NP>
 __device__ __forceinline__ void bf3_pairs(const float (&x)[2 * NP], unsigned (&h)[NP],
                                           unsigned (&m)[NP], unsigned (&l)[NP]) {

@@ -2069,9 +2069,12 @@ extern "C" int tdx_mat_plan_create(const tdx_mat_desc *d, tdx_mat_plan **out) {
     set_tiles();
   }
   // Two-launch step (train_step_to) where launches cost more than the Adam
-  // pass's extra word per point: up to 2^20 grid words (128 x 128: 63 -> 24 us
-  // a step with the smaller tiles); larger grids keep the boundary adjoint's
-  // own launch.  A touched point listed twice keeps it too.
+  // pass's extra word per point: up to 2^20 grid words; larger grids keep the
+  // boundary adjoint's own launch.  A step without and with it: float32 512^2
+  // 32.8, 29.0 us, 700^2 39.2, 37.1, 900^2 46.2, 45.4, 1000^2 54.2, 55.0;
+  // float64 512^2 37.1, 33.9, 777 x 1001 77.7, 74.8, 1000^2 89.3, 86.0.  From
+  // about 1.1 M words on float32 grids have a generated interior and its own
+  // step.  A touched point listed twice keeps the launch too.
   if (!p->nd && !p->jit_on && N * d->n_eq <= (1 << 20)) {
     std::vector<int32_t> map((size_t)(N * d->n_eq), -1);
     p->merged_step = 1;

@@ -2258,8 +2258,8 @@ static int nn_plan_create(const tdx_nn_desc *d, tdx_nn_plan **out, const tdx_nn_
   if (ik2i.empty()) ik2i.push_back(0);
 
   // fused training step for narrow float networks with one output and at
-  // most two inputs: work items of chunk_tiles 64-entry blocks (default 4)
-  // of one group, and each group's residual program as its own table pair
+  // most two inputs: work items of chunk_tiles 64-entry blocks
+  // (0: sized by pick_chunk, up to 4) of one group, and each group's residual program as its own table pair
   std::vector<int4> k3, prog_idx;
   std::vector<int32_t> prog_ints, ik3p(1, 0), ik3i, prog_kind;
   std::vector<float> prog_reals;
@@ -2329,7 +2329,7 @@ static int nn_plan_create(const tdx_nn_desc *d, tdx_nn_plan **out, const tdx_nn_
 
   // wide float networks: the training step's block-owning backward forms
   // its own seeds over tiles of whole entries (E = 64 / slots per tile),
-  // chunk_tiles tiles per work item (default 8)
+  // chunk_tiles tiles per work item (0: sized by pick_chunk, up to 16)
   std::vector<int4> k4;
   std::vector<int32_t> ik4p(1, 0), ik4i;
   std::vector<int> inst_k4_size(d->n_inst, 0);
