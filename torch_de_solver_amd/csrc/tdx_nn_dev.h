@@ -290,7 +290,7 @@ __device__ Net<T, NB, true> stage_net(const NNArgs<T> &a, int inst, T *dst, bool
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
       const int k = k0 + i * blockDim.x;
-      v[i] = s4[k < n4 ? k : k0];
+      if (k < n4) v[i] = s4[k];
     }
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
